@@ -15,6 +15,7 @@ SOURCES = [
     "afqmc_api.hip",
     "k_greens.hip",
     "k_gemm.hip",
+    "k_nt64.hip",
     "k_exchange.hip",
     "k_bf16.hip",
     "k_quad.hip",

@@ -531,9 +531,9 @@ int do_force_bias_bf16(afqmc_ctx* c, int nw, const double* ga, const double* gb)
 int do_force_bias(afqmc_ctx* c, int nw, const double* ga, const double* gb) {
   if (c->bf16_fb) return do_force_bias_bf16(c, nw, ga, gb);
   const int N = c->d.nbasis, na = c->d.nalpha, nb = c->d.nbeta;
-  ForceBiasArgs a;
-  a.nwalkers = nw;
-  a.nchol = c->d.nchol;
+  NtArgs a{};
+  a.m = nw;
+  a.n = c->d.nchol;
   a.ksplit = c->fb_ksplit;
   a.nseg = 1;
   a.seg[0] = NtSegment{ga, (int64_t)na * N, c->s.rchola, (int64_t)na * N, na * N};
@@ -544,9 +544,9 @@ int do_force_bias(afqmc_ctx* c, int nw, const double* ga, const double* gb) {
   } else if (c->d.rhf) {  // force_bias.py:101-104 doubles for rhf whatever ndown
     a.scale = 2.0;
   }
-  a.vbias_part = c->vbias_part;
+  a.out = c->vbias_part;
   PhaseScope ps(c, AFQMC_PHASE_FORCE_BIAS);
-  HIP_TRY(c, launch_force_bias(a, c->stream));
+  HIP_TRY(c, launch_nt64(a, c->stream));
   return AFQMC_OK;
 }
 
@@ -607,19 +607,20 @@ int do_vhs(afqmc_ctx* c, int nw) {
     HIP_TRY(c, launch_bf16_gemm(b, c->stream));
     return AFQMC_OK;
   }
-  VhsArgs a;
-  a.nwalkers = nw;
-  a.nbasis = c->d.nbasis;
-  a.nchol = c->d.nchol;
-  a.xshifted = c->xshifted;
-  a.chol_packed = c->s.chol_packed;
-  const int P = c->d.nbasis * (c->d.nbasis + 1) / 2;
+  const int64_t N = c->d.nbasis, X = c->d.nchol, P = N * (N + 1) / 2;
+  NtArgs a{};
+  a.m = nw;
+  a.n = P;
+  a.ksplit = 1;
+  a.nseg = 1;
+  a.seg[0] = NtSegment{c->xshifted, X, c->s.chol_packed, X, (int)X};
+  a.scale = sqrt(c->s.dt);
+  a.out = c->vhs;
   a.tri_i = c->tri;
   a.tri_j = c->tri + P;
-  a.sqrt_dt = sqrt(c->s.dt);
-  a.vhs = c->vhs;
+  a.nbasis = (int)N;
   PhaseScope ps(c, AFQMC_PHASE_VHS);
-  HIP_TRY(c, launch_vhs(a, c->stream));
+  HIP_TRY(c, launch_nt64(a, c->stream));
   return AFQMC_OK;
 }
 
@@ -1006,15 +1007,15 @@ int exchange_spin_quad(afqmc_ctx* c, int nw, int spin, const double* g, const in
       g = c->gcomp;
     }
     const int64_t nN = (int64_t)n * N;
-    ForceBiasArgs a;
-    a.nwalkers = nw;
-    a.nchol = (int)nN;
+    NtArgs a{};
+    a.m = nw;
+    a.n = nN;
     a.ksplit = 1;
     a.nseg = 1;
     a.seg[0] = NtSegment{g, nN, c->qw64[spin], nN, (int)nN};
     a.scale = 1.0;
-    a.vbias_part = c->qy;
-    HIP_TRY(c, launch_force_bias(a, c->stream));
+    a.out = c->qy;
+    HIP_TRY(c, launch_nt64(a, c->stream));
     HIP_TRY(c, launch_quad_reduce(c->qy, 1, nw, n, N, N, g, nullptr, part, c->stream));
   }
   c->xs_used[spin] = 1;
@@ -1338,16 +1339,8 @@ int afqmc_create(afqmc_ctx** out, int device, const afqmc_dims* dims) {
   const bool two = d.nbeta > 0 && !d.rhf;
   c->ncol = two ? d.nalpha + d.nbeta : d.nalpha;
   const int64_t W = d.nwalkers, N = d.nbasis, X = d.nchol > 0 ? d.nchol : 1;
-  // force-bias split-K: enough workgroups to fill the chip, >= 64 K chunks each
-  {
-    const int64_t tiles = ceil_div(W, 64) * ceil_div(X, 128);
-    const int64_t kch = ceil_div((int64_t)d.nalpha * N, 16) + (two ? ceil_div((int64_t)d.nbeta * N, 16) : 0);
-    int64_t ks = ceil_div(1024, tiles);
-    if (ks > kch / 64) ks = kch / 64;
-    if (ks > 8) ks = 8;
-    if (ks < 1) ks = 1;
-    c->fb_ksplit = (int)ks;
-  }
+  c->fb_ksplit = nt64_ksplit(W, X, ceil_div((int64_t)d.nalpha * N, 16) + (two ? ceil_div((int64_t)d.nbeta * N, 16) : 0),
+                             FB_MAX_SPLIT);
   c->xs_a = exchange_xsplit(d.nwalkers, (int)X, d.nalpha);
   c->xs_b = two ? exchange_xsplit(d.nwalkers, (int)X, d.nbeta) : 1;
   snprintf(c->describe_dims, sizeof(c->describe_dims), "N=%d X=%d na=%d nb=%d W=%d", d.nbasis, d.nchol, d.nalpha,
@@ -2210,7 +2203,7 @@ int tune_fb_max(const afqmc_ctx* c) {
   }
   const int64_t N = c->d.nbasis;
   const int64_t kch = ceil_div((int64_t)c->d.nalpha * N, 16) + (two_spins(c) ? ceil_div((int64_t)c->d.nbeta * N, 16) : 0);
-  return (int)std::max<int64_t>(1, std::min<int64_t>(32, kch / 8));
+  return (int)std::max<int64_t>(1, std::min<int64_t>(32, kch / 2));
 }
 int tune_exx_max(const afqmc_ctx* c) {
   int hi = 1;

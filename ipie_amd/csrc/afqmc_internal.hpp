@@ -81,24 +81,24 @@ struct NtSegment {
   int K;
 };
 
-struct ForceBiasArgs {
-  int nwalkers, nchol, nseg, ksplit;
+struct NtArgs {
+  int64_t m, n;      // rows of A, rows of B (columns of C)
+  int nseg, ksplit;  // segments; K ranges (over the chunks of all segments)
   NtSegment seg[2];
-  double scale;        // 1, or 2 for RHF walkers
-  double* vbias_part;  // [ksplit, W, X] complex
+  double scale;
+  double* out;       // [ksplit, m, n] complex: scale C; with tri_i: [m, nbasis, nbasis] complex
+  // packed-index row and column of each column of C, or null: C's columns are the
+  // packed upper triangle of symmetric matrices, written to both triangles times i scale
+  const int* tri_i;
+  const int* tri_j;
+  int nbasis;
 };
-hipError_t launch_force_bias(const ForceBiasArgs& a, hipStream_t stream);
-
-struct VhsArgs {
-  int nwalkers, nbasis, nchol;
-  const double* xshifted;     // [W, X] complex
-  const double* chol_packed;  // [P, X] real
-  const int* tri_i;           // [P] row of packed index p
-  const int* tri_j;           // [P] column of packed index p
-  double sqrt_dt;
-  double* vhs;                // [W, N, N] complex (full, symmetric)
-};
-hipError_t launch_vhs(const VhsArgs& a, hipStream_t stream);
+hipError_t launch_nt64(const NtArgs& a, hipStream_t stream);
+// K ranges (1 .. most) for an [m, n] product over `chunks` 16-wide K chunks: enough
+// workgroups to fill the GPU and rounds that end together, against the
+// partial sums each range adds
+int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, int most);
+constexpr int FB_MAX_SPLIT = 16;  // most K ranges of the FP64 force bias (heuristic)
 
 // Batched C[w] = A[w] * B[w] with A [N, N] (real shared or complex per walker)
 // and B [N, ncol] complex (columns contiguous).  Epilogue:
