@@ -36,6 +36,10 @@ namespace afqmc {
 
 namespace {
 
+// LDS is read through this vector type: a read through double2 makes the compiler
+// wait for every direct load in flight before it
+typedef double v2d __attribute__((ext_vector_type(2)));
+
 constexpr int NT_KC = 16;                // K per LDS stage
 constexpr int NT_RN = 2, NT_WAVES = 4;   // 16-column tiles per wave, waves side by side
 constexpr int NT_TN = 16 * NT_RN * NT_WAVES;
@@ -45,21 +49,46 @@ __device__ double2 nt_zero;  // source of the slots past K
 
 enum { NT_EPI_PART = 0, NT_EPI_VHS = 1 };
 
-__device__ __forceinline__ void nt_load16(const char* src, double2* dst) {
+// Direct global-to-LDS loads: lane l's 16 (4) bytes go to dst + 16 l (4 l).
+__device__ __forceinline__ void nt_load16(const char* src, void* dst) {
   __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
+__device__ __forceinline__ void nt_load4(const char* src, void* dst) {
+  __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
+}
 
-// How the operands reach LDS: NT_DIRECT both by direct loads (16-byte aligned
-// rows, K even); NT_BREG B's values one by one through registers (odd K or row
-// pitch), stored after the current chunk's MFMAs are issued; NT_REG both.
-enum { NT_DIRECT = 0, NT_BREG = 1, NT_REG = 2 };
+// Loads of 16 bytes a lane where the operand's rows are 16-byte aligned (and B's
+// K even, so that a pair is whole or absent), of 4 bytes otherwise.
+enum { NT_16 = 0, NT_B4 = 1, NT_AB4 = 2 };
+
+template <int RM, int MODE>
+struct NtPlan {
+  static constexpr int TM = 16 * RM;
+  static constexpr int A_SLOTS = TM * NT_KC, B_SLOTS = NT_TN * NT_KC / 2, STAGE = A_SLOTS + B_SLOTS;
+  static constexpr int A_LOADS = MODE == NT_AB4 ? 4 * RM : RM, B_LOADS = MODE == NT_16 ? 4 : 16;  // per wave
+  static constexpr int LOADS = A_LOADS + B_LOADS;
+  // LDS stages: a chunk of a small row tile is multiplied in less time than a
+  // load takes, so more of them are in flight (two workgroups still fit a CU)
+  static constexpr int STAGES = RM == 1 ? 4 : RM == 2 ? 3 : 2;
+  static constexpr int LDS_BYTES = 16 * STAGE * STAGES;
+  static_assert(2 * LDS_BYTES <= 160 * 1024 && STAGES * LOADS <= 63 + LOADS, "LDS and vmcnt");
+};
+
+template <int N>
+__device__ __forceinline__ void nt_barrier() {
+  // (this wave's LDS reads are waited for where the compiler sees it, or it waits
+  // for the next ones too before their use)
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+}
 
 template <int RM, int MODE, int EPI>
 __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
-  constexpr int TM = 16 * RM;
-  constexpr int A_SLOTS = TM * NT_KC, B_SLOTS = NT_TN * NT_KC / 2, STAGE = A_SLOTS + B_SLOTS;
-  __shared__ double2 lds[2 * STAGE];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+  using P = NtPlan<RM, MODE>;
+  constexpr int TM = P::TM, ST = P::STAGES;
+  extern __shared__ uint4 nt_lds[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
   const int nbm = (int)ceil_div(a.m, TM);
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
   const int bm = lin % nbm, bn = lin / nbm, z = blockIdx.y;
@@ -83,92 +112,102 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
     const NtSegment sg = s == 0 ? a.seg[0] : a.seg[1];
     const int c_begin = s == 0 ? z0 : max(z0, nch0) - nch0, c_end = s == 0 ? min(z1, nch0) : z1 - nch0;
     if (c_begin >= c_end) continue;
-    // this lane's slots: byte offsets from the tile's first row and column (rows
-    // and columns past the end read the last one; their results are not written)
+    // sources of this lane: byte offsets from the tile's first row and column
+    // (rows and columns past the end read the last one; their results are not
+    // written) and first K index of each load
     const char* abase = reinterpret_cast<const char*>(sg.A + 2 * (int64_t)row0 * sg.lda);
     const char* bbase = reinterpret_cast<const char*>(sg.B + col0 * sg.ldb);
-    const int last_r = (int)min((int64_t)TM, a.m - row0) - 1, last_c = (int)min((int64_t)NT_TN, a.n - col0) - 1;
-    auto a_k = [&](int j) { return (lane & 15) ^ ((4 * (wave * RM + j) + (lane >> 4)) & 15); };
-    auto b_k = [&](int) { return 2 * ((lane & 7) ^ (lane >> 3)); };  // column % 8 = lane / 8
-    uint32_t ao[RM], bo[4];
+    const uint32_t last_r = (uint32_t)min((int64_t)TM, a.m - row0) - 1, last_c = (uint32_t)min((int64_t)NT_TN, a.n - col0) - 1;
+    const uint32_t apitch = 16u * (uint32_t)sg.lda, bpitch = 8u * (uint32_t)sg.ldb;
+    auto a_row = [&](int j) { return MODE == NT_AB4 ? 4 * RM * wave + j : 4 * (RM * wave + j) + (lane >> 4); };
+    auto a_k = [&](int j) { return (MODE == NT_AB4 ? lane >> 2 : lane & 15) ^ (a_row(j) & 15); };
+    auto a_off = [&](int j) {
+      return min((uint32_t)a_row(j), last_r) * apitch + 16u * a_k(j) + (MODE == NT_AB4 ? 4u * (lane & 3) : 0u);
+    };
+    auto b_col = [&](int j) { return MODE == NT_16 ? 8 * (4 * wave + j) + (lane >> 3) : 2 * (16 * wave + j) + (lane >> 5); };
+    auto b_pair = [&](int j) { return (MODE == NT_16 ? lane & 7 : (lane & 31) >> 2) ^ (b_col(j) & 7); };
+    auto b_k = [&](int j) { return 2 * b_pair(j) + (MODE == NT_16 ? 0 : (lane & 3) >> 1); };
+    auto b_off = [&](int j) {
+      return min((uint32_t)b_col(j) * bpitch, last_c * bpitch) + 16u * b_pair(j) + (MODE == NT_16 ? 0u : 4u * (lane & 3));
+    };
+    uint32_t ao[RM], bo[4];  // of the 16-byte loads
 #pragma unroll
-    for (int j = 0; j < RM; ++j)
-      ao[j] = 16u * ((uint32_t)min(4 * (wave * RM + j) + (lane >> 4), last_r) * (uint32_t)sg.lda + a_k(j));
+    for (int j = 0; j < RM; ++j) ao[j] = a_off(j);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      bo[j] = 8u * ((uint32_t)min(8 * (wave * 4 + j) + (lane >> 3), last_c) * (uint32_t)sg.ldb + b_k(j));
-    double2 areg[RM], breg[4];
-    // starts the loads of chunk c, into the LDS stage or the registers
-    auto fetch = [&](int c, double2* stage) {
-      const int k0 = NT_KC * c, left = sg.K - k0;
+    for (int j = 0; j < 4; ++j) bo[j] = b_off(j);
+    // starts the loads of chunk c into its stage (zeros past K, and all zeros past
+    // c_end: every iteration issues the same number of loads, so that a wait can
+    // name the ones that may stay in flight, and has no branch, so that their
+    // addresses are computed between MFMAs)
+    auto fetch = [&](int c) {
+      const int k0 = NT_KC * c, left = c < c_end ? sg.K - k0 : 0;
+      uint4* As = nt_lds + (c - c_begin) % ST * P::STAGE;
+      uint4* Bs = As + P::A_SLOTS;
       const char* ac = abase + 16 * (int64_t)k0;
       const char* bc = bbase + 8 * (int64_t)k0;
-      double2* As = stage + wave * RM * 64;
-      double2* Bs = stage + A_SLOTS + wave * 4 * 64;
-      const bool full = left >= NT_KC;
       const char* zero = reinterpret_cast<const char*>(&nt_zero);
 #pragma unroll
-      for (int j = 0; j < RM; ++j) {
-        const char* p = full || a_k(j) < left ? ac + ao[j] : zero;
-        if (MODE != NT_REG) nt_load16(p, As + 64 * j);
-        else areg[j] = make_double2(reinterpret_cast<const double*>(p)[0], reinterpret_cast<const double*>(p)[1]);
+      for (int j = 0; j < P::A_LOADS; ++j) {
+        if constexpr (MODE == NT_AB4) nt_load4(a_k(j) < left ? ac + a_off(j) : zero, As + (4 * RM * wave + j) * 16);
+        else nt_load16(a_k(j) < left ? ac + ao[j] : zero, As + (RM * wave + j) * 64);
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (MODE == NT_DIRECT) {
-          nt_load16(full || b_k(j) < left ? bc + bo[j] : zero, Bs + 64 * j);
-        } else {
-          const double* p = reinterpret_cast<const double*>(bc + bo[j]);
-          breg[j].x = b_k(j) < left ? p[0] : 0.0;
-          breg[j].y = b_k(j) + 1 < left ? p[1] : 0.0;
-        }
+      for (int j = 0; j < P::B_LOADS; ++j) {
+        if constexpr (MODE == NT_16) nt_load16(b_k(j) < left ? bc + bo[j] : zero, Bs + (4 * wave + j) * 64);
+        else nt_load4(b_k(j) < left ? bc + b_off(j) : zero, Bs + (16 * wave + j) * 16);
       }
     };
-    auto stash = [&](double2* stage) {
-      if (MODE == NT_REG) {
+    // fragments of half h (K pairs h of every lane group) of chunk c
+    auto read = [&](int c, int h, v2d (&af)[RM][2], v2d (&bf)[NT_RN]) {
+      const v2d* As = reinterpret_cast<const v2d*>(nt_lds + (c - c_begin) % ST * P::STAGE);
+      const v2d* Bs = As + P::A_SLOTS;
 #pragma unroll
-        for (int j = 0; j < RM; ++j) stage[(wave * RM + j) * 64 + lane] = areg[j];
-      }
-      if (MODE != NT_DIRECT) {
+      for (int j = 0; j < NT_RN; ++j) bf[j] = Bs[(wave * 16 * NT_RN + 16 * j + l16) * 8 + ((2 * q + h) ^ (l16 & 7))];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) stage[A_SLOTS + (wave * 4 + j) * 64 + lane] = breg[j];
-      }
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int i = 0; i < RM; ++i) af[i][k] = As[(16 * i + l16) * 16 + ((4 * q + 2 * h + k) ^ l16)];
     };
-    if (s > 0) __syncthreads();  // the last chunk of the segment before has been read
-    fetch(c_begin, lds);
-    stash(lds);
-    int buf = 0;
-    for (int c = c_begin; c < c_end; ++c) {
-      // chunk c has landed for every wave, and every wave is done reading the other stage
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      const double2* As = lds + buf * STAGE;
-      const double2* Bs = As + A_SLOTS;
-      buf ^= 1;
-      // all fragments of the chunk before the next loads start: an LDS read after
-      // them would wait for them
-      double2 bf[NT_RN][2], af[RM][4];
+    auto multiply = [&](const v2d (&af)[RM][2], const v2d (&bf)[NT_RN]) {
 #pragma unroll
-      for (int j = 0; j < NT_RN; ++j)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          bf[j][h] = Bs[(wave * 16 * NT_RN + 16 * j + l16) * 8 + ((2 * q + h) ^ (l16 & 7))];
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int i = 0; i < RM; ++i) af[i][k] = As[(16 * i + l16) * 16 + ((4 * q + k) ^ l16)];
-      if (c + 1 < c_end) fetch(c + 1, lds + buf * STAGE);
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < 2; ++k)
 #pragma unroll
         for (int i = 0; i < RM; ++i)
 #pragma unroll
           for (int j = 0; j < NT_RN; ++j) {
-            const double b = (k & 1) ? bf[j][k >> 1].y : bf[j][k >> 1].x;
-            re[i][j] = mfma64(af[i][k].x, b, re[i][j]);
-            im[i][j] = mfma64(af[i][k].y, b, im[i][j]);
+            re[i][j] = mfma64(af[i][k][0], bf[j][k], re[i][j]);
+            im[i][j] = mfma64(af[i][k][1], bf[j][k], im[i][j]);
           }
-      if (c + 1 < c_end) stash(lds + buf * STAGE);
+    };
+    // Each half's fragments are read while the other half is multiplied.  Between
+    // the halves of chunk c: chunk c + 1 has landed for every wave (the later
+    // ones stay in flight) and every wave has read all of chunk c, whose stage
+    // takes chunk c + ST.
+    v2d af0[RM][2], bf0[NT_RN], af1[RM][2], bf1[NT_RN];
+    for (int t = 0; t < ST; ++t) fetch(c_begin + t);
+    nt_barrier<(ST - 1) * P::LOADS>();
+    read(c_begin, 0, af0, bf0);
+    for (int c = c_begin; c < c_end; ++c) {
+      read(c, 1, af1, bf1);
+      multiply(af0, bf0);
+      __builtin_amdgcn_sched_barrier(0);
+      nt_barrier<(ST - 2) * P::LOADS>();
+      __builtin_amdgcn_sched_barrier(0);
+      read(c + 1, 0, af0, bf0);
+      fetch(c + ST);
+      multiply(af1, bf1);
+      // the reads, then the loads with their address arithmetic spread over the MFMAs
+      __builtin_amdgcn_sched_group_barrier(0x100, 2 * RM + NT_RN, 0);
+      constexpr int MF = 4 * RM * NT_RN, PER = P::LOADS > MF ? 2 : 1;
+#pragma unroll
+      for (int t = 0; t < (P::LOADS + PER - 1) / PER; ++t) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x006, 12 * PER, 0);
+        __builtin_amdgcn_sched_group_barrier(0x010, PER, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    nt_barrier<0>();
   }
 
 #pragma unroll
@@ -202,10 +241,10 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
 // Cost of a launch in units of one 16-row tile's MFMA time per K chunk (1024
 // cycles): the workgroups of the fullest CU (a fraction of one once there are
 // many rounds), each its chunks and about two chunks' worth of start and
-// epilogue, a tenth of a tile per chunk for the B columns each row tile reads again.
+// epilogue, a quarter of a tile per chunk for the B columns each row tile reads again.
 double nt_cost(int64_t m, int64_t colblocks, int rm, double chunks) {
   const double rounds = (double)(ceil_div(m, 16 * rm) * colblocks) / 256.0;
-  return (rounds < 4.0 ? std::ceil(rounds) : rounds) * (chunks + 2.0) * (rm + 0.1);
+  return (rounds < 4.0 ? std::ceil(rounds) : rounds) * (chunks + 2.0) * (rm + 0.25);
 }
 
 // Rows per workgroup tile, in 16s (1 .. most): the least padding of m on a full
@@ -219,43 +258,41 @@ int nt_rows(int64_t m, int64_t colblocks, double chunks, int most) {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-template <int RM, int EPI>
-hipError_t launch_nt_rm(const NtArgs& a, bool direct, dim3 grid, hipStream_t stream) {
-  if (direct) hipLaunchKernelGGL((nt64_kernel<RM, NT_DIRECT, EPI>), grid, dim3(NT_THREADS), 0, stream, a);
-  else hipLaunchKernelGGL((nt64_kernel<RM, NT_BREG, EPI>), grid, dim3(NT_THREADS), 0, stream, a);
+template <int RM, int MODE, int EPI>
+hipError_t launch_nt_mode(const NtArgs& a, hipStream_t stream) {
+  using P = NtPlan<RM, MODE>;
+  const int64_t blocks = ceil_div(a.n, NT_TN) * ceil_div(a.m, P::TM);
+  if (blocks > INT32_MAX || a.ksplit > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((nt64_kernel<RM, MODE, EPI>), dim3((unsigned)blocks, a.ksplit), dim3(NT_THREADS), P::LDS_BYTES,
+                     stream, a);
   return hipGetLastError();
+}
+
+template <int RM, int EPI>
+hipError_t launch_nt_rm(const NtArgs& a, bool direct, hipStream_t stream) {
+  return direct ? launch_nt_mode<RM, NT_16, EPI>(a, stream) : launch_nt_mode<RM, NT_B4, EPI>(a, stream);
 }
 
 template <int EPI>
 hipError_t launch_nt(const NtArgs& a, hipStream_t stream) {
   if (a.m < 1 || a.n < 1 || a.nseg < 1 || a.nseg > 2 || a.ksplit < 1) return hipErrorInvalidValue;
   bool a_vec = true, b_vec = true;
+  int64_t chunks = 0;
   for (int s = 0; s < a.nseg; ++s) {
     const NtSegment& g = a.seg[s];
     // 32-bit byte offsets within a tile (64 complex rows, 128 real columns)
     if (g.K < 1 || g.lda < g.K || g.ldb < g.K || g.lda > (1 << 22) || g.ldb > (1 << 22)) return hipErrorInvalidValue;
     a_vec = a_vec && aligned16(g.A);
     b_vec = b_vec && g.K % 2 == 0 && g.ldb % 2 == 0 && aligned16(g.B);
+    chunks += ceil_div(g.K, NT_KC);
   }
-  const int64_t nbn = ceil_div(a.n, NT_TN);
-  int64_t chunks = 0;
-  for (int s = 0; s < a.nseg; ++s) chunks += ceil_div(a.seg[s].K, NT_KC);
-  // (64 rows do not fit the registers beside B's)
-  const int rm = a_vec ? nt_rows(a.m, nbn * a.ksplit, (double)chunks / a.ksplit, b_vec ? 4 : 3) : 1;
-  const int64_t blocks = nbn * ceil_div(a.m, 16 * rm);
-  if (blocks > INT32_MAX || a.ksplit > 65535) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)blocks, a.ksplit);
-  if (!a_vec) {
-    hipLaunchKernelGGL((nt64_kernel<1, NT_REG, EPI>), grid, dim3(NT_THREADS), 0, stream, a);
-    return hipGetLastError();
-  }
-  switch (rm) {
-    case 1: return launch_nt_rm<1, EPI>(a, b_vec, grid, stream);
-    case 2: return launch_nt_rm<2, EPI>(a, b_vec, grid, stream);
-    case 3: return launch_nt_rm<3, EPI>(a, b_vec, grid, stream);
-    default:
-      hipLaunchKernelGGL((nt64_kernel<4, NT_DIRECT, EPI>), grid, dim3(NT_THREADS), 0, stream, a);
-      return hipGetLastError();
+  if (!a_vec) return launch_nt_mode<1, NT_AB4, EPI>(a, stream);
+  // (the 4-byte loads' addresses and 64 rows do not fit the registers together)
+  switch (nt_rows(a.m, ceil_div(a.n, NT_TN) * a.ksplit, (double)chunks / a.ksplit, b_vec ? 4 : 3)) {
+    case 1: return launch_nt_rm<1, EPI>(a, b_vec, stream);
+    case 2: return launch_nt_rm<2, EPI>(a, b_vec, stream);
+    case 3: return launch_nt_rm<3, EPI>(a, b_vec, stream);
+    default: return launch_nt_mode<4, NT_16, EPI>(a, stream);
   }
 }
 
