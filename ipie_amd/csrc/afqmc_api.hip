@@ -72,7 +72,8 @@ struct afqmc_ctx {
   // exchange as g^T Wq g (when Wq fits the budget and N < X)
   bool quad_on = false;
   bool quad_ready = false;                    // Wq holds the current static tensors
-  double* qw64[2] = {nullptr, nullptr};       // FP64 Wq per spin [n_s N, n_s N]
+  double* qw64[2] = {nullptr, nullptr};       // FP64 W' per spin [n_s N, quad64_ld]
+  int quad64_chunks[2] = {0, 0};              // K chunks of its column units
   uint16_t* qwp[2] = {nullptr, nullptr};      // split-BF16 Wq per spin 2 x [n_s Kp, n_s Kp]
   // FP8 quadratic form of the control variate (made on first use): W' per spin
   // [q8_ld][q8_ld] bytes, q8_ld = n_s Kp rounded up to 64; the scales s_w (FP32,
@@ -86,9 +87,9 @@ struct afqmc_ctx {
   bool q8_ready = false;
   int4* qunits8[2] = {nullptr, nullptr};
   std::vector<int> qunit8_off[2], qunit8_n[2];
-  double* qy = nullptr;                       // FP64: Y = G Wq [W, n N]; BF16: dot partials [slots, W] (complex)
-  int4* qunits[2] = {nullptr, nullptr};       // BF16 column units per spin, one table per row-block count
-  std::vector<int> qunit_off[2], qunit_n[2];  // [mb - 1]: offset and length of the table for mb row blocks
+  double* qy = nullptr;                       // dot partials [slots, W] (complex)
+  int4* qunits[2] = {nullptr, nullptr};       // column units per spin (BF16: one table per row-block count; FP64: one)
+  std::vector<int> qunit_off[2], qunit_n[2];  // BF16 [mb - 1]: offset and length of the table for mb row blocks
   int xs_used[2] = {1, 1};  // partial-sum count of the last exchange per spin
   // launch shapes that afqmc_tune_set may change (heuristic defaults)
   int fb_split_spin = BF16_FB_SPLIT;  // split-BF16 force bias: K ranges per spin
@@ -234,6 +235,12 @@ int check_ready(afqmc_ctx* c, int32_t nw) {
   return AFQMC_OK;
 }
 
+// row length of the FP64 W' of a spin: even, so that every row is 16-byte aligned
+int64_t quad64_ld(const afqmc_ctx* c, int spin) {
+  const int64_t nN = (int64_t)(spin == 0 ? c->d.nalpha : c->d.nbeta) * c->d.nbasis;
+  return nN + nN % 2;
+}
+
 bool two_spins(const afqmc_ctx* c) { return c->d.nbeta > 0 && !c->d.rhf; }
 
 double* wv(afqmc_ctx* c, int i) { return c->wvec + 2 * (int64_t)i * c->d.nwalkers; }
@@ -302,9 +309,9 @@ int alloc_exchange_planes(afqmc_ctx* c) {
   return AFQMC_OK;
 }
 
-// Column-unit tables of the split-BF16 quadratic form for every row-block
-// count (quad_units with c->quad_target), and the dot-partial buffer qy sized
-// for the largest table.  A rebuild (afqmc_tune_set) keeps the tables and qy it
+// Column-unit tables of the quadratic form (FP64: one per spin, nt64_quad_units;
+// split-BF16: one for every row-block count, quad_units with c->quad_target), and
+// the dot-partial buffer qy sized for the largest table.  A rebuild (afqmc_tune_set) keeps the tables and qy it
 // replaces alive until afqmc_destroy: a graph captured before still uses them.
 int build_quad_units(afqmc_ctx* c) {
   const int64_t W = c->d.nwalkers;
@@ -312,7 +319,15 @@ int build_quad_units(afqmc_ctx* c) {
   // [0, 1]: BF16 tables (32-value chunks) per spin; [2, 3]: FP8 (64-value chunks)
   std::vector<int4> all[4];
   std::vector<int> off[4], cnt[4];
+  int64_t slots = QUAD_SLOTS;
   for (int s = 0; s < 2; ++s) {
+    if (c->qw64[s]) {
+      c->quad64_chunks[s] = nt64_quad_units(W, (int64_t)(s == 0 ? c->d.nalpha : c->d.nbeta) * c->d.nbasis, all[s]);
+      cnt[s].push_back((int)all[s].size());
+      off[s].push_back(0);
+      max_units = std::max<int64_t>(max_units, (int64_t)all[s].size());
+      slots = 1;
+    }
     if (!c->qwp[s]) continue;
     const int64_t ldn = (int64_t)(s == 0 ? c->d.nalpha : c->d.nbeta) * c->kpad;
     for (int f = 0; f < 2; ++f) {
@@ -328,7 +343,7 @@ int build_quad_units(afqmc_ctx* c) {
     }
   }
   if (max_units == 0) return AFQMC_OK;
-  const int64_t need = max_units * QUAD_SLOTS * W;
+  const int64_t need = max_units * slots * W;
   if (need > c->qy_cap) {
     double* qy = nullptr;
     if (dmalloc((void**)&qy, 16 * (size_t)need) != hipSuccess)
@@ -394,11 +409,8 @@ int ensure_ws(afqmc_ctx* c) {
     for (int s = 0; s < (two_spins(c) ? 2 : 1); ++s) {
       const int64_t rows = (int64_t)(s == 0 ? d.nalpha : d.nbeta) * Np;
       if (mixed) ok = ok && dmalloc((void**)&c->qwp[s], 2 * (size_t)2 * rows * rows) == hipSuccess;
-      else ok = ok && dmalloc((void**)&c->qw64[s], 8 * (size_t)rows * rows) == hipSuccess;
+      else ok = ok && dmalloc((void**)&c->qw64[s], 8 * (size_t)rows * quad64_ld(c, s)) == hipSuccess;
     }
-    // FP64: Y = G Wq; split-BF16: QUAD_SLOTS dot partials per column unit, sized
-    // with the unit tables (build_quad_units)
-    if (!mixed) ok = ok && dmalloc((void**)&c->qy, 16 * (size_t)W * nmax * Np) == hipSuccess;
   }
   // FP64 VHS [W, N, N] complex (2.6 GB at N=400); the split-BF16 path keeps VHS as atoms only
   if (d.precision != AFQMC_PREC_MIXED) ok = ok && dmalloc((void**)&c->vhs, 16 * (size_t)W * N * N) == hipSuccess;
@@ -853,8 +865,8 @@ int ensure_quad(afqmc_ctx* c) {
   for (int s = 0; s < (two_spins(c) ? 2 : 1); ++s) {
     const int n = s == 0 ? c->d.nalpha : c->d.nbeta;
     const double* rchol = s == 0 ? c->s.rchola : c->s.rcholb;
-    if (c->qwp[s]) HIP_TRY(c, launch_quad_w(rchol, c->d.nchol, n, N, c->kpad, nullptr, c->qwp[s], c->stream));
-    else HIP_TRY(c, launch_quad_w(rchol, c->d.nchol, n, N, N, c->qw64[s], nullptr, c->stream));
+    if (c->qwp[s]) HIP_TRY(c, launch_quad_w(rchol, c->d.nchol, n, N, c->kpad, nullptr, 0, c->qwp[s], c->stream));
+    else HIP_TRY(c, launch_quad_w(rchol, c->d.nchol, n, N, N, c->qw64[s], quad64_ld(c, s), nullptr, c->stream));
   }
   c->quad_ready = true;
   return AFQMC_OK;
@@ -989,8 +1001,9 @@ int quad_bf16(afqmc_ctx* c, int nw, int spin, const double* g, const int* walker
   return AFQMC_OK;
 }
 
-// Exchange of nw walkers for one spin as g^T Wq g: Y = G Wq (FP64 NT GEMM, or
-// split-BF16 GEMM with split K), then one dot product per walker.
+// Exchange of nw walkers for one spin as g^T Wq g: Y = G W' over the column units of
+// the block-triangular W' (FP64 or split-BF16) with the dot products in the
+// epilogue, then their sum per walker.
 int exchange_spin_quad(afqmc_ctx* c, int nw, int spin, const double* g, const int* walker_of) {
   const int N = c->d.nbasis;
   const int n = spin == 0 ? c->d.nalpha : c->d.nbeta;
@@ -1012,11 +1025,14 @@ int exchange_spin_quad(afqmc_ctx* c, int nw, int spin, const double* g, const in
     a.n = nN;
     a.ksplit = 1;
     a.nseg = 1;
-    a.seg[0] = NtSegment{g, nN, c->qw64[spin], nN, (int)nN};
-    a.scale = 1.0;
+    a.seg[0] = NtSegment{g, nN, c->qw64[spin], quad64_ld(c, spin), (int)nN};
     a.out = c->qy;
+    a.units = c->qunits[spin];
+    a.nunits = c->qunit_n[spin][0];
+    a.unit_chunks = c->quad64_chunks[spin];
+    a.dg = g;
     HIP_TRY(c, launch_nt64(a, c->stream));
-    HIP_TRY(c, launch_quad_reduce(c->qy, 1, nw, n, N, N, g, nullptr, part, c->stream));
+    HIP_TRY(c, launch_quad_sum(c->qy, a.nunits, nw, part, c->stream));
   }
   c->xs_used[spin] = 1;
   return AFQMC_OK;

@@ -1,6 +1,8 @@
 // Internal (non-exported) declarations shared by the kernel translation units.
 #pragma once
 
+#include <vector>
+
 #include "afqmc_common.hpp"
 
 namespace afqmc {
@@ -92,12 +94,25 @@ struct NtArgs {
   const int* tri_i;
   const int* tri_j;
   int nbasis;
+  // quadratic form (n = K): column units {tile, first chunk, end chunk, 0} from
+  // nt64_quad_units, or null; out[unit][m] = sum over the unit's columns c of
+  // dg[r, c] sum_{k in the unit's chunks} A[r, k] B[c, k] (dg [m, n] complex)
+  const int4* units;
+  int nunits, unit_chunks;
+  const double* dg;
 };
 hipError_t launch_nt64(const NtArgs& a, hipStream_t stream);
 // K ranges (1 .. most) for an [m, n] product over `chunks` 16-wide K chunks: enough
 // workgroups to fill the GPU and rounds that end together, against the
 // partial sums each range adds
 int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, int most);
+// Column units of the block-triangular quadratic form of m rows and n = K columns:
+// tile t of QUAD64_TILE columns sums the chunks up to its own columns' end, cut into
+// units of T chunks (returned; 4 .. 64, the largest that still fills the GPU),
+// listed by K range, then tile, so that the workgroups that run together read the
+// same range of A.
+int nt64_quad_units(int64_t m, int64_t n, std::vector<int4>& units);
+constexpr int QUAD64_TILE = 128;  // column tile of the FP64 W'
 constexpr int FB_MAX_SPLIT = 16;  // most K ranges of the FP64 force bias (heuristic)
 
 // Batched C[w] = A[w] * B[w] with A [N, N] (real shared or complex per walker)
@@ -222,19 +237,15 @@ constexpr double QUAD_BUDGET_BYTES = 24e9;  // largest Wq per spin held on the d
 constexpr int QUAD_TILE = 160;
 // Partial dot products written per column unit by the QDOT epilogue.
 constexpr int QUAD_SLOTS = 2;
-// Wq[(i,m'),(j,m)] = sum_x L_x[i][m] L_x[j][m'] from rchol [X, n, N]: FP64 [nN][nN]
-// (Np = N), or split-BF16 planes [2][n Np][n Np] (Np = Kp, zero padding) of the
-// block-triangular W' with plane row b, column a: W'_ab = 2 Wq_ab when tile(a) <
-// tile(b), Wq_ab when tile(a) = tile(b), 0 otherwise (tile(a) = a / QUAD_TILE),
-// so that g^T Wq g = sum_b g_b sum_{a < QUAD_TILE (tile(b) + 1)} g_a W'_ab.
-// Exactly one of w64 / wplanes is non-null.
-hipError_t launch_quad_w(const double* rchol, int X, int n, int N, int Np, double* w64, uint16_t* wplanes,
-                         hipStream_t stream);
-// part[w] = sum_z sum_{i, m < N} d[i][m] y[z][w][i Np + m], d = g[src] - gref (gref
-// [n, N] or null), src = walker_of[w] or w
-hipError_t launch_quad_reduce(const double* y, int ksplit, int nwalkers, int n, int N, int Np, const double* g,
-                              const int* walker_of, double* part, hipStream_t stream,
-                              const double* gref = nullptr);
+// Wq[(i,m'),(j,m)] = sum_x L_x[i][m] L_x[j][m'] from rchol [X, n, N], as the
+// block-triangular W' with row b, column a: W'_ab = 2 Wq_ab when tile(a) < tile(b),
+// Wq_ab when tile(a) = tile(b), 0 otherwise (tile(a) = a / T), so that
+// g^T Wq g = sum_b g_b sum_{a < T (tile(b) + 1)} g_a W'_ab.  Either FP64 rows of
+// length ld64 (Np = N, T = QUAD64_TILE; columns past the row's tile are not
+// written), or split-BF16 planes [2][n Np][n Np] (Np = Kp, zero padding, T =
+// QUAD_TILE).  Exactly one of w64 / wplanes is non-null.
+hipError_t launch_quad_w(const double* rchol, int X, int n, int N, int Np, double* w64, int64_t ld64,
+                         uint16_t* wplanes, hipStream_t stream);
 // out[w] = sum_{s < nslots} part[s][w] (complex, fixed order)
 hipError_t launch_quad_sum(const double* part, int nslots, int nwalkers, double* out, hipStream_t stream);
 // FP8 (E4M3) copy of the block-triangular W' for the control variate's single

@@ -6,7 +6,8 @@
 //                  triangle, written to both triangles
 //                  (ipie/propagation/phaseless_generic.py:67-97,
 //                   ipie/utils/pack_numba.py:22-33)
-//   * the exchange's Y = G Wq
+//   * the exchange as a quadratic form, sum_b g_b (G W')_b over the block-triangular
+//     W' (k_quad.hip), the dot products in the epilogue
 //
 // What bounds it: one 16x16x4 FP64 MFMA takes 64 cycles on gfx950, so the matrix
 // pipe is the limit as soon as a wave always has its operands in registers.
@@ -43,11 +44,12 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 constexpr int NT_KC = 16;                // K per LDS stage
 constexpr int NT_RN = 2, NT_WAVES = 4;   // 16-column tiles per wave, waves side by side
 constexpr int NT_TN = 16 * NT_RN * NT_WAVES;
+static_assert(NT_TN == QUAD64_TILE, "column tile of W'");
 constexpr int NT_THREADS = 64 * NT_WAVES;
 
 __device__ double2 nt_zero;  // source of the slots past K
 
-enum { NT_EPI_PART = 0, NT_EPI_VHS = 1 };
+enum { NT_EPI_PART = 0, NT_EPI_VHS = 1, NT_EPI_QDOT = 2 };
 
 // Direct global-to-LDS loads: lane l's 16 (4) bytes go to dst + 16 l (4 l).
 __device__ __forceinline__ void nt_load16(const char* src, void* dst) {
@@ -91,7 +93,11 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
   const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
   const int nbm = (int)ceil_div(a.m, TM);
   const int lin = xcd_remap(blockIdx.x, gridDim.x);
-  const int bm = lin % nbm, bn = lin / nbm, z = blockIdx.y;
+  // (QDOT: row blocks x column units, otherwise x column tiles, with K ranges in y)
+  const int bm = lin % nbm, bu = lin / nbm, z = blockIdx.y;
+  int4 unit = make_int4(bu, 0, 0, 0);
+  if (EPI == NT_EPI_QDOT) unit = a.units[bu];
+  const int bn = unit.x;
   const int row0 = bm * TM;
   const int64_t col0 = (int64_t)bn * NT_TN;
 
@@ -110,7 +116,11 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
   const int z0 = (int)((int64_t)nch * z / a.ksplit), z1 = (int)((int64_t)nch * (z + 1) / a.ksplit);
   for (int s = 0; s < a.nseg; ++s) {
     const NtSegment sg = s == 0 ? a.seg[0] : a.seg[1];
-    const int c_begin = s == 0 ? z0 : max(z0, nch0) - nch0, c_end = s == 0 ? min(z1, nch0) : z1 - nch0;
+    int c_begin = s == 0 ? z0 : max(z0, nch0) - nch0, c_end = s == 0 ? min(z1, nch0) : z1 - nch0;
+    if (EPI == NT_EPI_QDOT) {
+      c_begin = unit.y;
+      c_end = unit.z;
+    }
     if (c_begin >= c_end) continue;
     // sources of this lane: byte offsets from the tile's first row and column
     // (rows and columns past the end read the last one; their results are not
@@ -210,6 +220,37 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
     nt_barrier<0>();
   }
 
+  if (EPI == NT_EPI_QDOT) {
+    // per row: the dot of this wave's 32 columns with d, summed over the 16 lanes
+    // of the row, then over the waves (LDS is free: every wave passed the last barrier)
+    double2* part = reinterpret_cast<double2*>(nt_lds);  // [wave][row]
+#pragma unroll
+    for (int i = 0; i < RM; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * i + 4 * r + q;
+        const int64_t w = min((int64_t)row0 + row, a.m - 1);
+        cplx e = cmake(0.0, 0.0);
+#pragma unroll
+        for (int j = 0; j < NT_RN; ++j) {
+          const int64_t c = col0 + wave * 16 * NT_RN + 16 * j + l16;
+          if (c < a.n) cfma(e, ld(a.dg, w * a.n + c), cmake(re[i][j][r], im[i][j][r]));
+        }
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) {
+          e.re += __shfl_xor(e.re, off, 64);
+          e.im += __shfl_xor(e.im, off, 64);
+        }
+        if (l16 == 0) part[wave * TM + row] = make_double2(e.re, e.im);
+      }
+    __syncthreads();
+    if (threadIdx.x < TM && row0 + (int64_t)threadIdx.x < a.m) {
+      cplx e = cmake(0.0, 0.0);
+      for (int v = 0; v < NT_WAVES; ++v) e = cadd(e, ld(reinterpret_cast<const double*>(part), v * TM + threadIdx.x));
+      st(a.out, (int64_t)bu * a.m + row0 + threadIdx.x, e);
+    }
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < NT_RN; ++j) {
     const int64_t c = col0 + wave * 16 * NT_RN + 16 * j + l16;
@@ -256,12 +297,15 @@ int nt_rows(int64_t m, int64_t colblocks, double chunks, int most) {
   return best;
 }
 
+// what the dot products of a unit add to its start and end, in chunks
+constexpr double NT_QDOT_CHUNKS = 3.0;
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <int RM, int MODE, int EPI>
 hipError_t launch_nt_mode(const NtArgs& a, hipStream_t stream) {
   using P = NtPlan<RM, MODE>;
-  const int64_t blocks = ceil_div(a.n, NT_TN) * ceil_div(a.m, P::TM);
+  const int64_t blocks = (EPI == NT_EPI_QDOT ? a.nunits : ceil_div(a.n, NT_TN)) * ceil_div(a.m, P::TM);
   if (blocks > INT32_MAX || a.ksplit > 65535) return hipErrorInvalidValue;
   hipLaunchKernelGGL((nt64_kernel<RM, MODE, EPI>), dim3((unsigned)blocks, a.ksplit), dim3(NT_THREADS), P::LDS_BYTES,
                      stream, a);
@@ -287,8 +331,10 @@ hipError_t launch_nt(const NtArgs& a, hipStream_t stream) {
     chunks += ceil_div(g.K, NT_KC);
   }
   if (!a_vec) return launch_nt_mode<1, NT_AB4, EPI>(a, stream);
+  const int64_t colblocks = EPI == NT_EPI_QDOT ? a.nunits : ceil_div(a.n, NT_TN) * a.ksplit;
+  const double each = EPI == NT_EPI_QDOT ? a.unit_chunks + NT_QDOT_CHUNKS : (double)chunks / a.ksplit;
   // (the 4-byte loads' addresses and 64 rows do not fit the registers together)
-  switch (nt_rows(a.m, ceil_div(a.n, NT_TN) * a.ksplit, (double)chunks / a.ksplit, b_vec ? 4 : 3)) {
+  switch (nt_rows(a.m, colblocks, each, b_vec ? 4 : 3)) {
     case 1: return launch_nt_rm<1, EPI>(a, b_vec, stream);
     case 2: return launch_nt_rm<2, EPI>(a, b_vec, stream);
     case 3: return launch_nt_rm<3, EPI>(a, b_vec, stream);
@@ -315,7 +361,37 @@ int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, int most) {
   return best;
 }
 
+int nt64_quad_units(int64_t m, int64_t n, std::vector<int4>& units) {
+  const int64_t kchunks = ceil_div(n, NT_KC), tiles = ceil_div(n, NT_TN);
+  auto extent = [&](int64_t t) { return std::min<int64_t>((t + 1) * (NT_TN / NT_KC), kchunks); };
+  auto count = [&](int T) {
+    int64_t u = 0;
+    for (int64_t t = 0; t < tiles; ++t) u += ceil_div(extent(t), T);
+    return u;
+  };
+  int best = 0;
+  double least = 0.0;
+  for (int T = 64; T >= 4; T /= 2) {
+    const double each = T + NT_QDOT_CHUNKS;
+    const double cost = nt_cost(m, count(T), nt_rows(m, count(T), each, 4), each);
+    if (best == 0 || cost < 0.98 * least) {
+      best = T;
+      least = cost;
+    }
+  }
+  units.clear();
+  for (int64_t z = 0; z * best < kchunks; ++z)
+    for (int64_t t = 0; t < tiles; ++t)
+      if (z * best < extent(t))
+        units.push_back(make_int4((int)t, (int)(z * best), (int)std::min<int64_t>((z + 1) * best, extent(t)), 0));
+  return best;
+}
+
 hipError_t launch_nt64(const NtArgs& a, hipStream_t stream) {
+  if (a.units) {
+    if (a.nseg != 1 || a.ksplit != 1 || a.nunits < 1 || a.seg[0].K != a.n) return hipErrorInvalidValue;
+    return launch_nt<NT_EPI_QDOT>(a, stream);
+  }
   return a.tri_i ? launch_nt<NT_EPI_VHS>(a, stream) : launch_nt<NT_EPI_PART>(a, stream);
 }
 

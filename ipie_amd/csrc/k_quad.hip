@@ -9,14 +9,13 @@
 // is one GEMM Y = G Wq (M = W, N = K = n N) and a dot product per walker, about
 // X / N times fewer flops than forming every T_x (and no n x n trace epilogue).
 // Same value as ipie/estimators/local_energy_sd.py:263-303 (exx_kernel_batch_real_rchol).
-// Wq's symmetry halves the BF16 form: with column tiles of QUAD_TILE, the planes
-// hold W' = Wq on the diagonal tiles, 2 Wq above them and 0 below, and column
+// Wq's symmetry halves it: with column tiles of T (QUAD64_TILE in FP64, QUAD_TILE in
+// BF16), W' = Wq on the diagonal tiles, 2 Wq above them and 0 below, and column
 // tile b of Y = G W' sums K over the tiles up to b only (g^T W' g = g^T Wq g).
-//   quad_w_kernel       Wq from rchol, FP64 accumulation, written as FP64 [nN][nN]
-//                       or as the split-BF16 planes of W' [2][n Kp][n Kp] (zero padding)
-//   quad_reduce_kernel  E_w = sum_z sum_a g_w[a] Y_z[w][a]  (FP64 form)
-//   quad_sum_kernel     E_w = sum of the per-tile dot products written by the
-//                       BF16 GEMM's epilogue
+//   quad_w_kernel       W' from rchol, FP64 accumulation, written in FP64 or as
+//                       split-BF16 planes [2][n Kp][n Kp] (zero padding)
+//   quad_sum_kernel     E_w = sum of the per-unit dot products written by the
+//                       products' epilogues
 #include "afqmc_internal.hpp"
 
 namespace afqmc {
@@ -33,11 +32,14 @@ __device__ __forceinline__ uint16_t qf2bf(float f) {
 }
 __device__ __forceinline__ float qbf2f(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 
-// One 64 x 64 tile of Wq for the orbital pair (i, j): rows a = (i, m'), columns
-// b = (j, m); out[a][b] = sum_x R[x][j][m'] R[x][i][m].  Np is the column
-// stride per orbital of the output (N for FP64, Kp for the padded planes).
+// One 64 x 64 tile of W' for the orbital pair (i, j): rows a = (i, m'), columns
+// b = (j, m); out[a][b] = f sum_x R[x][j][m'] R[x][i][m].  Np is the column
+// stride per orbital of the output (N for FP64, Kp for the padded planes).  In
+// FP64 the tiles past their rows' column tile, which nothing reads, are skipped:
+// half the products.
 __global__ void __launch_bounds__(256) quad_w_kernel(const double* __restrict__ R, int X, int n, int N, int Np,
-                                                    double* __restrict__ w64, uint16_t* __restrict__ wplanes) {
+                                                    double* __restrict__ w64, int64_t ld64,
+                                                    uint16_t* __restrict__ wplanes) {
   __shared__ double fa[QW_XC][QW_T];  // R[x][j][m' range]
   __shared__ double fb[QW_XC][QW_T];  // R[x][i][m range]
   const int mblocks = (Np + QW_T - 1) / QW_T;
@@ -48,6 +50,7 @@ __global__ void __launch_bounds__(256) quad_w_kernel(const double* __restrict__ 
   blk /= mblocks;
   const int j = blk % n, i = blk / n;
   const int m0a = ma * QW_T, m0b = mb * QW_T;
+  if (w64 && ((int64_t)j * Np + m0b) / QUAD64_TILE > ((int64_t)i * Np + min(m0a + QW_T, N) - 1) / QUAD64_TILE) return;
   const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
   double acc[4][4];
 #pragma unroll
@@ -90,7 +93,7 @@ __global__ void __launch_bounds__(256) quad_w_kernel(const double* __restrict__ 
       if (m >= Np) continue;
       const int64_t b = (int64_t)j * Np + m;
       if (w64) {
-        w64[a * ldo + b] = acc[r][c];
+        w64[a * ld64 + b] = (b / QUAD64_TILE < a / QUAD64_TILE ? 2.0 : 1.0) * acc[r][c];
       } else {
         // plane row a is the output column, b the K index: W'_{b a}
         const int ta = (int)(a / QUAD_TILE), tb = (int)(b / QUAD_TILE);
@@ -103,36 +106,6 @@ __global__ void __launch_bounds__(256) quad_w_kernel(const double* __restrict__ 
       }
     }
   }
-}
-
-// E_w = sum_z sum_a d_w[a] Y_z[w][a]; Y index a = i Np + m (m < N used), d = g
-// from Ghalf [W, n, N] (or its sampled rows: walker_of), minus gref [n, N] when
-// given (the control variate's dG).  One workgroup per walker, result into
-// part[w] (complex).
-__global__ void __launch_bounds__(256) quad_reduce_kernel(const double* __restrict__ y, int ksplit, int nwalkers,
-                                                         int n, int N, int Np, const double* __restrict__ g,
-                                                         const int* __restrict__ walker_of,
-                                                         double* __restrict__ part, const double* __restrict__ gref) {
-  __shared__ double red[256 / 64];
-  const int w = blockIdx.x;
-  const int64_t ldy = (int64_t)n * Np;
-  const int src = walker_of ? walker_of[w] : w;
-  const double* gw = g + 2 * (int64_t)src * n * N;
-  double re = 0.0, im = 0.0;
-  for (int z = 0; z < ksplit; ++z) {
-    const double* yw = y + 2 * ((int64_t)z * nwalkers + w) * ldy;
-    for (int64_t e = threadIdx.x; e < (int64_t)n * N; e += blockDim.x) {
-      const int i = (int)(e / N), m = (int)(e % N);
-      cplx gv = ld(gw, e);
-      if (gref) gv = csub(gv, ld(gref, e));
-      const cplx yv = ld(yw, (int64_t)i * Np + m);
-      re += gv.re * yv.re - gv.im * yv.im;
-      im += gv.re * yv.im + gv.im * yv.re;
-    }
-  }
-  re = block_sum(re, red);
-  im = block_sum(im, red);
-  if (threadIdx.x == 0) st(part, w, cmake(re, im));
 }
 
 // out[w] = sum_s part[s][w]: WL walkers x 256 / WL slot lanes per workgroup, the
@@ -354,19 +327,14 @@ hipError_t launch_quad_sum(const double* part, int nslots, int nwalkers, double*
   return hipGetLastError();
 }
 
-hipError_t launch_quad_w(const double* rchol, int X, int n, int N, int Np, double* w64, uint16_t* wplanes,
-                         hipStream_t stream) {
+hipError_t launch_quad_w(const double* rchol, int X, int n, int N, int Np, double* w64, int64_t ld64,
+                         uint16_t* wplanes, hipStream_t stream) {
   if ((w64 == nullptr) == (wplanes == nullptr) || Np < N) return hipErrorInvalidValue;
+  if (w64 && (Np != N || ld64 < (int64_t)n * N)) return hipErrorInvalidValue;
   const int64_t mblocks = ceil_div(Np, QW_T);
   const int64_t grid = (int64_t)n * n * mblocks * mblocks;
-  hipLaunchKernelGGL(quad_w_kernel, dim3((unsigned)grid), dim3(256), 0, stream, rchol, X, n, N, Np, w64, wplanes);
-  return hipGetLastError();
-}
-
-hipError_t launch_quad_reduce(const double* y, int ksplit, int nwalkers, int n, int N, int Np, const double* g,
-                              const int* walker_of, double* part, hipStream_t stream, const double* gref) {
-  hipLaunchKernelGGL(quad_reduce_kernel, dim3(nwalkers), dim3(256), 0, stream, y, ksplit, nwalkers, n, N, Np, g,
-                     walker_of, part, gref);
+  hipLaunchKernelGGL(quad_w_kernel, dim3((unsigned)grid), dim3(256), 0, stream, rchol, X, n, N, Np, w64, ld64,
+                     wplanes);
   return hipGetLastError();
 }
 

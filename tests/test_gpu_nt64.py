@@ -91,3 +91,47 @@ def test_product_with_rows_off_sixteen_bytes():
     ctx._call("afqmc_force_bias", W, ctypes.c_void_p(bufs[0].data_ptr() + 8),
               ctypes.c_void_p(bufs[1].data_ptr() + 8), ctypes.c_void_p(out.data_ptr()))
     _check(out.cpu().numpy(), ra, rb, g, ctx.tune_get("fb_split")[0])
+
+
+# N, X, na, nb, W (X > N: the exchange as a quadratic form)
+QUAD_CASES = [
+    (4, 5, 2, 1, 1),        # less than a column tile
+    (16, 20, 8, 8, 17),     # one column tile exactly
+    (43, 50, 3, 3, 40),     # a column past a tile, odd n N
+    (33, 40, 31, 0, 130),   # eight tiles, the last one short, one spin
+    (60, 80, 20, 19, 70),   # several units per tile
+]
+
+
+@pytest.mark.parametrize("case", QUAD_CASES)
+def test_quadratic_form_at_tile_edges(case):
+    """Coulomb minus exchange of random walkers.  The sums over x, k and c and the
+    products of complex numbers are off by at most 4 (X + 2 n N) u of the same sums
+    of absolute values, on each side."""
+    import torch
+
+    N, X, na, nb, W = case
+    print(f"[case] nt64 quadratic form N={N} X={X} na={na} nb={nb} W={W}", flush=True)
+    ctx, dev, ra, rb, g = _context(N, X, na, nb, W)
+    assert ctx.exchange_form() == "quad"
+    ga, gb = (torch.from_numpy(x).to(dev) for x in g)
+    out = torch.empty(W, 3, dtype=torch.complex128, device=dev)
+    ctx.local_energy(ga, gb, out)
+    got = out.cpu().numpy()[:, 2]
+
+    def sums(mag):
+        coul, exx = 0.0, 0.0
+        for r, x in ((ra, g[0]), (rb, g[1])):
+            n = x.shape[1]
+            if n == 0:
+                continue
+            l, y = mag(r.reshape(X, n, N)), mag(x)
+            t = numpy.einsum("xim,wjm->wxij", l, y)
+            coul = coul + numpy.einsum("wxii->wx", t)
+            exx = exx + numpy.einsum("wxij,wxji->w", t, t)
+        return 0.5 * (coul * coul).sum(axis=1), 0.5 * exx
+
+    coul, exx = sums(lambda v: v)
+    ca, ea = sums(numpy.abs)
+    bound = 2 * 4 * (X + 2 * max(na, nb) * N) * 2.0**-53 * (ca + ea)
+    assert (numpy.abs(got - (coul - exx)) <= bound).all()
