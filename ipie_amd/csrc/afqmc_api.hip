@@ -39,9 +39,10 @@ struct afqmc_ctx {
   double* wvec = nullptr;        // 6 x [W] complex: cmf, cfb, ecoul, ovlp_old, ovlp_new, spare
   double* exx_a = nullptr;       // [xs_a, W] complex
   double* exx_b = nullptr;       // [xs_b, W] complex
-  double* vhs = nullptr;         // [W, N, N] complex
-  double* buf[4] = {nullptr, nullptr, nullptr, nullptr};  // P, Ta, Tb, Q: [W, N, ncol] complex
-  int* tri = nullptr;            // [2, P] packed-index rows / cols
+  double* vhs = nullptr;         // FP64: packed upper triangles [W, N (N + 1) / 2] complex
+  double* buf[4] = {nullptr, nullptr, nullptr, nullptr};  // P, Ta, Tb, Q (mixed): [W, N, ncol] complex
+  double* exp_pad = nullptr;     // FP64: expH1 [2, N, exp_ld], zero past N
+  bool exp_ready = false;        // exp_pad holds the current expH1
   int* flags = nullptr;
   int* wflags = nullptr;    // [W] per-walker flags (OR of AFQMC_FLAG_*) since the last take
   int* psi_flag = nullptr;  // scratch of afqmc_set_static's check of the trial orbitals
@@ -241,6 +242,9 @@ int64_t quad64_ld(const afqmc_ctx* c, int spin) {
   return nN + nN % 2;
 }
 
+// row length of the FP64 path's copy of expH1: whole K chunks, zero past N
+int exp_ld(const afqmc_ctx* c) { return (c->d.nbasis + 15) / 16 * 16; }
+
 bool two_spins(const afqmc_ctx* c) { return c->d.nbeta > 0 && !c->d.rhf; }
 
 double* wv(afqmc_ctx* c, int i) { return c->wvec + 2 * (int64_t)i * c->d.nwalkers; }
@@ -412,19 +416,16 @@ int ensure_ws(afqmc_ctx* c) {
       else ok = ok && dmalloc((void**)&c->qw64[s], 8 * (size_t)rows * quad64_ld(c, s)) == hipSuccess;
     }
   }
-  // FP64 VHS [W, N, N] complex (2.6 GB at N=400); the split-BF16 path keeps VHS as atoms only
-  if (d.precision != AFQMC_PREC_MIXED) ok = ok && dmalloc((void**)&c->vhs, 16 * (size_t)W * N * N) == hipSuccess;
-  for (int i = 0; i < 4; ++i) ok = ok && dmalloc((void**)&c->buf[i], 16 * (size_t)W * N * c->ncol) == hipSuccess;
-  ok = ok && dmalloc((void**)&c->tri, sizeof(int) * 2 * (size_t)P) == hipSuccess;
+  // FP64 VHS, packed upper triangles (1.3 GB at N=400); the split-BF16 path keeps VHS as atoms only
+  if (d.precision != AFQMC_PREC_MIXED) {
+    ok = ok && dmalloc((void**)&c->vhs, 16 * (size_t)W * P) == hipSuccess;
+    ok = ok && dmalloc((void**)&c->exp_pad, 8 * (size_t)2 * N * exp_ld(c)) == hipSuccess;
+  }
+  for (int i = 0; i < 4; ++i) {  // (the FP64 path takes three)
+    if (i == 3 && d.precision != AFQMC_PREC_MIXED) continue;
+    ok = ok && dmalloc((void**)&c->buf[i], 16 * (size_t)W * N * c->ncol) == hipSuccess;
+  }
   if (!ok) return fail(c, AFQMC_ERR_ALLOC, "workspace allocation failed (%s)", c->describe_dims);
-  std::vector<int> tri(2 * P);
-  int64_t p = 0;
-  for (int i = 0; i < N; ++i)
-    for (int j = i; j < N; ++j, ++p) {
-      tri[p] = i;
-      tri[P + p] = j;
-    }
-  HIP_TRY(c, hipMemcpy(c->tri, tri.data(), sizeof(int) * 2 * P, hipMemcpyHostToDevice));
   const int r = build_quad_units(c);
   if (r) return r;
   HIP_TRY(c, hipMemset(c->wvec, 0, 16 * (size_t)6 * W));
@@ -628,35 +629,41 @@ int do_vhs(afqmc_ctx* c, int nw) {
   a.seg[0] = NtSegment{c->xshifted, X, c->s.chol_packed, X, (int)X};
   a.scale = sqrt(c->s.dt);
   a.out = c->vhs;
-  a.tri_i = c->tri;
-  a.tri_j = c->tri + P;
-  a.nbasis = (int)N;
+  a.times_i = 1;
   PhaseScope ps(c, AFQMC_PHASE_VHS);
   HIP_TRY(c, launch_nt64(a, c->stream));
   return AFQMC_OK;
 }
 
-// C[w] (ldc, c_stride) = alpha * A * B[w] (ldb, b_stride), ncol columns.
-int nn(afqmc_ctx* c, int nw, const double* A, bool acplx, int64_t a_stride, const double* B, int64_t b_stride,
-       int64_t ldb, double* C, int64_t c_stride, int64_t ldc, int ncol, double alpha, double* accum,
-       const double* accum_init) {
-  BatchedNNArgs a;
+// FP64 one body of both spins: phi_s -> the concatenated buffer dst (gather) or the
+// concatenated buffer src -> phi_s (scatter).
+int one_body64(afqmc_ctx* c, int nw, const double* const phi[2], double* const phi_out[2], const double* src,
+               double* dst) {
+  const int N = c->d.nbasis, nc = c->ncol, n[2] = {c->d.nalpha, c->d.nbeta};
+  if (!c->exp_ready) {
+    HIP_TRY(c, launch_pad_rows(c->s.expH1, 2 * N, N, exp_ld(c), c->exp_pad, c->stream));
+    c->exp_ready = true;
+  }
+  OneBody64Args a{};
   a.nwalkers = nw;
-  a.nrows = c->d.nbasis;
-  a.ncol = ncol;
-  a.A = A;
-  a.a_complex = acplx;
-  a.a_stride = a_stride;
-  a.B = B;
-  a.b_stride = b_stride;
-  a.ldb = ldb;
-  a.C = C;
-  a.c_stride = c_stride;
-  a.ldc = ldc;
-  a.alpha = alpha;
-  a.accum = accum;
-  a.accum_init = accum_init;
-  HIP_TRY(c, launch_batched_nn(a, c->stream));
+  a.nbasis = N;
+  a.nspin = two_spins(c) ? 2 : 1;
+  a.ld_exp = exp_ld(c);
+  for (int s = 0; s < a.nspin; ++s) {
+    OneBody64Spin& p = a.spin[s];
+    const int off = s == 0 ? 0 : n[0];
+    p.n = n[s];
+    p.exp = c->exp_pad + (int64_t)s * N * a.ld_exp;
+    p.src = src ? src : phi[s];
+    p.src_ws = (int64_t)N * (src ? nc : n[s]);
+    p.src_ld = src ? nc : n[s];
+    p.src_off = src ? off : 0;
+    p.out = dst ? dst : phi_out[s];
+    p.out_ws = (int64_t)N * (dst ? nc : n[s]);
+    p.out_ld = dst ? nc : n[s];
+    p.out_off = dst ? off : 0;
+  }
+  HIP_TRY(c, launch_one_body64(a, c->stream));
   return AFQMC_OK;
 }
 
@@ -714,7 +721,6 @@ int one_body_bf16(afqmc_ctx* c, int nw, int s, const uint16_t* aplanes, int64_t 
 int gather(afqmc_ctx* c, int nw, const double* phia, const double* phib, bool with_expH1) {
   PhaseScope ps(c, AFQMC_PHASE_ONE_BODY);
   const int N = c->d.nbasis, na = c->d.nalpha, nb = c->d.nbeta, nc = c->ncol;
-  const int64_t NN = (int64_t)N * N;
   double* P = c->buf[0];
   c->ptp_ready = false;
   if (with_expH1 && c->dplanes) {
@@ -732,13 +738,8 @@ int gather(afqmc_ctx* c, int nw, const double* phia, const double* phib, bool wi
     return AFQMC_OK;
   }
   if (with_expH1) {
-    int r = nn(c, nw, c->s.expH1, false, 0, phia, (int64_t)N * na, na, P, (int64_t)N * nc, nc, na, 1.0, nullptr,
-               nullptr);
-    if (r) return r;
-    if (two_spins(c))
-      return nn(c, nw, c->s.expH1 + NN, false, 0, phib, (int64_t)N * nb, nb, P + 2 * na, (int64_t)N * nc, nc, nb,
-                1.0, nullptr, nullptr);
-    return AFQMC_OK;
+    const double* const phi[2] = {phia, phib};
+    return one_body64(c, nw, phi, nullptr, nullptr, P);
   }
   HIP_TRY(c, hipMemcpy2DAsync(P, 16 * nc, phia, 16 * na, 16 * na, (size_t)nw * N, hipMemcpyDeviceToDevice,
                               c->stream));
@@ -754,7 +755,6 @@ int scatter(afqmc_ctx* c, int nw, const double* src, double* phia, double* phib,
             const uint16_t* srcT = nullptr) {
   PhaseScope ps(c, AFQMC_PHASE_ONE_BODY);
   const int N = c->d.nbasis, na = c->d.nalpha, nb = c->d.nbeta, nc = c->ncol;
-  const int64_t NN = (int64_t)N * N;
   if (with_expH1 && c->dplanes) {
     int r = ensure_planes(c);
     if (r) return r;
@@ -772,13 +772,8 @@ int scatter(afqmc_ctx* c, int nw, const double* src, double* phia, double* phib,
     return AFQMC_OK;
   }
   if (with_expH1) {
-    int r = nn(c, nw, c->s.expH1, false, 0, src, (int64_t)N * nc, nc, phia, (int64_t)N * na, na, na, 1.0, nullptr,
-               nullptr);
-    if (r) return r;
-    if (two_spins(c))
-      return nn(c, nw, c->s.expH1 + NN, false, 0, src + 2 * na, (int64_t)N * nc, nc, phib, (int64_t)N * nb, nb, nb,
-                1.0, nullptr, nullptr);
-    return AFQMC_OK;
+    double* const phi[2] = {phia, phib};
+    return one_body64(c, nw, nullptr, phi, src, nullptr);
   }
   HIP_TRY(c, hipMemcpy2DAsync(phia, 16 * na, src, 16 * nc, 16 * na, (size_t)nw * N, hipMemcpyDeviceToDevice,
                               c->stream));
@@ -839,22 +834,29 @@ int taylor(afqmc_ctx* c, int nw, const double** result, const uint16_t** resultT
   PhaseScope ps(c, AFQMC_PHASE_TAYLOR);
   if (resultT) *resultT = nullptr;
   if (c->vatoms && c->d.exp_nmax > 0) return taylor_bf16(c, nw, result, resultT);
-  const int N = c->d.nbasis, nc = c->ncol;
-  const int64_t NN = (int64_t)N * N, stride = (int64_t)N * nc;
-  double* P = c->buf[0];
-  double* Q = c->buf[3];
-  if (c->d.exp_nmax <= 0) {
-    *result = P;
+  const double* P = c->buf[0];
+  const double* prev = P;
+  Taylor64Args t{};
+  t.nwalkers = nw;
+  t.nbasis = c->d.nbasis;
+  t.ncol = c->ncol;
+  t.vhs = c->vhs;
+  t.base = P;
+  if (taylor64_in_one(t.nbasis)) {
+    t.out = c->buf[1];
+    t.terms = c->d.exp_nmax;
+    HIP_TRY(c, launch_taylor64_series(t, c->stream));
+    *result = t.out;
     return AFQMC_OK;
   }
-  const double* prev = P;
-  for (int k = 1; k <= c->d.exp_nmax; ++k) {
-    double* out = (k & 1) ? c->buf[1] : c->buf[2];
-    int r = nn(c, nw, c->vhs, true, NN, prev, stride, nc, out, stride, nc, nc, 1.0 / k, Q, k == 1 ? P : nullptr);
-    if (r) return r;
-    prev = out;
+  for (int k = c->d.exp_nmax; k >= 1; --k) {  // Horner: T <- P + (VHS T) / k
+    t.prev = prev;
+    t.out = prev == c->buf[1] ? c->buf[2] : c->buf[1];
+    t.alpha = 1.0 / k;
+    HIP_TRY(c, launch_taylor64(t, c->stream));
+    prev = t.out;
   }
-  *result = Q;
+  *result = prev;
   return AFQMC_OK;
 }
 
@@ -1404,7 +1406,7 @@ void afqmc_destroy(afqmc_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   else (void)hipDeviceSynchronize();
   void* ptrs[] = {c->vbias_part, c->xshifted, c->wvec, c->exx_a, c->exx_b, c->vhs, c->buf[0], c->buf[1],
-                  c->buf[2], c->buf[3], c->tri, c->flags, c->wflags, c->psi_flag, c->nfb, c->gplanes[0], c->gplanes[1], c->lplanes[0],
+                  c->buf[2], c->buf[3], c->exp_pad, c->flags, c->wflags, c->psi_flag, c->nfb, c->gplanes[0], c->gplanes[1], c->lplanes[0],
                   c->lplanes[1], c->xplanes, c->cplanes, c->vatoms, c->zatom, c->dplanes, c->oplanes, c->gcomp, c->gf_o, c->gf_oinv, c->qw64[0], c->qw64[1], c->qwp[0],
                   c->qwp[1], c->qy, c->qunits[0], c->qunits[1], c->sur.feat, c->sur.pred, c->sur.est, c->sur.target,
                   c->sur.resid, c->sur.walker_of, c->sur.xbar, c->sur.e1, c->sur.master, c->sur.m,
@@ -1456,6 +1458,7 @@ int afqmc_set_static(afqmc_ctx* c, const afqmc_static* s) {
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   c->psi_real = any == 0;
   c->planes_ready = false;
+  c->exp_ready = false;
   c->quad_ready = false;
   c->q8_ready = false;
   c->sur.cv_ready = false;

@@ -88,12 +88,8 @@ struct NtArgs {
   int nseg, ksplit;  // segments; K ranges (over the chunks of all segments)
   NtSegment seg[2];
   double scale;
-  double* out;       // [ksplit, m, n] complex: scale C; with tri_i: [m, nbasis, nbasis] complex
-  // packed-index row and column of each column of C, or null: C's columns are the
-  // packed upper triangle of symmetric matrices, written to both triangles times i scale
-  const int* tri_i;
-  const int* tri_j;
-  int nbasis;
+  double* out;       // [ksplit, m, n] complex: scale C, or i scale C (times_i)
+  int times_i;
   // quadratic form (n = K): column units {tile, first chunk, end chunk, 0} from
   // nt64_quad_units, or null; out[unit][m] = sum over the unit's columns c of
   // dg[r, c] sum_{k in the unit's chunks} A[r, k] B[c, k] (dg [m, n] complex)
@@ -115,23 +111,43 @@ int nt64_quad_units(int64_t m, int64_t n, std::vector<int4>& units);
 constexpr int QUAD64_TILE = 128;  // column tile of the FP64 W'
 constexpr int FB_MAX_SPLIT = 16;  // most K ranges of the FP64 force bias (heuristic)
 
-// Batched C[w] = A[w] * B[w] with A [N, N] (real shared or complex per walker)
-// and B [N, ncol] complex (columns contiguous).  Epilogue:
-//   out = alpha * (A B);  if accum: accum_buf += out
-struct BatchedNNArgs {
-  int nwalkers, nrows, ncol;
-  const double* A;       // real [N, N] (shared) or complex [W, N, N]
-  bool a_complex;
-  int64_t a_stride;      // walker stride of A in elements of its type (0 = shared)
-  const double* B;       // complex, walker w at B + 2 * w * b_stride, row k at + 2 * k * ldb
-  int64_t b_stride, ldb;
-  double* C;             // complex output, same addressing as B (c_stride, ldc)
-  int64_t c_stride, ldc;
-  double alpha;
-  double* accum;         // optional complex accumulator, same addressing as C
-  const double* accum_init;  // optional: accum = accum_init + out (else accum += out)
+// One body of both spins: out[w][i][out_off + c] = sum_k exp[i][k] src[w][k][src_off + c],
+// c < n (complex; walker strides ws and row lengths ld in complex values; exp real,
+// rows of ld_exp, a multiple of 16, zero past nbasis).
+struct OneBody64Spin {
+  int n;
+  const double* exp;
+  const double* src;
+  int64_t src_ws;
+  int src_ld, src_off;
+  double* out;
+  int64_t out_ws;
+  int out_ld, out_off;
 };
-hipError_t launch_batched_nn(const BatchedNNArgs& a, hipStream_t stream);
+struct OneBody64Args {
+  int nwalkers, nbasis, nspin, ld_exp;
+  OneBody64Spin spin[2];
+};
+hipError_t launch_one_body64(const OneBody64Args& a, hipStream_t stream);
+// rows of n values -> rows of ld, zero past n
+hipError_t launch_pad_rows(const double* src, int rows, int n, int ld, double* dst, hipStream_t stream);
+
+// out[w] = base[w] + alpha V[w] prev[w] ([W, N, ncol] complex; V symmetric, as the
+// packed upper triangle [W, N (N + 1) / 2] complex)
+struct Taylor64Args {
+  int nwalkers, nbasis, ncol;
+  const double* vhs;
+  const double* prev;
+  const double* base;
+  double* out;
+  double alpha;
+  int terms;                // launch_taylor64_series: all terms at once (prev, alpha unused)
+  int colblocks, colwidth;  // set by the launcher
+};
+hipError_t launch_taylor64(Taylor64Args a, hipStream_t stream);
+// out = sum_{k <= terms} V^k base / k!
+bool taylor64_in_one(int nbasis);
+hipError_t launch_taylor64_series(Taylor64Args a, hipStream_t stream);
 
 // ---------------------------------------------------------------- exchange
 struct ExchangeArgs {

@@ -2,10 +2,9 @@
 // (K contiguous in both), on v_mfma_f64_16x16x4f64:
 //   * force bias   vbias[w, x] = sum_s sum_k Ghalf_s[w, k] rchol_s[x, k]
 //                  (ipie/propagation/force_bias.py:79-121)
-//   * VHS          VHS[w] = i sqrt(dt) sum_x xshifted[w, x] L_x from the packed upper
-//                  triangle, written to both triangles
-//                  (ipie/propagation/phaseless_generic.py:67-97,
-//                   ipie/utils/pack_numba.py:22-33)
+//   * VHS          VHS[w] = i sqrt(dt) sum_x xshifted[w, x] L_x, its packed upper
+//                  triangle (ipie/propagation/phaseless_generic.py:67-97; not unpacked:
+//                  the Taylor kernel reads the triangle)
 //   * the exchange as a quadratic form, sum_b g_b (G W')_b over the block-triangular
 //     W' (k_quad.hip), the dot products in the epilogue
 //
@@ -49,7 +48,7 @@ constexpr int NT_THREADS = 64 * NT_WAVES;
 
 __device__ double2 nt_zero;  // source of the slots past K
 
-enum { NT_EPI_PART = 0, NT_EPI_VHS = 1, NT_EPI_QDOT = 2 };
+enum { NT_EPI_PART = 0, NT_EPI_QDOT = 1 };
 
 // Direct global-to-LDS loads: lane l's 16 (4) bytes go to dst + 16 l (4 l).
 __device__ __forceinline__ void nt_load16(const char* src, void* dst) {
@@ -255,26 +254,14 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
   for (int j = 0; j < NT_RN; ++j) {
     const int64_t c = col0 + wave * 16 * NT_RN + 16 * j + l16;
     if (c >= a.n) continue;
-    int ti = 0, tj = 0;
-    if (EPI == NT_EPI_VHS) {
-      ti = a.tri_i[c];
-      tj = a.tri_j[c];
-    }
 #pragma unroll
     for (int i = 0; i < RM; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int64_t w = row0 + 16 * i + 4 * r + q;
         if (w >= a.m) continue;
-        if (EPI == NT_EPI_PART) {
-          st(a.out, ((int64_t)z * a.m + w) * a.n + c, cmake(a.scale * re[i][j][r], a.scale * im[i][j][r]));
-        } else {
-          // i scale (re + i im), to both triangles
-          const cplx v = cmake(-a.scale * im[i][j][r], a.scale * re[i][j][r]);
-          double* base = a.out + 2 * w * a.nbasis * a.nbasis;
-          st(base, (int64_t)ti * a.nbasis + tj, v);
-          if (ti != tj) st(base, (int64_t)tj * a.nbasis + ti, v);
-        }
+        const cplx v = cmake(a.scale * re[i][j][r], a.scale * im[i][j][r]);
+        st(a.out, ((int64_t)z * a.m + w) * a.n + c, a.times_i ? cmake(-v.im, v.re) : v);
       }
   }
 }
@@ -392,7 +379,7 @@ hipError_t launch_nt64(const NtArgs& a, hipStream_t stream) {
     if (a.nseg != 1 || a.ksplit != 1 || a.nunits < 1 || a.seg[0].K != a.n) return hipErrorInvalidValue;
     return launch_nt<NT_EPI_QDOT>(a, stream);
   }
-  return a.tri_i ? launch_nt<NT_EPI_VHS>(a, stream) : launch_nt<NT_EPI_PART>(a, stream);
+  return launch_nt<NT_EPI_PART>(a, stream);
 }
 
 }  // namespace afqmc
