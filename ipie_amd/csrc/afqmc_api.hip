@@ -41,6 +41,7 @@ struct afqmc_ctx {
   double* exx_b = nullptr;       // [xs_b, W] complex
   double* vhs = nullptr;         // FP64: packed upper triangles [W, N (N + 1) / 2] complex
   double* buf[4] = {nullptr, nullptr, nullptr, nullptr};  // P, Ta, Tb, Q (mixed): [W, N, ncol] complex
+  int* qr_slow = nullptr;        // [W] scratch of the re-orthogonalisation
   double* exp_pad = nullptr;     // FP64: expH1 [2, N, exp_ld], zero past N
   bool exp_ready = false;        // exp_pad holds the current expH1
   int* flags = nullptr;
@@ -384,6 +385,7 @@ int ensure_ws(afqmc_ctx* c) {
   if (ok) c->fb_cap = c->fb_ksplit;
   ok = ok && dmalloc((void**)&c->xshifted, 16 * (size_t)W * X) == hipSuccess;
   ok = ok && dmalloc((void**)&c->wvec, 16 * (size_t)6 * W) == hipSuccess;
+  ok = ok && dmalloc((void**)&c->qr_slow, sizeof(int) * (size_t)W) == hipSuccess;
   // partial sums: at most one per Cholesky vector per walker, whatever the split
   c->exx_cap = (int64_t)X * W;
   ok = ok && dmalloc((void**)&c->exx_a, 16 * (size_t)c->exx_cap) == hipSuccess;
@@ -1406,7 +1408,7 @@ void afqmc_destroy(afqmc_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   else (void)hipDeviceSynchronize();
   void* ptrs[] = {c->vbias_part, c->xshifted, c->wvec, c->exx_a, c->exx_b, c->vhs, c->buf[0], c->buf[1],
-                  c->buf[2], c->buf[3], c->exp_pad, c->flags, c->wflags, c->psi_flag, c->nfb, c->gplanes[0], c->gplanes[1], c->lplanes[0],
+                  c->buf[2], c->buf[3], c->exp_pad, c->qr_slow, c->flags, c->wflags, c->psi_flag, c->nfb, c->gplanes[0], c->gplanes[1], c->lplanes[0],
                   c->lplanes[1], c->xplanes, c->cplanes, c->vatoms, c->zatom, c->dplanes, c->oplanes, c->gcomp, c->gf_o, c->gf_oinv, c->qw64[0], c->qw64[1], c->qwp[0],
                   c->qwp[1], c->qy, c->qunits[0], c->qunits[1], c->sur.feat, c->sur.pred, c->sur.est, c->sur.target,
                   c->sur.resid, c->sur.walker_of, c->sur.xbar, c->sur.e1, c->sur.master, c->sur.m,
@@ -2004,6 +2006,7 @@ int afqmc_reortho(afqmc_ctx* c, int32_t nw, double* phia, double* phib, double* 
   a.detR_shift = detR_shift;
   a.flags = c->flags;
   a.wflags = c->wflags;
+  a.slow = c->qr_slow;
   PhaseScope ps(c, AFQMC_PHASE_REORTHO);
   HIP_TRY(c, launch_reortho(a, c->stream));
   return AFQMC_OK;

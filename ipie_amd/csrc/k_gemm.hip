@@ -474,6 +474,8 @@ template <int RM>
 hipError_t launch_ob_rm(const OneBody64Args& a, int64_t colblocks, hipStream_t stream) {
   const int64_t blocks = colblocks * ceil_div(a.nbasis, 16 * RM);
   if (blocks > INT32_MAX) return hipErrorInvalidValue;
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(one_body64_kernel<RM>), ObPlan<RM>::LDS_BYTES);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(one_body64_kernel<RM>, dim3((unsigned)blocks), dim3(PG_THREADS), ObPlan<RM>::LDS_BYTES, stream, a);
   return hipGetLastError();
 }
@@ -482,6 +484,8 @@ template <int RN>
 hipError_t launch_ty_rn(const Taylor64Args& a, hipStream_t stream) {
   const int64_t blocks = (int64_t)a.nwalkers * ceil_div(a.nbasis, 64) * a.colblocks;
   if (blocks > INT32_MAX) return hipErrorInvalidValue;
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(taylor64_kernel<RN>), TyPlan<RN>::LDS_BYTES);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(taylor64_kernel<RN>, dim3((unsigned)blocks), dim3(PG_THREADS), TyPlan<RN>::LDS_BYTES, stream, a);
   return hipGetLastError();
 }
@@ -491,6 +495,8 @@ hipError_t launch_ty_series(const Taylor64Args& a, hipStream_t stream) {
   const int64_t blocks = (int64_t)a.nwalkers * a.colblocks;
   if (blocks > INT32_MAX) return hipErrorInvalidValue;
   const unsigned tiles = (unsigned)ceil_div(a.nbasis, 16);
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(taylor64_series_kernel<NCH, RN>), tiles * 2048 * RN);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL((taylor64_series_kernel<NCH, RN>), dim3((unsigned)blocks), dim3(64 * tiles), tiles * 2048 * RN,
                      stream, a);
   return hipGetLastError();

@@ -294,6 +294,8 @@ hipError_t launch_nt_mode(const NtArgs& a, hipStream_t stream) {
   using P = NtPlan<RM, MODE>;
   const int64_t blocks = (EPI == NT_EPI_QDOT ? a.nunits : ceil_div(a.n, NT_TN)) * ceil_div(a.m, P::TM);
   if (blocks > INT32_MAX || a.ksplit > 65535) return hipErrorInvalidValue;
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(nt64_kernel<RM, MODE, EPI>), P::LDS_BYTES);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL((nt64_kernel<RM, MODE, EPI>), dim3((unsigned)blocks, a.ksplit), dim3(NT_THREADS), P::LDS_BYTES,
                      stream, a);
   return hipGetLastError();

@@ -7,6 +7,8 @@
 //   G = X^H X (+ shift),  G = R^H R,  X <- X R^{-1},
 // as sweeps over the rows of X on FP64 MFMA: the Gram matrix of pass p + 1 is
 // formed from the rows of X R_p^{-1} while they are written.
+// Walkers with at most 48 columns that take the first branch below, that is all but
+// ill-conditioned ones, run in reortho_fast_kernel, the others in reortho_kernel.
 //   - CholeskyQR2 (two passes, three sweeps; Yamamoto, Nakatsukasa, Yanagisawa,
 //     Fukaya, ETNA 44 (2015) 306) when the unshifted Cholesky of X^H X succeeds
 //     and 8 kappa sqrt(N n u + n (n + 1) u) <= 1/2 with kappa bounded by
@@ -28,6 +30,8 @@ namespace {
 
 constexpr int QR_THREADS = 256;
 constexpr int QR_WAVES = QR_THREADS / 64;
+
+__device__ double2 qr_zero;  // source of values past a matrix
 
 // Row stride of G and Ri for at most 16 NT columns.
 __host__ __device__ inline int qr_ld(int nt) { return 16 * nt + 1; }
@@ -250,10 +254,388 @@ __device__ void qr_upper_inverse(const cplx* R, int ldr, int n, int np, cplx* Ri
   __syncthreads();
 }
 
+// detR and what follows from it, from log det R of walker w.
+__device__ void qr_finish(const ReorthoArgs& a, int w, double logdet) {
+  const double shift = a.detR_shift ? a.detR_shift[w] : 0.0;
+  const double detR = exp(logdet - shift);
+  a.detR[w] = detR;
+  if (a.log_detR) a.log_detR[w] += log(detR);
+  if (a.ovlp) {
+    const cplx o = ld(a.ovlp, w);
+    st(a.ovlp, w, cmake(o.re / detR, o.im / detR));
+  }
+}
+
+// ---------------------------------------------------------------- well-conditioned walkers
+// CholeskyQR2 of both spins in one workgroup of four waves, the same sweeps as
+// above with 256 registers a wave, so that two workgroups share a CU: one is in
+// its sweeps (bound by the FP64 matrix pipe: 19200 MFMAs a walker at N = 400,
+// n = 40, 131 us on a CU) while the other factors.  The factorisation, a serial chain
+// that took most of the time column by column with a barrier each, is blocked by
+// 16: a diagonal block is factored and inverted in one wave's registers (lane =
+// column), the rest is 16 x 16 MFMA products, and the two spins' matrices run side
+// by side on two waves each.  S holds one matrix per spin: the Gram matrix,
+// then R, then R^-1, all in place, identity in the padding.
+//   N = 400, n = 40, 1024 walkers: 0.98 ms against 2.54 ms in reortho_kernel; 12 walkers 276 us
+//   against 577 us.
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Upper Cholesky D = R^H R of a 16 x 16 block and D <- R^-1 (zero below the
+// diagonal); lane % 16 owns a column.  Adds this lane's log R_jj to logd; false
+// (the same in every lane) if D is not numerically positive definite.
+__device__ __forceinline__ bool qr_block_factor(cplx* D, int ld, double& logd) {
+  const int l16 = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+  cplx c[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) c[i] = D[i * ld + l16];
+  double diag = 1.0, inv = 1.0;  // R_jj and 1 / R_jj of this lane's column
+  bool ok = true;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const double dkk = lane_value(c[k].re, k);
+    ok = ok && dkk > 0.0;
+    const double r = rsqrt(dkk);
+    double d = dkk * r;
+    d = fma(fma(-d, d, dkk), 0.5 * r, d);
+    const cplx scaled = cscale(c[k], r);
+    c[k].re = l16 == k ? d : scaled.re;
+    c[k].im = l16 == k ? 0.0 : scaled.im;
+    diag = l16 == k ? d : diag;
+    inv = l16 == k ? r : inv;
+#pragma unroll
+    for (int i = k + 1; i < 16; ++i) {  // c_ij -= conj(R_ki) R_kj
+      const double br = lane_value(c[k].re, i), bi = lane_value(c[k].im, i);
+      c[i].re = fma(-br, c[k].re, c[i].re);
+      c[i].re = fma(-bi, c[k].im, c[i].re);
+      c[i].im = fma(-br, c[k].im, c[i].im);
+      c[i].im = fma(bi, c[k].re, c[i].im);
+    }
+    // (the updates of a step before the next: the compiler would delay them and
+    // keep every broadcast value)
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  logd += log(diag);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    c[i].re = l16 < i ? 0.0 : c[i].re;
+    c[i].im = l16 < i ? 0.0 : c[i].im;
+  }
+  // X = R^-1 by rows from the last: X_ij = (delta_ij - sum_{k > i} R_ik X_kj) / R_ii
+#pragma unroll
+  for (int i = 15; i >= 0; --i) {
+    cplx s0 = cmake(l16 == i ? 1.0 : 0.0, 0.0), s1 = cmake(0.0, 0.0);
+#pragma unroll
+    for (int k = i + 1; k < 16; ++k) {
+      const double br = lane_value(c[i].re, k), bi = lane_value(c[i].im, k);
+      cplx& t = (k & 1) ? s1 : s0;
+      t.re = fma(-br, c[k].re, t.re);
+      t.re = fma(bi, c[k].im, t.re);
+      t.im = fma(-br, c[k].im, t.im);
+      t.im = fma(-bi, c[k].re, t.im);
+    }
+    c[i] = cscale(cadd(s0, s1), lane_value(inv, i));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    if ((i & 3) == q) D[i * ld + l16] = c[i];
+  return ok;
+}
+
+// acc += A B for 16 x 16 blocks in LDS; A read as stored, or conjugate transposed
+// (HA); the result's register r of lane (q, l16) is element (4 r + q, l16), which is also
+// the B operand of K step r.
+struct QrAcc {
+  v4d re, im;
+};
+template <bool HA>
+__device__ __forceinline__ void qr_mma(const cplx* A, int ld, const cplx (&b)[4], QrAcc& acc) {
+  const int l16 = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int k = 4 * r + q;
+    cplx x = HA ? A[k * ld + l16] : A[l16 * ld + k];
+    if (HA) x.im = -x.im;
+    acc.re = mfma64(x.re, b[r].re, acc.re);
+    acc.re = mfma64(-x.im, b[r].im, acc.re);
+    acc.im = mfma64(x.re, b[r].im, acc.im);
+    acc.im = mfma64(x.im, b[r].re, acc.im);
+  }
+}
+__device__ __forceinline__ void qr_block_load(const cplx* B, int ld, cplx (&b)[4]) {
+  const int l16 = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) b[r] = B[(4 * r + q) * ld + l16];
+}
+__device__ __forceinline__ void qr_block_store(cplx* B, int ld, const QrAcc& v, double scale) {
+  const int l16 = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) B[(4 * r + q) * ld + l16] = cmake(scale * v.re[r], scale * v.im[r]);
+}
+
+// S_s <- R_s^-1 for every spin s < nspin (wave pair s), G = R^H R; log det R_s and
+// whether the factorisation went through into logdet and ok.
+template <int NT>
+__device__ __forceinline__ void qr_factor(cplx* S, int nspin, double* logdet, int* ok) {
+  constexpr int LD = 16 * NT + 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), spin = wave >> 1, part = wave & 1;
+  const int l16 = threadIdx.x & 15, q = (threadIdx.x & 63) >> 4;
+  const bool mine = spin < nspin;
+  cplx* G = S + spin * 16 * NT * LD;
+  auto block = [&](int I, int J) { return G + 16 * I * LD + 16 * J; };
+  double logd = 0.0;
+  bool good = true;
+#pragma unroll 1
+  for (int b = 0; b < NT; ++b) {
+    if (mine && part == 0) {
+      const bool g = qr_block_factor(block(b, b), LD, logd);
+      good = good && g;
+    }
+    __syncthreads();
+    // the block row: R_bJ = (R_bb^-1)^H G_bJ
+    for (int J = b + 1 + part; mine && J < NT; J += 2) {
+      cplx x[4];
+      qr_block_load(block(b, J), LD, x);
+      QrAcc v{zero4d(), zero4d()};
+      qr_mma<true>(block(b, b), LD, x, v);
+      qr_block_store(block(b, J), LD, v, 1.0);
+    }
+    __syncthreads();
+    // G_IJ -= R_bI^H R_bJ
+    int t = 0;
+    for (int I = b + 1; mine && I < NT; ++I)
+      for (int J = I; J < NT; ++J, ++t) {
+        if ((t & 1) != part) continue;
+        cplx x[4];
+        qr_block_load(block(b, J), LD, x);
+        QrAcc v{zero4d(), zero4d()};
+        qr_mma<true>(block(b, I), LD, x, v);
+        cplx g[4];
+        qr_block_load(block(I, J), LD, g);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v.re[r] = g[r].re - v.re[r];
+          v.im[r] = g[r].im - v.im[r];
+        }
+        qr_block_store(block(I, J), LD, v, 1.0);
+      }
+    __syncthreads();
+  }
+  // the inverse's block columns from the left, in place: T_K = R_KJ X_JJ, X_IJ = - sum_K X_IK T_K
+#pragma unroll 1
+  for (int J = 1; J < NT; ++J) {
+    for (int K = part; mine && K < J; K += 2) {
+      cplx x[4];
+      qr_block_load(block(J, J), LD, x);
+      QrAcc v{zero4d(), zero4d()};
+      qr_mma<false>(block(K, J), LD, x, v);
+      qr_block_store(block(K, J), LD, v, 1.0);
+    }
+    __syncthreads();
+    QrAcc v[2] = {{zero4d(), zero4d()}, {zero4d(), zero4d()}};  // I = part, part + 2
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      for (int K = part + 2 * u; mine && K < J; ++K) {
+        cplx x[4];
+        qr_block_load(block(K, J), LD, x);
+        qr_mma<false>(block(part + 2 * u, K), LD, x, v[u]);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (mine && part + 2 * u < J) qr_block_store(block(part + 2 * u, J), LD, v[u], -1.0);
+    __syncthreads();
+  }
+  if (mine && part == 0) {
+    if (q != 0) logd = 0.0;
+    for (int off = 8; off > 0; off >>= 1) logd += __shfl_xor(logd, off, 64);
+    if (l16 == 0 && q == 0) {
+      logdet[spin] = logd;
+      ok[spin] = good;
+    }
+  }
+  __syncthreads();
+}
+
+// The sweep of one matrix (as qr_sweep): APPLY replaces the rows by X S, GRAM leaves
+// the Gram matrix of the (new) rows in S with identity padding and returns its
+// trace.  A tile's 4 NT loads are in flight under the MFMAs before it; values past
+// the matrix come from a zero line, so that nothing branches around a load.
+template <int NT, bool APPLY, bool GRAM>
+__device__ __forceinline__ double qr_fast_sweep(double* __restrict__ X, int N, int n, cplx* S, double* sums) {
+  constexpr int LD = 16 * NT + 1, NPAIR = NT * (NT + 1) / 2;
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  typedef const __attribute__((address_space(1))) v2d* gptr;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+  const int ntile = (N + 15) / 16;
+  const gptr zero = (gptr)(const void*)&qr_zero, base = (gptr)(const void*)X;
+  v4d gr[GRAM ? NPAIR : 1], gi[GRAM ? NPAIR : 1], yr[NT], yi[NT];
+  if (GRAM) {
+#pragma unroll
+    for (int p = 0; p < NPAIR; ++p) gr[p] = gi[p] = zero4d();
+  }
+  v2d x[4 * NT];
+  // tile t: as the A operand of the product (row l16, column 4 u + q), or without it in
+  // the accumulators' layout (row 4 r + q, column 16 J + l16; u = 4 J + r)
+  auto fetch = [&](int t) {
+#pragma unroll
+    for (int u = 0; u < 4 * NT; ++u) {
+      const int row = 16 * t + (APPLY ? l16 : 4 * (u & 3) + q), col = APPLY ? 4 * u + q : 16 * (u >> 2) + l16;
+      const gptr p = base + (int64_t)row * n + col;
+      x[u] = *(row < N && col < n ? p : zero);
+    }
+  };
+  if (wave < ntile) fetch(wave);
+#pragma unroll 1
+  for (int t = wave; t < ntile; t += QR_WAVES) {
+    if constexpr (APPLY) {
+#pragma unroll
+      for (int J = 0; J < NT; ++J) yr[J] = yi[J] = zero4d();
+      int off = l16;  // (opaque: S would be held in registers over the tiles)
+      asm volatile("" : "+v"(off));
+#pragma unroll
+      for (int u = 0; u < 4 * NT; ++u) {
+        if (u % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int J = u / 4; J < NT; ++J) {  // R^-1 is upper triangular
+          const cplx r = S[(4 * u + q) * LD + 16 * J + off];
+          yr[J] = mfma64(x[u][0], r.re, yr[J]);
+          yr[J] = mfma64(-x[u][1], r.im, yr[J]);
+          yi[J] = mfma64(x[u][0], r.im, yi[J]);
+          yi[J] = mfma64(x[u][1], r.re, yi[J]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int J = 0; J < NT; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * t + 4 * r + q, col = 16 * J + l16;
+          if (row < N && col < n) st(X, (int64_t)row * n + col, cmake(yr[J][r], yi[J][r]));
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4 * NT; ++u) {
+        yr[u >> 2][u & 3] = x[u][0];
+        yi[u >> 2][u & 3] = x[u][1];
+      }
+    }
+    if (t + QR_WAVES < ntile) fetch(t + QR_WAVES);
+    if constexpr (GRAM) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        int p = 0;
+#pragma unroll
+        for (int I = 0; I < NT; ++I)
+#pragma unroll
+          for (int J = I; J < NT; ++J, ++p) {
+            gr[p] = mfma64(yr[I][r], yr[J][r], gr[p]);
+            gr[p] = mfma64(yi[I][r], yi[J][r], gr[p]);
+            gi[p] = mfma64(yr[I][r], yi[J][r], gi[p]);
+            gi[p] = mfma64(-yi[I][r], yr[J][r], gi[p]);
+          }
+      }
+    }
+  }
+  __syncthreads();  // S has been read
+  if constexpr (!GRAM) return 0.0;
+  // the waves' sums in wave order; identity in the padding
+#pragma unroll 1
+  for (int w = 0; w < QR_WAVES; ++w) {
+    if (wave == w) {
+      int p = 0;
+#pragma unroll
+      for (int I = 0; I < NT; ++I)
+#pragma unroll
+        for (int J = I; J < NT; ++J, ++p)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int i = 16 * I + 4 * r + q, j = 16 * J + l16;
+            cplx v = cmake(gr[p][r], gi[p][r]);
+            if (w > 0) v = cadd(v, S[i * LD + j]);
+            if (w == QR_WAVES - 1 && i == j && i >= n) v = cmake(1.0, 0.0);
+            S[i * LD + j] = v;
+          }
+    }
+    __syncthreads();
+  }
+  return block_sum((int)threadIdx.x < n ? S[threadIdx.x * (LD + 1)].re : 0.0, sums);
+}
+
+template <int NT>
+__global__ void __launch_bounds__(QR_THREADS, 2) reortho_fast_kernel(ReorthoArgs a) {
+  constexpr int LD = 16 * NT + 1;
+  extern __shared__ cplx smem[];
+  __shared__ double logdet[2], sums[QR_WAVES];
+  __shared__ int ok[2];
+  cplx* S = smem;  // per spin [16 NT][LD]
+  const int w = blockIdx.x, N = a.nbasis, nspin = a.nbeta > 0 ? 2 : 1;
+  constexpr double u = 1.1102230246251565e-16;  // 2^-53
+  double tr0 = 0.0, tr1 = 0.0;
+#pragma unroll 1
+  for (int s = 0; s < nspin; ++s) {
+    const int n = s == 0 ? a.nalpha : a.nbeta;
+    double* X = (s == 0 ? a.phia : a.phib) + 2 * (int64_t)w * N * n;
+    (s == 0 ? tr0 : tr1) = qr_fast_sweep<NT, false, true>(X, N, n, S + s * 16 * NT * LD, sums);
+  }
+  double ld = 0.0;
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {  // (one call site: the factorisation is inlined once)
+    qr_factor<NT>(S, nspin, logdet, ok);
+    ld += logdet[0] + (nspin > 1 ? logdet[1] : 0.0);
+    if (pass == 1) break;
+    bool slow = false;
+    for (int s = 0; s < nspin; ++s) {
+      const int n = s == 0 ? a.nalpha : a.nbeta;
+      const double mn = (double)N * n + (double)n * (n + 1);
+      // ||R^-1||_F^2 (||R||_F^2 is the Gram matrix's trace)
+      double x2 = 0.0;
+      for (int e = threadIdx.x; e < n * n; e += QR_THREADS) {
+        const int i = e / n, j = e % n;
+        if (j >= i) {
+          const cplx x = S[s * 16 * NT * LD + i * LD + j];
+          x2 += x.re * x.re + x.im * x.im;
+        }
+      }
+      x2 = block_sum(x2, sums);
+      slow = slow || !ok[s] || !(8.0 * sqrt((s == 0 ? tr0 : tr1) * x2) * sqrt(mn * u) <= 0.5);
+    }
+    if (threadIdx.x == 0) a.slow[w] = slow ? 1 : 0;
+    if (slow) return;  // nothing written yet: reortho_kernel takes this walker
+    __syncthreads();
+#pragma unroll 1
+    for (int s = 0; s < nspin; ++s) {
+      const int n = s == 0 ? a.nalpha : a.nbeta;
+      double* X = (s == 0 ? a.phia : a.phib) + 2 * (int64_t)w * N * n;
+      qr_fast_sweep<NT, true, true>(X, N, n, S + s * 16 * NT * LD, sums);
+    }
+  }
+  if (!ok[0] || (nspin > 1 && !ok[1])) {
+    if (threadIdx.x == 0) {
+      if (a.flags) atomicOr(a.flags, AFQMC_FLAG_CHOLESKY);
+      if (a.wflags) atomicOr(a.wflags + w, AFQMC_FLAG_CHOLESKY);
+      a.detR[w] = NAN;
+    }
+    return;
+  }
+#pragma unroll 1
+  for (int s = 0; s < nspin; ++s) {
+    const int n = s == 0 ? a.nalpha : a.nbeta;
+    double* X = (s == 0 ? a.phia : a.phib) + 2 * (int64_t)w * N * n;
+    qr_fast_sweep<NT, true, false>(X, N, n, S + s * 16 * NT * LD, sums);
+  }
+  if (threadIdx.x == 0) qr_finish(a, w, ld);
+}
+
 template <int NT>
 __global__ void __launch_bounds__(QR_THREADS) reortho_kernel(ReorthoArgs a) {
   extern __shared__ cplx smem[];
   const int w = blockIdx.x;
+  if (a.slow && !a.slow[w]) return;  // done by reortho_fast_kernel
   const int N = a.nbasis;
   const int ldg = qr_ld(NT);
   cplx* G = smem;                  // [16 NT][ldg]: Gram matrix, then R
@@ -308,35 +690,44 @@ __global__ void __launch_bounds__(QR_THREADS) reortho_kernel(ReorthoArgs a) {
       a.detR[w] = NAN;
       return;
     }
-    const double shift = a.detR_shift ? a.detR_shift[w] : 0.0;
-    const double detR = exp(logdet - shift);
-    a.detR[w] = detR;
-    if (a.log_detR) a.log_detR[w] += log(detR);
-    if (a.ovlp) {
-      const cplx o = ld(a.ovlp, w);
-      st(a.ovlp, w, cmake(o.re / detR, o.im / detR));
-    }
+    qr_finish(a, w, logdet);
   }
+}
+
+}  // namespace
+
+namespace {
+
+template <int NT>
+hipError_t launch_qr_nt(const ReorthoArgs& a, hipStream_t stream) {
+  const size_t matrix = sizeof(cplx) * 16 * (size_t)NT * qr_ld(NT);
+  hipError_t e = allow_lds((const void*)reortho_kernel<NT>, 2 * matrix);
+  if (e != hipSuccess) return e;
+  ReorthoArgs b = a;
+  if constexpr (NT <= 3) {  // (64 columns do not fit the fast kernel's registers)
+    const size_t lds = matrix * (a.nbeta > 0 ? 2 : 1);
+    e = allow_lds((const void*)reortho_fast_kernel<NT>, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(reortho_fast_kernel<NT>, dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a);
+  } else {
+    b.slow = nullptr;
+  }
+  hipLaunchKernelGGL(reortho_kernel<NT>, dim3(a.nwalkers), dim3(QR_THREADS), 2 * matrix, stream, b);
+  return hipGetLastError();
 }
 
 }  // namespace
 
 hipError_t launch_reortho(const ReorthoArgs& a, hipStream_t stream) {
   const int nmax = a.nalpha > a.nbeta ? a.nalpha : a.nbeta;
-  const int nt = (nmax + 15) / 16;
-  if (nt < 1 || nt > 4) return hipErrorInvalidValue;
-  const size_t lds = sizeof(cplx) * 2 * 16 * (size_t)nt * qr_ld(nt);
-  const void* k = nt == 1 ? (const void*)reortho_kernel<1> : nt == 2 ? (const void*)reortho_kernel<2>
-                : nt == 3 ? (const void*)reortho_kernel<3> : (const void*)reortho_kernel<4>;
-  hipError_t e = allow_lds(k, lds);
-  if (e != hipSuccess) return e;
-  switch (nt) {
-    case 1: hipLaunchKernelGGL(reortho_kernel<1>, dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a); break;
-    case 2: hipLaunchKernelGGL(reortho_kernel<2>, dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a); break;
-    case 3: hipLaunchKernelGGL(reortho_kernel<3>, dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a); break;
-    default: hipLaunchKernelGGL(reortho_kernel<4>, dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a); break;
+  if (!a.slow) return hipErrorInvalidValue;
+  switch ((nmax + 15) / 16) {
+    case 1: return launch_qr_nt<1>(a, stream);
+    case 2: return launch_qr_nt<2>(a, stream);
+    case 3: return launch_qr_nt<3>(a, stream);
+    case 4: return launch_qr_nt<4>(a, stream);
+    default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 }  // namespace afqmc
