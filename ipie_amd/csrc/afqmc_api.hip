@@ -844,7 +844,7 @@ int taylor(afqmc_ctx* c, int nw, const double** result, const uint16_t** resultT
   t.ncol = c->ncol;
   t.vhs = c->vhs;
   t.base = P;
-  if (taylor64_in_one(t.nbasis)) {
+  if (c->d.exp_nmax > 0 && taylor64_in_one(t.nbasis)) {  // (no terms: P itself)
     t.out = c->buf[1];
     t.terms = c->d.exp_nmax;
     HIP_TRY(c, launch_taylor64_series(t, c->stream));

@@ -15,6 +15,7 @@ U = 2.0**-53
 CASES = [
     (1, 1, 0, 1, 6),
     (15, 3, 1, 3, 1),       # below one tile, a single term
+    (40, 4, 3, 2, 0),       # no terms: the walkers unchanged
     (17, 5, 4, 2, 2),       # one past a tile
     (24, 12, 12, 10, 6),    # columns of three 8-column blocks exactly
     (113, 13, 12, 5, 6),    # eight row tiles, the last with one row
