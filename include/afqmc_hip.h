@@ -53,7 +53,7 @@ extern "C" {
 #define AFQMC_FLAG_NONFINITE 2   /* a non-finite weight was produced */
 #define AFQMC_FLAG_CHOLESKY 4    /* reortho met a numerically rank-deficient walker */
 
-/* phases timed by afqmc_profile (HIP events on the context's stream) */
+/* phases timed by afqmc_profile (device clock, stamped on the context's stream) */
 #define AFQMC_PHASE_GF 0          /* Green's function (PropagatorTimer.tgf) */
 #define AFQMC_PHASE_ONE_BODY 1    /* exp(-dt/2 H1) products and walker copies (tgemm) */
 #define AFQMC_PHASE_FORCE_BIAS 2  /* force-bias contraction (tfbias) */
@@ -285,8 +285,9 @@ int afqmc_local_energy(afqmc_ctx* ctx, int32_t nwalkers, const double* ghalfa, c
  * real; log_detR [W] real is incremented; detR_shift [W] real or NULL. */
 int afqmc_reortho(afqmc_ctx* ctx, int32_t nwalkers, double* phia, double* phib, double* ovlp, double* detR,
                   double* log_detR, const double* detR_shift);
-/* Per-phase timing: afqmc_profile(ctx, 1) clears the totals and starts
- * recording HIP events around every phase; afqmc_profile_read synchronises
+/* Per-phase timing: afqmc_profile(ctx, 1) clears the totals and stamps
+ * the device clock where every phase starts and ends (in the phases' own kernels
+ * where they can); afqmc_profile_read synchronises
  * and returns accumulated milliseconds and launch counts per phase
  * (arrays of AFQMC_NPHASES). */
 int afqmc_profile(afqmc_ctx* ctx, int enable);

@@ -18,11 +18,6 @@
 
 using namespace afqmc;
 
-struct PendingEvent {
-  int phase;
-  hipEvent_t start, stop;
-};
-
 struct afqmc_ctx {
   afqmc_dims d;
   int device = 0;
@@ -151,11 +146,13 @@ struct afqmc_ctx {
   int capture_steps = 0, capture_sur = 0;  // field draws / control-variate energies recorded
   hipGraphExec_t graph = nullptr;
   int graph_steps = 0, graph_sur = 0;
-  // per-phase HIP-event timing (afqmc_profile / afqmc_profile_read)
+  // per-phase device times (afqmc_profile / afqmc_profile_read)
   bool prof = false;
-  std::vector<hipEvent_t> ev_free;
-  std::vector<PendingEvent> ev_pending;
-  double prof_ms[AFQMC_NPHASES] = {0};
+  bool prof_clear = true;                 // the ticks are cleared before the next phase
+  bool prof_chain = false;                // phases follow each other: the next one closes the open one
+  int prof_open = -1;                     // phase open on the device, or -1
+  unsigned long long* prof_acc = nullptr; // [AFQMC_NPHASES] ticks
+  double prof_tick_ms = 1e-5;             // ms per tick
   int64_t prof_count[AFQMC_NPHASES] = {0};
 };
 
@@ -177,54 +174,55 @@ int fail(afqmc_ctx* c, int code, const char* fmt, ...) {
     if (_e != hipSuccess) return fail((c), AFQMC_ERR_HIP, "%s: %s", #expr, hipGetErrorString(_e)); \
   } while (0)
 
-hipEvent_t take_event(afqmc_ctx* c) {
-  if (!c->ev_free.empty()) {
-    hipEvent_t e = c->ev_free.back();
-    c->ev_free.pop_back();
-    return e;
-  }
-  hipEvent_t e = nullptr;
-  if (hipEventCreate(&e) != hipSuccess) return nullptr;
-  return e;
+// Closes the phase that is open on the device, if any.
+void close_phase(afqmc_ctx* c) {
+  if (c->prof_open < 0) return;
+  (void)launch_phase_mark(PhaseMark{c->prof_acc, c->prof_open, -1}, c->stream);
+  c->prof_open = -1;
 }
 
-// Adds the phases whose stop event has completed, oldest first, to the totals
-// and returns their events to the pool (no wait): keeps the pending list short
-// when profiling stays on and the totals are read rarely.
-void drain_completed(afqmc_ctx* c) {
-  size_t k = 0;
-  for (; k < c->ev_pending.size(); ++k) {
-    const PendingEvent& pe = c->ev_pending[k];
-    if (hipEventQuery(pe.stop) != hipSuccess) break;
-    float t = 0.0f;
-    if (hipEventElapsedTime(&t, pe.start, pe.stop) == hipSuccess) {
-      c->prof_ms[pe.phase] += t;
-      c->prof_count[pe.phase] += 1;
-    }
-    c->ev_free.push_back(pe.start);
-    c->ev_free.push_back(pe.stop);
-  }
-  c->ev_pending.erase(c->ev_pending.begin(), c->ev_pending.begin() + (std::ptrdiff_t)k);
-}
-
-// Records a start/stop event pair around one phase when profiling is on.
+// One phase of the per-phase times (PhaseMark), when they are on and no capture is
+// open.  The first kernel of the phase takes mark() and stamps the boundary; a scope
+// that is told so (STAMP) or whose mark nothing took stamps it with a kernel of its
+// own.  The end is stamped by the next phase inside a PhaseChain, else when the
+// scope ends.
 struct PhaseScope {
+  enum How { KERNEL, STAMP };
   afqmc_ctx* c;
-  int phase;
-  hipEvent_t start = nullptr;
-  PhaseScope(afqmc_ctx* ctx, int ph) : c(ctx), phase(ph) {
-    if (c->prof && !c->capturing) {
-      if (c->ev_pending.size() >= 1024) drain_completed(c);
-      start = take_event(c);
-      if (start) (void)hipEventRecord(start, c->stream);
+  int phase;  // -1 once marked
+  PhaseScope(afqmc_ctx* ctx, int ph, How how) : c(ctx), phase(ctx->prof && !ctx->capturing ? ph : -1) {
+    if (how == STAMP) stamp();
+  }
+  PhaseMark mark() {
+    if (phase < 0) return PhaseMark{};
+    if (c->prof_clear) {
+      (void)launch_phase_clear(c->prof_acc, AFQMC_NPHASES, c->stream);
+      c->prof_clear = false;
     }
+    const PhaseMark m{c->prof_acc, c->prof_open, phase};
+    c->prof_open = phase;
+    c->prof_count[phase] += 1;
+    phase = -1;
+    return m;
+  }
+  void stamp() {
+    if (phase >= 0) (void)launch_phase_mark(mark(), c->stream);
   }
   ~PhaseScope() {
-    if (!start) return;
-    hipEvent_t stop = take_event(c);
-    if (!stop) return;
-    (void)hipEventRecord(stop, c->stream);
-    c->ev_pending.push_back(PendingEvent{phase, start, stop});
+    stamp();
+    if (!c->prof_chain) close_phase(c);
+  }
+};
+
+// A sequence of phases with nothing between them: each phase's start is the end of
+// the one before.  Not for the control variate's energies, whose kernels between the
+// phases belong to none.
+struct PhaseChain {
+  afqmc_ctx* c;
+  explicit PhaseChain(afqmc_ctx* ctx) : c(ctx) { c->prof_chain = !c->sur.enabled; }
+  ~PhaseChain() {
+    c->prof_chain = false;
+    close_phase(c);
   }
 };
 
@@ -449,6 +447,7 @@ int need_static(afqmc_ctx* c) {
 // made on first use after afqmc_set_static.
 int ensure_planes(afqmc_ctx* c) {
   if (c->planes_ready) return AFQMC_OK;
+  close_phase(c);  // once per static set, in no phase
   const int N = c->d.nbasis;
   for (int s = 0; s < 2; ++s)
     if (c->lplanes[s]) {
@@ -502,7 +501,8 @@ int do_gf(afqmc_ctx* c, int nw, const double* phia, const double* phib, double* 
     if (dmalloc((void**)&c->gf_o, bytes) != hipSuccess || dmalloc((void**)&c->gf_oinv, bytes) != hipSuccess)
       return fail(c, AFQMC_ERR_ALLOC, "Green's function workspace allocation failed");
   }
-  PhaseScope ps(c, want_ghalf ? AFQMC_PHASE_GF : AFQMC_PHASE_OVERLAP);
+  PhaseScope ps(c, want_ghalf ? AFQMC_PHASE_GF : AFQMC_PHASE_OVERLAP, PhaseScope::KERNEL);
+  a.mark = ps.mark();
   HIP_TRY(c, launch_gf(a, want_ghalf, c->gf_o, c->gf_oinv, c->stream));
   return AFQMC_OK;
 }
@@ -514,7 +514,7 @@ int do_force_bias_bf16(afqmc_ctx* c, int nw, const double* ga, const double* gb)
   const int N = c->d.nbasis;
   int r = ensure_planes(c);
   if (r) return r;
-  PhaseScope ps(c, AFQMC_PHASE_FORCE_BIAS);
+  PhaseScope ps(c, AFQMC_PHASE_FORCE_BIAS, PhaseScope::STAMP);
   const int nspin = two_spins(c) ? 2 : 1;
   for (int s = 0; s < nspin; ++s) {
     const int n = s == 0 ? c->d.nalpha : c->d.nbeta;
@@ -560,7 +560,8 @@ int do_force_bias(afqmc_ctx* c, int nw, const double* ga, const double* gb) {
     a.scale = 2.0;
   }
   a.out = c->vbias_part;
-  PhaseScope ps(c, AFQMC_PHASE_FORCE_BIAS);
+  PhaseScope ps(c, AFQMC_PHASE_FORCE_BIAS, PhaseScope::KERNEL);
+  a.mark = ps.mark();
   HIP_TRY(c, launch_nt64(a, c->stream));
   return AFQMC_OK;
 }
@@ -590,7 +591,8 @@ int do_fields(afqmc_ctx* c, int nw, bool want_fields, const double* xi, uint64_t
   a.want_fields = want_fields ? 1 : 0;
   a.xbar_mean = c->sur.enabled ? c->sur.xbar : nullptr;
   a.xbar_max = c->sur.enabled ? c->sur.xbar + c->d.nwalkers : nullptr;
-  PhaseScope ps(c, AFQMC_PHASE_FIELDS);
+  PhaseScope ps(c, AFQMC_PHASE_FIELDS, PhaseScope::KERNEL);
+  a.mark = ps.mark();
   HIP_TRY(c, launch_fields(a, c->stream));
   return AFQMC_OK;
 }
@@ -599,7 +601,7 @@ int do_vhs(afqmc_ctx* c, int nw) {
   if (c->cplanes) {  // split-BF16: VHS[w] = i sqrt(dt) sum_x xshifted[w, x] L_x, as atoms
     int r = ensure_planes(c);
     if (r) return r;
-    PhaseScope ps(c, AFQMC_PHASE_VHS);
+    PhaseScope ps(c, AFQMC_PHASE_VHS, PhaseScope::STAMP);
     const int64_t ncols = vhs_atom_count(c->d.nbasis) * 256;
     HIP_TRY(c, launch_split_ghalf(c->xshifted, nw, c->d.nchol, c->xpad, c->xplanes, c->stream));
     Bf16GemmArgs b{};
@@ -632,7 +634,8 @@ int do_vhs(afqmc_ctx* c, int nw) {
   a.scale = sqrt(c->s.dt);
   a.out = c->vhs;
   a.times_i = 1;
-  PhaseScope ps(c, AFQMC_PHASE_VHS);
+  PhaseScope ps(c, AFQMC_PHASE_VHS, PhaseScope::KERNEL);
+  a.mark = ps.mark();
   HIP_TRY(c, launch_nt64(a, c->stream));
   return AFQMC_OK;
 }
@@ -640,13 +643,14 @@ int do_vhs(afqmc_ctx* c, int nw) {
 // FP64 one body of both spins: phi_s -> the concatenated buffer dst (gather) or the
 // concatenated buffer src -> phi_s (scatter).
 int one_body64(afqmc_ctx* c, int nw, const double* const phi[2], double* const phi_out[2], const double* src,
-               double* dst) {
+               double* dst, const PhaseMark& mark) {
   const int N = c->d.nbasis, nc = c->ncol, n[2] = {c->d.nalpha, c->d.nbeta};
   if (!c->exp_ready) {
     HIP_TRY(c, launch_pad_rows(c->s.expH1, 2 * N, N, exp_ld(c), c->exp_pad, c->stream));
     c->exp_ready = true;
   }
   OneBody64Args a{};
+  a.mark = mark;
   a.nwalkers = nw;
   a.nbasis = N;
   a.nspin = two_spins(c) ? 2 : 1;
@@ -721,7 +725,7 @@ int one_body_bf16(afqmc_ctx* c, int nw, int s, const uint16_t* aplanes, int64_t 
 // precision the one body is P = phi + (expH1 - I) phi with the product in
 // split-BF16, and the transposed planes of P go to tplanes[0] for the Taylor series.
 int gather(afqmc_ctx* c, int nw, const double* phia, const double* phib, bool with_expH1) {
-  PhaseScope ps(c, AFQMC_PHASE_ONE_BODY);
+  PhaseScope ps(c, AFQMC_PHASE_ONE_BODY, with_expH1 && !c->dplanes ? PhaseScope::KERNEL : PhaseScope::STAMP);
   const int N = c->d.nbasis, na = c->d.nalpha, nb = c->d.nbeta, nc = c->ncol;
   double* P = c->buf[0];
   c->ptp_ready = false;
@@ -741,7 +745,7 @@ int gather(afqmc_ctx* c, int nw, const double* phia, const double* phib, bool wi
   }
   if (with_expH1) {
     const double* const phi[2] = {phia, phib};
-    return one_body64(c, nw, phi, nullptr, nullptr, P);
+    return one_body64(c, nw, phi, nullptr, nullptr, P, ps.mark());
   }
   HIP_TRY(c, hipMemcpy2DAsync(P, 16 * nc, phia, 16 * na, 16 * na, (size_t)nw * N, hipMemcpyDeviceToDevice,
                               c->stream));
@@ -755,7 +759,7 @@ int gather(afqmc_ctx* c, int nw, const double* phia, const double* phib, bool wi
 // layout (mixed precision with the one body), or null.
 int scatter(afqmc_ctx* c, int nw, const double* src, double* phia, double* phib, bool with_expH1,
             const uint16_t* srcT = nullptr) {
-  PhaseScope ps(c, AFQMC_PHASE_ONE_BODY);
+  PhaseScope ps(c, AFQMC_PHASE_ONE_BODY, with_expH1 && !c->dplanes ? PhaseScope::KERNEL : PhaseScope::STAMP);
   const int N = c->d.nbasis, na = c->d.nalpha, nb = c->d.nbeta, nc = c->ncol;
   if (with_expH1 && c->dplanes) {
     int r = ensure_planes(c);
@@ -775,7 +779,7 @@ int scatter(afqmc_ctx* c, int nw, const double* src, double* phia, double* phib,
   }
   if (with_expH1) {
     double* const phi[2] = {phia, phib};
-    return one_body64(c, nw, nullptr, phi, src, nullptr);
+    return one_body64(c, nw, nullptr, phi, src, nullptr, ps.mark());
   }
   HIP_TRY(c, hipMemcpy2DAsync(phia, 16 * na, src, 16 * nc, 16 * na, (size_t)nw * N, hipMemcpyDeviceToDevice,
                               c->stream));
@@ -833,7 +837,7 @@ int taylor_bf16(afqmc_ctx* c, int nw, const double** result, const uint16_t** re
 }
 
 int taylor(afqmc_ctx* c, int nw, const double** result, const uint16_t** resultT = nullptr) {
-  PhaseScope ps(c, AFQMC_PHASE_TAYLOR);
+  PhaseScope ps(c, AFQMC_PHASE_TAYLOR, c->vatoms ? PhaseScope::STAMP : PhaseScope::KERNEL);
   if (resultT) *resultT = nullptr;
   if (c->vatoms && c->d.exp_nmax > 0) return taylor_bf16(c, nw, result, resultT);
   const double* P = c->buf[0];
@@ -847,6 +851,7 @@ int taylor(afqmc_ctx* c, int nw, const double** result, const uint16_t** resultT
   if (c->d.exp_nmax > 0 && taylor64_in_one(t.nbasis)) {  // (no terms: P itself)
     t.out = c->buf[1];
     t.terms = c->d.exp_nmax;
+    t.mark = ps.mark();
     HIP_TRY(c, launch_taylor64_series(t, c->stream));
     *result = t.out;
     return AFQMC_OK;
@@ -855,6 +860,7 @@ int taylor(afqmc_ctx* c, int nw, const double** result, const uint16_t** resultT
     t.prev = prev;
     t.out = prev == c->buf[1] ? c->buf[2] : c->buf[1];
     t.alpha = 1.0 / k;
+    t.mark = ps.mark();  // the first term's; later ones get none
     HIP_TRY(c, launch_taylor64(t, c->stream));
     prev = t.out;
   }
@@ -865,6 +871,7 @@ int taylor(afqmc_ctx* c, int nw, const double** result, const uint16_t** resultT
 // Wq per spin from the half-rotated Cholesky vectors, once per static set.
 int ensure_quad(afqmc_ctx* c) {
   if (c->quad_ready) return AFQMC_OK;
+  close_phase(c);  // once per static set, in no phase
   const int N = c->d.nbasis;
   for (int s = 0; s < (two_spins(c) ? 2 : 1); ++s) {
     const int n = s == 0 ? c->d.nalpha : c->d.nbeta;
@@ -919,11 +926,11 @@ int quad_fp8(afqmc_ctx* c, int nw, int spin, const double* g, const double* gref
   const int n = spin == 0 ? c->d.nalpha : c->d.nbeta;
   const int64_t ld8 = c->q8_ld[spin];
   {
-    PhaseScope ps(c, AFQMC_PHASE_SPLIT);
+    PhaseScope ps(c, AFQMC_PHASE_SPLIT, PhaseScope::STAMP);
     HIP_TRY(c, launch_split_fp8_rows(g, gref, nw, n, N, c->kpad, ld8, c->g8, c->q8_scale + spin, c->q8_rowinv,
                                      c->stream));
   }
-  PhaseScope ps(c, phase);
+  PhaseScope ps(c, phase, PhaseScope::STAMP);
   const int64_t mb = ceil_div(nw, 128);
   if (mb < 1 || mb > (int64_t)c->qunit8_n[spin].size()) return fail(c, AFQMC_ERR_INVALID_ARG, "walker count");
   const int nunits = c->qunit8_n[spin][mb - 1];
@@ -968,10 +975,10 @@ int quad_bf16(afqmc_ctx* c, int nw, int spin, const double* g, const int* walker
   const int N = c->d.nbasis;
   const int n = spin == 0 ? c->d.nalpha : c->d.nbeta;
   {
-    PhaseScope ps(c, AFQMC_PHASE_SPLIT);
+    PhaseScope ps(c, AFQMC_PHASE_SPLIT, PhaseScope::STAMP);
     HIP_TRY(c, launch_split_ghalf(g, (int64_t)nw * n, N, c->kpad, c->gplanes[spin], c->stream, walker_of, n, gref));
   }
-  PhaseScope ps(c, phase);
+  PhaseScope ps(c, phase, PhaseScope::STAMP);
   const int64_t ldn = (int64_t)n * c->kpad;
   const int64_t mb = ceil_div(nw, 128);
   if (mb < 1 || mb > (int64_t)c->qunit_n[spin].size()) return fail(c, AFQMC_ERR_INVALID_ARG, "walker count");
@@ -1018,7 +1025,7 @@ int exchange_spin_quad(afqmc_ctx* c, int nw, int spin, const double* g, const in
     r = quad_bf16(c, nw, spin, g, walker_of, nullptr, false, part, AFQMC_PHASE_EXCHANGE);
     if (r) return r;
   } else {
-    PhaseScope ps(c, AFQMC_PHASE_EXCHANGE);
+    PhaseScope ps(c, AFQMC_PHASE_EXCHANGE, walker_of ? PhaseScope::STAMP : PhaseScope::KERNEL);
     if (walker_of) {
       HIP_TRY(c, launch_sur_gather(g, walker_of, nw, (int64_t)n * N, c->gcomp, c->stream));
       g = c->gcomp;
@@ -1035,6 +1042,7 @@ int exchange_spin_quad(afqmc_ctx* c, int nw, int spin, const double* g, const in
     a.nunits = c->qunit_n[spin][0];
     a.unit_chunks = c->quad64_chunks[spin];
     a.dg = g;
+    a.mark = ps.mark();
     HIP_TRY(c, launch_nt64(a, c->stream));
     HIP_TRY(c, launch_quad_sum(c->qy, a.nunits, nw, part, c->stream));
   }
@@ -1053,7 +1061,7 @@ int exchange_spin(afqmc_ctx* c, int nw, int spin, const double* g, const int* wa
   if (c->d.precision == AFQMC_PREC_MIXED && c->bx_ok[spin]) {
     int r = ensure_planes(c);
     if (r) return r;
-    PhaseScope ps(c, AFQMC_PHASE_EXCHANGE);
+    PhaseScope ps(c, AFQMC_PHASE_EXCHANGE, PhaseScope::STAMP);
     HIP_TRY(c, launch_split_ghalf(g, (int64_t)nw * n, N, c->kpad, c->gplanes[spin], c->stream, walker_of, n));
     ExchangeBf16Args b{};
     b.split = 1;
@@ -1076,7 +1084,7 @@ int exchange_spin(afqmc_ctx* c, int nw, int spin, const double* g, const int* wa
     c->xs_used[spin] = b.xsplit;
     return AFQMC_OK;
   }
-  PhaseScope ps(c, AFQMC_PHASE_EXCHANGE);
+  PhaseScope ps(c, AFQMC_PHASE_EXCHANGE, PhaseScope::STAMP);
   if (walker_of) {
     HIP_TRY(c, launch_sur_gather(g, walker_of, nw, (int64_t)n * N, c->gcomp, c->stream));
     g = c->gcomp;
@@ -1125,7 +1133,8 @@ int do_energy(afqmc_ctx* c, int nw, const double* ga, const double* gb, double* 
   a.exx_est = exx_est;
   a.e1_out = e1_out;
   a.e1_in = e1_in;
-  PhaseScope ps(c, AFQMC_PHASE_ENERGY);
+  PhaseScope ps(c, AFQMC_PHASE_ENERGY, PhaseScope::KERNEL);
+  a.mark = ps.mark();
   HIP_TRY(c, launch_energy(a, c->stream));
   return AFQMC_OK;
 }
@@ -1187,7 +1196,7 @@ int exchange_q_spin(afqmc_ctx* c, int nw, int spin, const double* g) {
     c->xs_used[spin] = 1;
     return AFQMC_OK;
   }
-  PhaseScope ps(c, AFQMC_PHASE_EXCHANGE_CV);
+  PhaseScope ps(c, AFQMC_PHASE_EXCHANGE_CV, PhaseScope::STAMP);
   HIP_TRY(c, launch_split_ghalf(g, (int64_t)nw * n, N, c->kpad, c->gplanes[spin], c->stream, nullptr, n, gT));
   ExchangeBf16Args b{};
   b.split = 0;
@@ -1254,7 +1263,7 @@ int do_energy_surrogate(afqmc_ctx* c, int nw, const double* ga, const double* gb
   cva.e1_factor = c->d.rhf ? 2.0 : 1.0;
   cva.ecore = c->s.ecore;
   {
-    PhaseScope ps(c, AFQMC_PHASE_ENERGY);
+    PhaseScope ps(c, AFQMC_PHASE_ENERGY, PhaseScope::STAMP);
     HIP_TRY(c, launch_sur_cv(cva, c->stream));
   }
   // the MLP term from the features, folded into the predictor
@@ -1387,7 +1396,8 @@ int afqmc_create(afqmc_ctx** out, int device, const afqmc_dims* dims) {
   if (dmalloc((void**)&c->flags, sizeof(int)) != hipSuccess ||
       dmalloc((void**)&c->wflags, sizeof(int) * (size_t)d.nwalkers) != hipSuccess ||
       dmalloc((void**)&c->nfb, sizeof(unsigned long long)) != hipSuccess ||
-      dmalloc((void**)&c->dstate, sizeof(StepState)) != hipSuccess) {
+      dmalloc((void**)&c->dstate, sizeof(StepState)) != hipSuccess ||
+      dmalloc((void**)&c->prof_acc, sizeof(unsigned long long) * AFQMC_NPHASES) != hipSuccess) {
     afqmc_destroy(c);
     return AFQMC_ERR_ALLOC;
   }
@@ -1398,6 +1408,9 @@ int afqmc_create(afqmc_ctx** out, int device, const afqmc_dims* dims) {
     afqmc_destroy(c);
     return AFQMC_ERR_HIP;
   }
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
+    c->prof_tick_ms = 1.0 / khz;
   *out = c;
   return AFQMC_OK;
 }
@@ -1423,11 +1436,7 @@ void afqmc_destroy(afqmc_ctx* c) {
     if (p) (void)hipFree(p);
   for (void* p : c->retired) (void)hipFree(p);
   if (c->graph) (void)hipGraphExecDestroy(c->graph);
-  for (hipEvent_t e : c->ev_free) (void)hipEventDestroy(e);
-  for (const PendingEvent& pe : c->ev_pending) {
-    (void)hipEventDestroy(pe.start);
-    (void)hipEventDestroy(pe.stop);
-  }
+  if (c->prof_acc) (void)hipFree(c->prof_acc);
   delete c;
 }
 
@@ -1894,7 +1903,9 @@ int afqmc_update_weight(afqmc_ctx* c, int32_t nw, const double* ovlp, const doub
   a.walker_ovlp = walker_ovlp;
   a.flags = c->flags;
   a.wflags = c->wflags;
-  PhaseScope ps(c, AFQMC_PHASE_WEIGHT);
+  PhaseScope ps(c, AFQMC_PHASE_WEIGHT, PhaseScope::KERNEL);
+  a.mark = ps.mark();
+  if (a.mark.acc) c->prof_open = -1;  // the kernel closes its phase itself
   HIP_TRY(c, launch_update_weight(a, c->stream));
   return AFQMC_OK;
 }
@@ -1908,6 +1919,7 @@ int afqmc_propagate(afqmc_ctx* c, int32_t nw, double* phia, double* phib, double
   if (r) return r;
   if (!phia || !ga || !weight || !ovlp || !hybrid_energy || (two_spins(c) && (!phib || !gb)))
     return fail(c, AFQMC_ERR_INVALID_ARG, "null array");
+  PhaseChain chain(c);
   r = do_gf(c, nw, phia, phib, ga, gb, wv(c, WV_OVLP_OLD), log_shift, true, true);
   if (r) return r;
   r = gather(c, nw, phia, phib, true);
@@ -1934,6 +1946,7 @@ int afqmc_local_energy(afqmc_ctx* c, int32_t nw, const double* ga, const double*
   r = need_static(c);
   if (r) return r;
   if (!ga || !energy || (two_spins(c) && !gb)) return fail(c, AFQMC_ERR_INVALID_ARG, "null array");
+  PhaseChain chain(c);
   r = do_force_bias(c, nw, ga, gb);
   if (r) return r;
   r = do_fields(c, nw, false, nullptr, 0, 0, nullptr, nullptr);
@@ -2007,7 +2020,8 @@ int afqmc_reortho(afqmc_ctx* c, int32_t nw, double* phia, double* phib, double* 
   a.flags = c->flags;
   a.wflags = c->wflags;
   a.slow = c->qr_slow;
-  PhaseScope ps(c, AFQMC_PHASE_REORTHO);
+  PhaseScope ps(c, AFQMC_PHASE_REORTHO, PhaseScope::KERNEL);
+  a.mark = ps.mark();
   HIP_TRY(c, launch_reortho(a, c->stream));
   return AFQMC_OK;
 }
@@ -2337,36 +2351,21 @@ int afqmc_tune_set(afqmc_ctx* c, int32_t knob, int32_t value) {
 int afqmc_profile(afqmc_ctx* c, int enable) {
   if (!c) return AFQMC_ERR_INVALID_ARG;
   c->prof = enable != 0;
-  for (int i = 0; i < AFQMC_NPHASES; ++i) {
-    c->prof_ms[i] = 0.0;
-    c->prof_count[i] = 0;
-  }
-  // phases recorded before the reset and not yet read are dropped with the
-  // totals (their events go back to the pool; recording an event again
-  // replaces its earlier record)
-  for (const PendingEvent& pe : c->ev_pending) {
-    c->ev_free.push_back(pe.start);
-    c->ev_free.push_back(pe.stop);
-  }
-  c->ev_pending.clear();
+  // the ticks of phases before the reset are cleared on the stream, before the next phase
+  c->prof_clear = true;
+  for (int i = 0; i < AFQMC_NPHASES; ++i) c->prof_count[i] = 0;
   return AFQMC_OK;
 }
 
 int afqmc_profile_read(afqmc_ctx* c, double* ms, int64_t* launches) {
   if (!c || !ms || !launches) return AFQMC_ERR_INVALID_ARG;
   if (c->capturing) return refuse_in_capture(c, "afqmc_profile_read");
+  unsigned long long ticks[AFQMC_NPHASES] = {0};
+  if (!c->prof_clear)
+    HIP_TRY(c, hipMemcpyAsync(ticks, c->prof_acc, sizeof(ticks), hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
-  for (const PendingEvent& pe : c->ev_pending) {
-    float t = 0.0f;
-    HIP_TRY(c, hipEventElapsedTime(&t, pe.start, pe.stop));
-    c->prof_ms[pe.phase] += t;
-    c->prof_count[pe.phase] += 1;
-    c->ev_free.push_back(pe.start);
-    c->ev_free.push_back(pe.stop);
-  }
-  c->ev_pending.clear();
   for (int i = 0; i < AFQMC_NPHASES; ++i) {
-    ms[i] = c->prof_ms[i];
+    ms[i] = (double)ticks[i] * c->prof_tick_ms;
     launches[i] = c->prof_count[i];
   }
   return AFQMC_OK;

@@ -44,8 +44,34 @@ __device__ __forceinline__ uint4 philox4x32(uint4 ctr, uint2 key) {
   return ctr;
 }
 
+// ---------------------------------------------------------------- phase clock
+// Device time per phase, stamped by the kernels themselves: the first kernel of a
+// phase closes the phase that was open (prev, or -1) and opens its own, one atomic
+// add per side without a return value, so acc[p] holds the ticks of the device's
+// wall clock (100 MHz) that phase p's closed intervals took.  An event pair around
+// each phase instead (18 records in a step) took half of a small system's step:
+// loop of N = 24, 16 walkers 747 us with events and 384 us without timing.
+struct PhaseMark {
+  unsigned long long* acc = nullptr;  // [AFQMC_NPHASES], or null: not timed
+  int prev = -1, phase = -1;          // phase to close, phase to open (-1: none)
+};
+__device__ __forceinline__ void phase_add(unsigned long long* acc, int phase, unsigned long long v) {
+  if (phase >= 0) (void)__hip_atomic_fetch_add(acc + phase, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// at the start of a phase's first kernel; one thread of the grid passes `one`
+__device__ __forceinline__ void phase_mark(const PhaseMark& m, bool one) {
+  if (!m.acc || !one) return;
+  const unsigned long long now = wall_clock64();
+  phase_add(m.acc, m.prev, now);
+  phase_add(m.acc, m.phase, 0ull - now);
+}
+// stamps a boundary by itself (a phase whose kernels take no mark; the last phase's end)
+hipError_t launch_phase_mark(const PhaseMark& m, hipStream_t stream);
+hipError_t launch_phase_clear(unsigned long long* acc, int n, hipStream_t stream);
+
 // ---------------------------------------------------------------- GF / overlap
 struct GfArgs {
+  PhaseMark mark;
   int nwalkers, nbasis, nalpha, nbeta, rhf;
   const double* phia;   // [W, N, na] complex
   const double* phib;   // [W, N, nb] complex
@@ -84,6 +110,7 @@ struct NtSegment {
 };
 
 struct NtArgs {
+  PhaseMark mark;
   int64_t m, n;      // rows of A, rows of B (columns of C)
   int nseg, ksplit;  // segments; K ranges (over the chunks of all segments)
   NtSegment seg[2];
@@ -125,6 +152,7 @@ struct OneBody64Spin {
   int out_ld, out_off;
 };
 struct OneBody64Args {
+  PhaseMark mark;
   int nwalkers, nbasis, nspin, ld_exp;
   OneBody64Spin spin[2];
 };
@@ -135,6 +163,7 @@ hipError_t launch_pad_rows(const double* src, int rows, int n, int ld, double* d
 // out[w] = base[w] + alpha V[w] prev[w] ([W, N, ncol] complex; V symmetric, as the
 // packed upper triangle [W, N (N + 1) / 2] complex)
 struct Taylor64Args {
+  PhaseMark mark;
   int nwalkers, nbasis, ncol;
   const double* vhs;
   const double* prev;
@@ -334,6 +363,7 @@ int taylor_rows_padded(int ncol);
 
 // ---------------------------------------------------------------- elementwise
 struct FieldsArgs {
+  PhaseMark mark;
   int nwalkers, nchol, ksplit;
   const double* vbias_part;   // [ksplit, W, X] complex (complex FP32 when part32)
   int part32;
@@ -356,6 +386,7 @@ struct FieldsArgs {
 hipError_t launch_fields(const FieldsArgs& a, hipStream_t stream);
 
 struct WeightArgs {
+  PhaseMark mark;            // phase: opened and closed by the kernel
   int nwalkers;
   const double* ovlp_old;  // [W] complex
   const double* ovlp_new;  // [W] complex
@@ -374,6 +405,7 @@ hipError_t launch_update_weight(const WeightArgs& a, hipStream_t stream);
 hipError_t launch_take_flags(int* src, int* dst, int n, int clear, hipStream_t stream);
 
 struct EnergyArgs {
+  PhaseMark mark;
   int nwalkers, nbasis, nalpha, nbeta, rhf;
   const double* ghalfa;
   const double* ghalfb;
@@ -520,6 +552,7 @@ hipError_t launch_sur_gather(const double* g, const int* walker_of, int k, int64
 
 // ---------------------------------------------------------------- reortho
 struct ReorthoArgs {
+  PhaseMark mark;
   int nwalkers, nbasis, nalpha, nbeta;
   double* phia;
   double* phib;

@@ -36,6 +36,7 @@ __device__ __forceinline__ double draw_normal(uint64_t seed, uint64_t counter, u
 }
 
 __global__ void __launch_bounds__(FLD_THREADS) fields_kernel(FieldsArgs a) {
+  phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
   __shared__ double red[FLD_THREADS / 64];
   const int w = blockIdx.x;
   const int X = a.nchol;
@@ -116,6 +117,7 @@ __global__ void __launch_bounds__(FLD_THREADS) fields_kernel(FieldsArgs a) {
 
 __global__ void update_weight_kernel(WeightArgs a) {
   const int w = blockIdx.x * blockDim.x + threadIdx.x;
+  phase_mark(a.mark, w == 0);
   if (w >= a.nwalkers) return;
   const cplx o_old = ld(a.ovlp_old, w), o_new = ld(a.ovlp_new, w);
   const cplx ratio = cdiv(o_new, o_old);
@@ -139,9 +141,12 @@ __global__ void update_weight_kernel(WeightArgs a) {
   st(a.walker_ovlp, w, o_new);
   if (!isfinite(wnew) && a.flags) atomicOr(a.flags, AFQMC_FLAG_NONFINITE);
   if (!isfinite(wnew) && a.wflags) atomicOr(a.wflags + w, AFQMC_FLAG_NONFINITE);
+  // the step's last phase is this kernel alone: walker 0's thread closes it
+  phase_mark(PhaseMark{a.mark.acc, a.mark.phase, -1}, w == 0);
 }
 
 __global__ void __launch_bounds__(FLD_THREADS) energy_kernel(EnergyArgs a) {
+  phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
   __shared__ double red[FLD_THREADS / 64];
   const int w = blockIdx.x;
   const int N = a.nbasis;
@@ -188,6 +193,12 @@ __global__ void step_set_kernel(StepState* s, unsigned long long counter, double
   }
 }
 
+__global__ void phase_mark_kernel(PhaseMark m) { phase_mark(m, threadIdx.x == 0); }
+
+__global__ void phase_clear_kernel(unsigned long long* acc, int n) {
+  if ((int)threadIdx.x < n) acc[threadIdx.x] = 0;
+}
+
 __global__ void step_advance_kernel(StepState* s, long long dcounter, long long dadam) {
   if (threadIdx.x == 0) {
     s->counter += (unsigned long long)dcounter;
@@ -222,6 +233,16 @@ hipError_t launch_energy(const EnergyArgs& a, hipStream_t stream) {
 
 hipError_t launch_step_set(StepState* state, unsigned long long counter, double eshift, hipStream_t stream) {
   hipLaunchKernelGGL(step_set_kernel, dim3(1), dim3(64), 0, stream, state, counter, eshift);
+  return hipGetLastError();
+}
+
+hipError_t launch_phase_mark(const PhaseMark& m, hipStream_t stream) {
+  hipLaunchKernelGGL(phase_mark_kernel, dim3(1), dim3(64), 0, stream, m);
+  return hipGetLastError();
+}
+
+hipError_t launch_phase_clear(unsigned long long* acc, int n, hipStream_t stream) {
+  hipLaunchKernelGGL(phase_clear_kernel, dim3(1), dim3(64), 0, stream, acc, n);
   return hipGetLastError();
 }
 

@@ -72,6 +72,7 @@ struct ObPlan {
 
 template <int RM>
 __global__ void __launch_bounds__(PG_THREADS, 2) one_body64_kernel(OneBody64Args a) {
+  phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
   using P = ObPlan<RM>;
   constexpr int ST = P::STAGES, TM = 16 * RM;
   extern __shared__ uint4 pg_lds[];
@@ -201,6 +202,7 @@ struct TyPlan {
 
 template <int RN>
 __global__ void __launch_bounds__(PG_THREADS, 2) taylor64_kernel(Taylor64Args a) {
+  phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
   using P = TyPlan<RN>;
   constexpr int ST = P::STAGES;
   extern __shared__ uint4 pg_lds[];
@@ -339,6 +341,7 @@ __global__ void __launch_bounds__(PG_THREADS, 2) taylor64_kernel(Taylor64Args a)
 // values of a row (or, mirrored, 16 of a stored row).
 template <int NCH, int RN>
 __global__ void __launch_bounds__(NCH > 0 ? 512 : 1024) taylor64_series_kernel(Taylor64Args a) {
+  phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
   extern __shared__ uint4 pg_lds[];
   constexpr bool KEEP = NCH > 0 || RN <= 2;  // the base in registers
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

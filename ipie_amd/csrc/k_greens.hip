@@ -28,6 +28,7 @@ __device__ __forceinline__ int gf_nspin(const GfArgs& a) { return (a.nbeta > 0 &
 // psi has zero imaginary parts, whose two MFMAs per step would add only zeros.
 template <int NT, bool REAL>
 __global__ void __launch_bounds__(64 * GF_WAVES) gf_obuild_kernel(GfArgs a, double* __restrict__ obuf, int nmax) {
+  phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
   const int gw = blockIdx.x * GF_WAVES + (threadIdx.x >> 6);
   const int nspin = gf_nspin(a);
   const int task = gw / NT, it = gw % NT;

@@ -85,6 +85,7 @@ __device__ __forceinline__ void nt_barrier() {
 
 template <int RM, int MODE, int EPI>
 __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
+  phase_mark(a.mark, blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0);
   using P = NtPlan<RM, MODE>;
   constexpr int TM = P::TM, ST = P::STAGES;
   extern __shared__ uint4 nt_lds[];

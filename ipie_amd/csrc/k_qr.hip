@@ -568,6 +568,7 @@ __device__ __forceinline__ double qr_fast_sweep(double* __restrict__ X, int N, i
 
 template <int NT>
 __global__ void __launch_bounds__(QR_THREADS, 2) reortho_fast_kernel(ReorthoArgs a) {
+  phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
   constexpr int LD = 16 * NT + 1;
   extern __shared__ cplx smem[];
   __shared__ double logdet[2], sums[QR_WAVES];
@@ -711,6 +712,7 @@ hipError_t launch_qr_nt(const ReorthoArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(reortho_fast_kernel<NT>, dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a);
   } else {
     b.slow = nullptr;
+    if (a.mark.acc && (e = launch_phase_mark(a.mark, stream)) != hipSuccess) return e;
   }
   hipLaunchKernelGGL(reortho_kernel<NT>, dim3(a.nwalkers), dim3(QR_THREADS), 2 * matrix, stream, b);
   return hipGetLastError();

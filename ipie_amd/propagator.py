@@ -44,7 +44,7 @@ class PropagatorTimer:
     tgf the Green's function, tgemm the two one-body halves and the Taylor
     series, tfbias the force bias and xbar, tvhs the VHS construction, tovlp the
     new overlap, tupdate the weight update.  Here the step is one fused C-ABI
-    call, so the fields are read from the context's HIP-event time of the same
+    call, so the fields are read from the context's device time of the same
     phases (afqmc_profile_read; reading one synchronises the context's
     stream, as ipie's own timing does after every phase).  A field may be
     assigned (e.g. reset to 0); later reads add the device time since."""
