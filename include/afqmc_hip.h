@@ -393,12 +393,11 @@ int afqmc_draw_normals(afqmc_ctx* ctx, double* out, int64_t n, uint64_t seed, ui
  * context: psia [N, n_a] / psib [N, n_b] complex are the trial orbitals, the
  * other arrays as in afqmc_greens_function, walker_flags [W] int32 (optional)
  * receives AFQMC_FLAG_SINGULAR OR-ed per walker, and the work is enqueued on
- * `stream` (a hipStream_t, NULL for the null stream).  The LU and inverse work
- * buffers live in a static device array of AFQMC_NOALLOC_SCRATCH_BYTES per
- * GPU (held until the process ends); afqmc_noalloc_scratch_bytes gives what a
- * call needs, and a call that needs more returns AFQMC_ERR_SHAPE.  Every call
- * on one GPU shares that GPU's array: calls that overlap in time on one GPU
- * race.  afqmc_noalloc_last_error returns the calling thread's message of its
+ * `stream` (a hipStream_t, NULL for the null stream).  Calls share no device
+ * memory, so they may overlap in time.  The size of a call is limited:
+ * afqmc_noalloc_scratch_bytes gives its measure, and a call of more than
+ * AFQMC_NOALLOC_SCRATCH_BYTES returns AFQMC_ERR_SHAPE.
+ * afqmc_noalloc_last_error returns the calling thread's message of its
  * last failed call. */
 #define AFQMC_NOALLOC_SCRATCH_BYTES 134217728ULL /* 128 MiB */
 size_t afqmc_noalloc_scratch_bytes(int32_t nwalkers, int32_t nalpha, int32_t nbeta);

@@ -89,13 +89,10 @@ struct GfArgs {
   uint16_t* gplanes[2];
   int kpad;
 };
-size_t gf_lds_bytes(int nalpha, int nbeta);
 // *flag = 1 if any of the n complex values z has a nonzero imaginary part (flag
 // must be zero before; every writer stores 1)
 hipError_t launch_imag_any(const double* z, int64_t n, int* flag, hipStream_t stream);
-// bytes of each GF work buffer (O, O^{-1}): [W][2][nmax][nmax] complex
-size_t gf_work_bytes(int nwalkers, int nalpha, int nbeta);
-hipError_t launch_gf(const GfArgs& a, bool want_ghalf, double* obuf, double* oinv, hipStream_t stream);
+hipError_t launch_gf(const GfArgs& a, bool want_ghalf, hipStream_t stream);
 
 // ---------------------------------------------------------------- GEMMs
 // Rows of a complex operand A (K contiguous) times rows of a real operand B
