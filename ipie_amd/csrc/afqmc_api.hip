@@ -92,7 +92,7 @@ struct afqmc_ctx {
   int fb_split_spin = BF16_FB_SPLIT;  // split-BF16 force bias: K ranges per spin
   int fb_cap = 0;                     // K ranges vbias_part holds (0: not allocated yet)
   int quad_target = QUAD_TARGET_WGS;  // split-BF16 quadratic form: workgroups the column units aim for
-  int tile_fb = 0, tile_vhs = 0, tile_ob = 0;  // split-BF16 GEMM tile shapes (force bias, VHS, one body)
+  int tile_fb = -1, tile_vhs = -1, tile_ob = -1;  // split-BF16 GEMM tile shapes (force bias, VHS, one body; -1: by rule)
   int quad_rgroup = 0;  // split-BF16 quadratic form: row blocks per workgroup group (0: all)
   int taylor_variant = 0;  // split-BF16 Taylor kernel (TaylorBf16Args::variant)
   int64_t qy_cap = 0;                 // complex entries qy holds (split-BF16 quadratic form)
@@ -988,6 +988,8 @@ int quad_bf16(afqmc_ctx* c, int nw, int spin, const double* g, const int* walker
   b.kchunks = (int)(ldn / 32);
   b.ksplit = 1;
   b.single = single ? 1 : 0;
+  b.tile = -1;
+
   b.epilogue = BF16_EPI_QDOT;
   b.out = c->qy;
   b.scale = 1.0;
@@ -2287,7 +2289,7 @@ int afqmc_tune_get(afqmc_ctx* c, int32_t knob, int32_t* value, int32_t* lo, int3
     case AFQMC_TUNE_TILE_ONE_BODY:
       // split-BF16 GEMM tile shapes (mixed precision; the force bias needs Cholesky vectors)
       if (c->d.precision != AFQMC_PREC_MIXED || c->d.nchol < 1) return AFQMC_OK;
-      *value = knob == AFQMC_TUNE_TILE_FB ? c->tile_fb : knob == AFQMC_TUNE_TILE_VHS ? c->tile_vhs : c->tile_ob;
+      *value = std::max(0, knob == AFQMC_TUNE_TILE_FB ? c->tile_fb : knob == AFQMC_TUNE_TILE_VHS ? c->tile_vhs : c->tile_ob);  // 0 until it is set
       *lo = 0;
       *hi = BF16_TILES - 1;
       return AFQMC_OK;

@@ -249,11 +249,12 @@ struct Bf16GemmArgs {
   // i scale C[row][col], col = atom 256 + r 16 + c, rounded to FP32 first
   uint16_t* out16;
   int64_t atom_stride;
-  // workgroup tile shape 0 .. BF16_TILES - 1 (bf16_tile_dims); the quadratic form
-  // (QDOT, unit tables) and the single product take shape 0
+  // workgroup tile shape 0 .. BF16_SHAPES - 1 (bf16_tile_dims), negative: by the
+  // launcher's rule; the quadratic form (QDOT, unit tables) takes the shapes of its
+  // columns (0, 5, 6), the single product shape 0.  Every shape gives the same bits.
   int tile;
-  // with a unit table: consecutive workgroups cover rgroup row blocks x units
-  // (row blocks fastest), group after group of row blocks; 0 or >= the row-block
+  // with a unit table: consecutive workgroups cover rgroup row blocks (of 128 rows) x
+  // units (row blocks fastest), group after group of row blocks; 0 or >= the row-block
   // count: all row blocks x units
   int rgroup;
   // single product in FP8 (E4M3): the operands are byte arrays addressed in
@@ -269,7 +270,8 @@ struct Bf16GemmArgs {
   int cols_fast;
 };
 hipError_t launch_bf16_gemm(const Bf16GemmArgs& a, hipStream_t stream);
-constexpr int BF16_TILES = 6;
+constexpr int BF16_TILES = 6;   // shapes 0 .. 5 are the tuning values
+constexpr int BF16_SHAPES = 7;  // shape 6: picked by the rule only
 // rows x columns of a workgroup tile shape (false for an unknown shape)
 bool bf16_tile_dims(int tile, int* rows, int* cols);
 

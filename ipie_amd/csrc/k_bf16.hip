@@ -52,13 +52,21 @@ struct Tile {
 // waves; shapes 0-3 three LDS stages of the 3-product form within 160 KiB,
 // shape 4 (64 x 80 per wave: 29% fewer LDS bytes per MFMA than 32 x 80) two,
 // shape 5 two stages of 36 KiB, so that two workgroups share a CU (one can
-// run its epilogue while the other computes: short K, heavy epilogues).
+// run its epilogue while the other computes: short K, heavy epilogues).  Shape 6,
+// 4 waves and two workgroups a CU, is for few rows and is not a tuning value.
 using Tile0 = Tile<4, 2, 2, 5>;     // 128 x 160
 using Tile1 = Tile<4, 2, 2, 4>;     // 128 x 128
 using Tile2 = Tile<8, 1, 1, 5>;     // 128 x 80
 using Tile3 = Tile<4, 2, 1, 5>;     // 64 x 160
 using Tile4 = Tile<2, 4, 4, 5, 2>;  // 128 x 320
 using Tile5 = Tile<4, 2, 1, 5, 2>;  // 64 x 160
+using Tile6 = Tile<2, 2, 1, 5, 2>;  // 32 x 160, 4 waves
+
+// shapes whose column tiles and waves are the quadratic form's (units and dot slots)
+template <class TL>
+struct QdotTile {
+  static constexpr bool value = TL::C == Tile0::C && TL::GC == Tile0::GC;
+};
 
 // 8 waves in a BX_GR x BX_GC grid, each owning BX_MR x BX_MC tiles of 16 x 16 (shape 0)
 constexpr int BX_GR = Tile0::GR, BX_GC = Tile0::GC, BX_MR = Tile0::MR, BX_MC = Tile0::MC;
@@ -474,6 +482,48 @@ __device__ __forceinline__ void bx_sub(const uint4* sub, int wr, int wc, int l16
   }
 }
 
+// The operand fragments of one K chunk of the 3-product form in registers, and the
+// chunk's products in the order of bx_sub.
+template <class TL>
+struct BxFrags {
+  v8bf arh[(TL::MR)], arl[(TL::MR)], aih[(TL::MR)], ail[(TL::MR)], bh[(TL::MC)], bl[(TL::MC)];
+  static constexpr int READS = 4 * TL::MR + 2 * TL::MC, MFMAS = 6 * TL::MR * TL::MC;
+};
+template <class TL>
+__device__ __forceinline__ void bx_read(BxFrags<TL>& f, const uint4* stage, int wr, int wc, int l16, int q) {
+  const uint16_t* As = reinterpret_cast<const uint16_t*>(stage);
+  const uint16_t* Bs = As + 8 * Bx<true, TL>::A_VEC;
+#pragma unroll
+  for (int j = 0; j < TL::MC; ++j) {
+    const int col = (wc * TL::MC + j) * 16 + l16;
+    f.bh[j] = lds_frag(Bs, col, q);
+    f.bl[j] = lds_frag(Bs, TL::C + col, q);
+  }
+#pragma unroll
+  for (int i = 0; i < TL::MR; ++i) {
+    const int row = (wr * TL::MR + i) * 16 + l16;
+    f.arh[i] = lds_frag(As, row, q);
+    f.arl[i] = lds_frag(As, TL::R + row, q);
+    f.aih[i] = lds_frag(As, 2 * TL::R + row, q);
+    f.ail[i] = lds_frag(As, 3 * TL::R + row, q);
+  }
+}
+template <bool TR, class TL>
+__device__ __forceinline__ void bx_multiply(const BxFrags<TL>& f, v4f (&re)[(TL::MR)][(TL::MC)],
+                                            v4f (&im)[(TL::MR)][(TL::MC)]) {
+#pragma unroll
+  for (int i = 0; i < TL::MR; ++i)
+#pragma unroll
+    for (int j = 0; j < TL::MC; ++j) {
+      re[i][j] = mfma_ab(f.arh[i], f.bh[j], re[i][j], TR);
+      im[i][j] = mfma_ab(f.aih[i], f.bh[j], im[i][j], TR);
+      re[i][j] = mfma_ab(f.arh[i], f.bl[j], re[i][j], TR);
+      im[i][j] = mfma_ab(f.aih[i], f.bl[j], im[i][j], TR);
+      re[i][j] = mfma_ab(f.arl[i], f.bh[j], re[i][j], TR);
+      im[i][j] = mfma_ab(f.ail[i], f.bh[j], im[i][j], TR);
+    }
+}
+
 // The nsub sub-chunks of LDS stage `stage`.  A full stage is one straight
 // block, so that the LDS reads of a sub-chunk can be scheduled under the
 // MFMAs of the one before.
@@ -682,10 +732,11 @@ __global__ void __launch_bounds__(TL::THREADS) bf16_gemm_kernel(Bf16GemmArgs a) 
     rb = (lin / ncu) % mb;
     z = lin / ncu / mb;
   }
-  if (a.units && a.rgroup > 0 && a.rgroup < mb) {
+  const int rgroup = a.rgroup * (128 / TL::R);  // (counted in row blocks of 128)
+  if (a.units && rgroup > 0 && rgroup < mb) {
     // groups of rgroup row blocks, each over every unit (the workgroups that run
     // together on one XCD: rgroup row blocks x several units of one K block)
-    const int R = a.rgroup, rem = lin % (ncu * R);
+    const int R = rgroup, rem = lin % (ncu * R);
     rb = (lin / (ncu * R)) * R + rem % R;
     cu = rem / R;
     z = 0;
@@ -745,6 +796,52 @@ __global__ void __launch_bounds__(TL::THREADS) bf16_gemm_kernel(Bf16GemmArgs a) 
       static_assert(ST >= 2 && ST <= 4 && (ST - 2) * C::KS <= 3, "two to four LDS stages, at most 3 sub-chunks pending");
       int64_t da[(Dl<SPLIT, TL>::A_INS)], db[(Dl<SPLIT, TL>::B_INS)];
       dl_sources<SPLIT, TL>(da, db, a, rb, cb, wave, lane);
+      if constexpr (SPLIT && ST == 3) {
+        // Fragments one chunk ahead: while chunk t is multiplied from registers, chunk
+        // t + 1 is read from its stage, t + 2 lands and t + 3 is issued into t's buffer,
+        // which every wave read a chunk before.
+        // (Bound by the matrix units between barriers: N = 400, 1024 walkers, VHS 2404 ->
+        // 2129 us, 1150 TFLOP/s computed, and exchange 3767 -> 3546 us, against every
+        // fragment of a chunk read before its first product.)
+        static_assert(C::KS == 1, "a stage is a chunk");
+        constexpr int I = Dl<SPLIT, TL>::INS_SUB;
+        BxFrags<TL> f[2];
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+          if (s < nst) dl_issue<SPLIT, TL>(lds_u4, s, 1, a.a, a.b, da, db, c0 + s, wave, lane);
+        dl_wait<SPLIT, TL>(min(2, nst - 1));
+        dl_barrier();
+        bx_read<TL>(f[0], lds_u4, wr, wc, l16, q);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        dl_wait<SPLIT, TL>(nst > 2 ? 1 : 0);
+        dl_barrier();
+        int buf = 0;  // t % 3
+        const auto step = [&](int t, const BxFrags<TL>& now, BxFrags<TL>& next) __attribute__((always_inline)) {
+          const bool more = t + 3 < nst;
+          if (more) dl_issue<SPLIT, TL>(lds_u4, buf, 1, a.a, a.b, da, db, c0 + t + 3, wave, lane);
+          buf = buf == 2 ? 0 : buf + 1;
+          __builtin_amdgcn_sched_barrier(0);
+          bx_read<TL>(next, lds_u4 + buf * C::STAGE_VEC, wr, wc, l16, q);  // (past the end: stale, not used)
+          bx_multiply<TR, TL>(now, re, im);
+          // a read after every few products
+          constexpr int EACH = BxFrags<TL>::MFMAS / (BxFrags<TL>::READS + 1);
+#pragma unroll
+          for (int k = 0; k < BxFrags<TL>::READS; ++k) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, EACH, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+          if (more) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(I) : "memory");
+          else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        };
+        int t = 0;
+        for (; t + 1 < nst; t += 2) {
+          step(t, f[0], f[1]);
+          step(t + 1, f[1], f[0]);
+        }
+        if (t < nst) step(t, f[0], f[1]);
+      } else {
       // prologue: stages 0 .. ST - 2 issued; stage 0 landed, the rest may stay in flight
       int pend0 = 0;
 #pragma unroll
@@ -769,6 +866,7 @@ __global__ void __launch_bounds__(TL::THREADS) bf16_gemm_kernel(Bf16GemmArgs a) 
         dl_wait<SPLIT, TL>(pend);
         dl_barrier();
         buf = buf == ST - 1 ? 0 : buf + 1;
+      }
       }
     } else {
       static_assert(TL::ST == 3, "register staging uses three stages");
@@ -796,7 +894,7 @@ __global__ void __launch_bounds__(TL::THREADS) bf16_gemm_kernel(Bf16GemmArgs a) 
     if (a.epilogue == BF16_EPI_QDOT) {
       // (the quadratic form runs with tile shape 0 and plain accumulators only:
       // launch_bf16_gemm; each epilogue is compiled only where it can run)
-      if constexpr (!TR && std::is_same<TL, Tile0>::value) {
+      if constexpr (!TR && QdotTile<TL>::value) {
       // per-row dot with d over this wave's 80 columns, then across the 16 lanes
       // of a row; lane l16 = 4 i + r keeps the sum of row (i, r).  The lane's
       // columns and d_ref are set up once, and the next row's d values are
@@ -1520,7 +1618,8 @@ constexpr bool kDl = AFQMC_BF16_DL != 0;
 template <bool SPLIT, bool TR, class TL, bool F8 = false>
 hipError_t launch_bf16_gemm_t(const Bf16GemmArgs& a, hipStream_t stream) {
   const int64_t nb = ceil_div(a.nn, TL::C), mb = ceil_div(a.m, TL::R);
-  const int64_t mbg = (a.units && a.rgroup > 0 && a.rgroup < mb) ? ceil_div(mb, a.rgroup) * a.rgroup : mb;
+  const int rgroup = a.rgroup * (128 / TL::R);  // (counted in row blocks of 128)
+  const int64_t mbg = (a.units && rgroup > 0 && rgroup < mb) ? ceil_div(mb, rgroup) * rgroup : mb;
   const int64_t grid = mbg * (a.units ? (int64_t)a.nunits : nb * a.ksplit);
   constexpr size_t lds = Bx<SPLIT, TL>::STAGES_ALL;
   hipError_t e = allow_lds((const void*)bf16_gemm_kernel<SPLIT, TR, kDl, TL, F8>, lds);
@@ -1538,17 +1637,65 @@ hipError_t launch_bf16_gemm_shape(const Bf16GemmArgs& a, hipStream_t stream) {
     case 3: return launch_bf16_gemm_t<true, TR, Tile3>(a, stream);
     case 4: return launch_bf16_gemm_t<true, TR, Tile4>(a, stream);
     case 5: return launch_bf16_gemm_t<true, TR, Tile5>(a, stream);
+    case 6: return launch_bf16_gemm_t<true, TR, Tile6>(a, stream);
     default: return launch_bf16_gemm_t<true, TR, Tile0>(a, stream);
   }
 }
 
-hipError_t launch_bf16_gemm(const Bf16GemmArgs& a, hipStream_t stream) {
+// Tile shape of a 3-product GEMM (Bf16GemmArgs::tile < 0): the smallest rounds of
+// workgroups x (K chunks x time per chunk + epilogue), the quadratic form among the
+// shapes with its columns.  Time per chunk of a busy CU (us, two workgroups for the
+// two-stage 64- and 32-row shapes, less where each CU has one); the epilogue moves its bytes
+// per output at the CU's share of 4.4 TB/s, 50 GB/s at most; two workgroups on a CU
+// hide a quarter.  Measured (us; 128 x 160 always -> by this rule):
+//   N   W     force bias    VHS          one body x 4   exchange
+//   24  10    19 -> 16      13 -> 11     47 -> 37       41 -> 30
+//   150 300   56 -> 41      82 -> 63     133 -> 85      118 -> 109
+//   200 512   90 -> 80      180 -> 159   193 -> 144     229
+//   400 12    180 -> 123    306 -> 230   159 -> 108     389 -> 264
+//   400 1024  911 -> 864    2129         1197 -> 1148   3546
+int bf16_tile_by_rule(const Bf16GemmArgs& a) {
+  struct Shape {
+    int rows, cols, per_cu;
+    double chunk, chunk_alone;
+  };
+  constexpr Shape shapes[] = {{128, 160, 1, 1.67, 1.67}, {128, 128, 1, 1.44, 1.44}, {128, 80, 1, 1.20, 1.20},
+                              {64, 160, 1, 1.11, 1.11},  {128, 320, 1, 3.19, 3.19}, {64, 160, 2, 1.85, 1.40},
+                              {32, 160, 2, 1.52, 1.30}};
+  const bool quad = a.epilogue == BF16_EPI_QDOT || a.units;
+  const double bytes = a.epilogue == BF16_EPI_ADD ? 40.0 : quad ? 16.0 : 8.0;
+  int best = 0;
+  double least = 0.0;
+  for (int t = 0; t < BF16_SHAPES; ++t) {
+    const Shape& s = shapes[t];
+    if (quad && t != 0 && t != 5 && t != 6) continue;
+    const int64_t blocks = a.units ? a.nunits : ceil_div(a.nn, s.cols) * a.ksplit;
+    const int64_t wgs = ceil_div(a.m, s.rows) * blocks;
+    const bool shared = s.per_cu > 1 && wgs > 256;
+    // (units cover half of the chunks of each column tile)
+    const double chunks = a.units ? 0.5 * a.kchunks * ceil_div(a.nn, s.cols) / a.nunits : (double)a.kchunks / a.ksplit;
+    const double bw = wgs > 88 ? 4.4e6 / (double)(wgs < 256 ? wgs : 256) : 5e4;  // bytes per us and CU
+    const double round = chunks * (shared ? s.chunk : s.chunk_alone) + (shared ? 2 : 1) * s.rows * s.cols * bytes / bw;
+    const double time = (double)ceil_div(wgs, 256 * (shared ? s.per_cu : 1)) * round * (shared ? 0.75 + 0.25 * (bytes < 40.0) : 1.0);
+    if (t == 0 || time < least) {
+      least = time;
+      best = t;
+    }
+  }
+  return best;
+}
+
+hipError_t launch_bf16_gemm(const Bf16GemmArgs& args, hipStream_t stream) {
+  Bf16GemmArgs a = args;
   if (a.m < 1 || a.nn < 1 || a.kchunks < 1 || a.ksplit < 1 || a.lda % BX_KC != 0 || a.ldb % BX_KC != 0 ||
       (int64_t)a.kchunks * BX_KC > a.lda || (int64_t)a.kchunks * BX_KC > a.ldb)
     return hipErrorInvalidValue;
-  if (a.tile < 0 || a.tile >= BF16_TILES) return hipErrorInvalidValue;
-  // the quadratic form's unit tables and dot slots, and the single product, use shape 0
-  if (a.tile != 0 && (a.epilogue == BF16_EPI_QDOT || a.units || a.single)) return hipErrorInvalidValue;
+  if (a.tile < 0) a.tile = a.single ? 0 : bf16_tile_by_rule(a);
+  if (a.tile >= BF16_SHAPES) return hipErrorInvalidValue;
+  // the single product uses shape 0, the quadratic form's unit tables and dot slots
+  // the shapes with its columns
+  if (a.tile != 0 && a.single) return hipErrorInvalidValue;
+  if ((a.epilogue == BF16_EPI_QDOT || a.units) && a.tile != 0 && a.tile != 5 && a.tile != 6) return hipErrorInvalidValue;
   if (a.epilogue == BF16_EPI_VHS && (int64_t)a.nbasis * (a.nbasis + 1) / 2 != a.nn) return hipErrorInvalidValue;
   if (a.epilogue == BF16_EPI_VATOM && (a.out16 == nullptr || a.nn % 256 != 0 || a.atom_stride < a.nn / 256 * 1024))
     return hipErrorInvalidValue;
@@ -1579,6 +1726,7 @@ bool bf16_tile_dims(int tile, int* rows, int* cols) {
     case 3: *rows = Tile3::R; *cols = Tile3::C; return true;
     case 4: *rows = Tile4::R; *cols = Tile4::C; return true;
     case 5: *rows = Tile5::R; *cols = Tile5::C; return true;
+    case 6: *rows = Tile6::R; *cols = Tile6::C; return true;
     default: return false;
   }
 }
