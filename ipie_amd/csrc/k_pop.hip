@@ -4,8 +4,7 @@
 //                      then the method's decisions as a source map src[i]
 //                      (slot i takes walker src[i]'s buffer) and the weights
 //                      afterwards:
-//                        pair_branch  stable sort of |w| (bitonic on the key
-//                                     (|w|, index)), lightest and heaviest
+//                        pair_branch  stable sort of |w|, lightest and heaviest
 //                                     paired while outside [min, max]; the
 //                                     k-th branched walker (slot order) fills
 //                                     the k-th killed slot
@@ -41,16 +40,55 @@ namespace afqmc {
 namespace {
 
 constexpr int POP_THREADS = 1024;
+constexpr int POP_RANK = 1024;  // walkers whose sort counts ranks (one per thread)
 
+// key[0] + key[1] + ... in this order (one thread; the reads do not wait for the sum)
+__device__ __forceinline__ double serial_sum(const double* key, int n) {
+  double t = 0.0;
+  int i = 0;
+  for (; i + 16 <= n; i += 16) {
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = key[i + u];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) t += v[u];
+  }
+  for (; i < n; ++i) t += key[i];
+  return t;
+}
+
+// Sum of `count` over the threads before this one (waves: one int per wave).
+__device__ __forceinline__ int slots_before(int count, int* waves) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int incl = count;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += v;
+  }
+  if (lane == 63) waves[wid] = incl;
+  __syncthreads();
+  int before = incl - count;
+  for (int v = 0; v < wid; ++v) before += waves[v];
+  __syncthreads();
+  return before;
+}
+
+// One workgroup, latency-bound: every chain over the walkers but the total (whose order
+// numpy.cumsum's sums fix) is spread over the threads.  512 walkers, pair branching:
+// 82 us with the total, the pairs and the map walked by one thread and a bitonic sort
+// (45 barriers), 25 us now.
 __global__ void __launch_bounds__(POP_THREADS) pop_plan_kernel(PopPlanArgs a) {
   __shared__ double key[POP_MAX];   // |scaled w| (sorted for pair_branch; cumulative for comb / SR)
   __shared__ int idx[POP_MAX];      // walker index of key (pair_branch); parent count (comb)
   __shared__ unsigned char stat[POP_MAX];  // pair_branch: 1 live, 2 branched, 0 killed
   __shared__ double s_total, s_scale;
+  __shared__ int s_pairs, waves[2][POP_THREADS / 64];
   const int tid = threadIdx.x, nw = a.nwalkers;
+  for (int i = tid; i < nw; i += POP_THREADS) key[i] = fabs(a.weight[i]);
+  if (tid == 0) s_pairs = nw / 2;
+  __syncthreads();
   if (tid == 0) {
-    double t = 0.0;
-    for (int i = 0; i < nw; ++i) t += fabs(a.weight[i]);
+    const double t = serial_sum(key, nw);
     s_total = t;
     s_scale = t / a.target;
     a.total[0] = t;
@@ -62,6 +100,7 @@ __global__ void __launch_bounds__(POP_THREADS) pop_plan_kernel(PopPlanArgs a) {
     const double ws = ok ? a.weight[i] / scale : a.weight[i];
     a.new_weight[i] = ws;
     a.src[i] = i;
+    key[i] = fabs(ws);
   }
   if (!ok) {  // the caller raises on total < 1e-8; weights and map untouched
     if (tid == 0) a.npairs[0] = 0;
@@ -71,72 +110,101 @@ __global__ void __launch_bounds__(POP_THREADS) pop_plan_kernel(PopPlanArgs a) {
   if (a.method == POP_RESCALE) {
     if (tid == 0) a.npairs[0] = 0;
   } else if (a.method == POP_PAIR_BRANCH) {
-    int np2 = 1;
-    while (np2 < nw) np2 <<= 1;
-    for (int i = tid; i < np2; i += POP_THREADS) {
-      key[i] = i < nw ? fabs(a.new_weight[i]) : INFINITY;
-      idx[i] = i;
-      stat[i] = 1;
-    }
-    __syncthreads();
-    // bitonic sort ascending by (key, index): equal keys keep the input order
-    for (int size = 2; size <= np2; size <<= 1)
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
-        for (int i = tid; i < np2; i += POP_THREADS) {
-          const int j = i ^ stride;
-          if (j > i) {
-            const bool up = (i & size) == 0;
-            const bool gt = key[i] > key[j] || (key[i] == key[j] && idx[i] > idx[j]);
-            if (gt == up) {
-              const double tk = key[i];
-              key[i] = key[j];
-              key[j] = tk;
+    // ascending by (|w|, index), equal weights in the input order: by the bits of
+    // |w|, as ordered as the values and total, so that the result is a permutation
+    // whatever the weights
+    unsigned long long* bits = reinterpret_cast<unsigned long long*>(key);
+    double* sk = key;
+    int* si = idx;
+    for (int i = tid; i < nw; i += POP_THREADS) stat[i] = 1;
+    if (nw <= POP_RANK) {
+      // the rank of walker i among all: fewer instructions than the sort's barriers take
+      // up to 1024 walkers
+      sk = key + POP_RANK;
+      si = idx + POP_RANK;
+      if (tid < nw) {
+        const unsigned long long mine = bits[tid];
+        int rank = 0;
+#pragma unroll 8
+        for (int j = 0; j < nw; ++j) rank += bits[j] < mine || (bits[j] == mine && j < tid);
+        sk[rank] = key[tid];
+        si[rank] = tid;
+      }
+      __syncthreads();
+    } else {
+      int np2 = 1;
+      while (np2 < nw) np2 <<= 1;
+      for (int i = tid; i < np2; i += POP_THREADS) {
+        if (i >= nw) bits[i] = ~0ull;  // after every |w|, NaN too
+        idx[i] = i;
+      }
+      __syncthreads();
+      // bitonic sort
+      for (int size = 2; size <= np2; size <<= 1)
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+          for (int i = tid; i < np2; i += POP_THREADS) {
+            const int j = i ^ stride;
+            if (j > i) {
+              const bool up = (i & size) == 0;
+              const unsigned long long ki = bits[i], kj = bits[j];
+              const bool gt = ki > kj || (ki == kj && idx[i] > idx[j]);
+              if (gt == up) {
+                bits[i] = kj;
+                bits[j] = ki;
               const int ti = idx[i];
-              idx[i] = idx[j];
-              idx[j] = ti;
+                idx[i] = idx[j];
+                idx[j] = ti;
+              }
             }
           }
+          __syncthreads();
         }
-        __syncthreads();
-      }
-    if (tid == 0) {
-      int s = 0, e = nw - 1, k = 0;
-      while (s < e) {
-        const double ws = key[s], we = key[e];
-        if (!(ws < a.min_weight || we > a.max_weight)) break;
-        const double wab = ws + we;
-        const double r = a.uniforms[k++];
-        const int is = idx[s], ie = idx[e];
-        const bool heavy = r < we / wab;  // clone the heavy walker, kill the light one
-        const int ib = heavy ? ie : is;
-        stat[ib] = 2;
-        stat[heavy ? is : ie] = 0;
-        a.new_weight[ib] = 0.5 * wab;
-        ++s;
-        --e;
-      }
-      a.npairs[0] = k;
-      int kb = 0, kk = 0;
-      for (int p = 0; p < k; ++p) {
-        while (stat[kb] != 2) ++kb;
-        while (stat[kk] != 0) ++kk;
-        a.src[kk] = kb;
-        a.new_weight[kk] = a.new_weight[kb];
-        ++kb;
-        ++kk;
-      }
     }
+    // pairs (p, nw - 1 - p) from the outside in, up to the first within the bounds
+    for (int q = tid; q < nw / 2; q += POP_THREADS)
+      if (!(sk[q] < a.min_weight || sk[nw - 1 - q] > a.max_weight)) atomicMin(&s_pairs, q);
+    __syncthreads();
+    const int k = s_pairs;
+    for (int q = tid; q < k; q += POP_THREADS) {
+      const double ws = sk[q], we = sk[nw - 1 - q];
+      const double wab = ws + we;
+      const double r = a.uniforms[q];
+      const int is = si[q], ie = si[nw - 1 - q];
+      const bool heavy = r < we / wab;  // clone the heavy walker, kill the light one
+      const int ib = heavy ? ie : is;
+      stat[ib] = 2;
+      stat[heavy ? is : ie] = 0;
+      a.new_weight[ib] = 0.5 * wab;
+    }
+    if (tid == 0) a.npairs[0] = k;
+    __syncthreads();
+    // the k-th branched slot fills the k-th killed one
+    const int chunk = (nw + POP_THREADS - 1) / POP_THREADS, i0 = min(tid * chunk, nw), i1 = min(i0 + chunk, nw);
+    int nb = 0, nk = 0;
+    for (int i = i0; i < i1; ++i) {
+      nb += stat[i] == 2;
+      nk += stat[i] == 0;
+    }
+    int kb = slots_before(nb, waves[0]), kk = slots_before(nk, waves[1]);
+    int* branched = idx;  // (the sorted indices are no longer needed)
+    for (int i = i0; i < i1; ++i)
+      if (stat[i] == 2) branched[kb++] = i;
+    __syncthreads();
+    for (int i = i0; i < i1; ++i)
+      if (stat[i] == 0) {
+        const int b = branched[kk++];
+        a.src[i] = b;
+        a.new_weight[i] = a.new_weight[b];
+      }
   } else if (a.method == POP_COMB) {
     if (tid == 0) {
       // cumulative scaled weights and the comb (i + r) total / target
-      double c = 0.0;
+      double tw = 0.0;
       for (int i = 0; i < nw; ++i) {
-        c += fabs(a.new_weight[i]);
-        key[i] = c;
+        tw += key[i];
+        key[i] = tw;
         idx[i] = 0;
       }
-      double tw = 0.0;
-      for (int i = 0; i < nw; ++i) tw += fabs(a.new_weight[i]);
       const int target = (int)a.target;
       const double r = a.uniforms[0];
       int iw = 0, ic = 0;
@@ -168,7 +236,7 @@ __global__ void __launch_bounds__(POP_THREADS) pop_plan_kernel(PopPlanArgs a) {
     if (tid == 0) {
       double c = 0.0;
       for (int i = 0; i < nw; ++i) {
-        c += fabs(a.new_weight[i]);
+        c += key[i];
         key[i] = c;
       }
       a.npairs[0] = 0;
