@@ -795,6 +795,28 @@ int taylor_bf16(afqmc_ctx* c, int nw, const double** result, const uint16_t** re
   if (!c->ptp_ready)
     HIP_TRY(c, launch_split_transpose(P, nw, (int)c->d.nwalkers, N, nc, rpad, c->kpad, c->tplanes[0], c->stream));
   c->ptp_ready = false;
+  if (c->taylor_variant == 0 && taylor_bf16_in_one(N, c->kpad)) {
+    TaylorBf16Args t{};
+    t.nwalkers = nw;
+    t.wcap = (int)c->d.nwalkers;
+    t.nbasis = N;
+    t.ncol = nc;
+    t.rpad = rpad;
+    t.kpad = c->kpad;
+    t.tin = c->tplanes[0];
+    t.vatoms = c->vatoms;
+    t.zatom = c->zatom;
+    t.natom_side = vhs_atom_side(N);
+    t.atom_stride = vhs_atom_count(N) * 1024;
+    t.init = P;
+    t.q = Q;
+    t.nterms = c->d.exp_nmax;
+    t.qout = c->tplanes[c->d.exp_nmax == 1 ? 1 : 0];
+    HIP_TRY(c, launch_taylor_bf16_series(t, c->stream));
+    *result = Q;
+    if (resultT) *resultT = t.qout;
+    return AFQMC_OK;
+  }
   for (int k = 1; k <= c->d.exp_nmax; ++k) {
     TaylorBf16Args t{};
     t.nwalkers = nw;

@@ -332,6 +332,9 @@ struct TaylorBf16Args {
                             // (taylor16_kernel)
 };
 hipError_t launch_taylor_bf16(const TaylorBf16Args& a, hipStream_t stream);
+// all nterms terms in one launch (tin: planes of init^T; q, qout as the last term's)
+bool taylor_bf16_in_one(int nbasis, int kpad);
+hipError_t launch_taylor_bf16_series(const TaylorBf16Args& a, hipStream_t stream);
 // Taylor terms k <= TAYLOR_SPLIT_TERMS use three BF16 products, later ones one.
 // Each term but the last writes its four split planes to a buffer of its own
 // (the next term's operand, hi planes alone for a one-product term) and the

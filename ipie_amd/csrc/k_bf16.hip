@@ -1135,8 +1135,12 @@ __device__ __forceinline__ int atom_vec(int r, int h) { return r * 2 + (h ^ (((r
 // 8 (q & 1) .. + 7, two transposing loads of 4 rows each (lane r' of a 16-lane
 // group supplies row r' / 4, quarter r' % 4; lane i receives element i of each
 // of the 4 rows).
-__device__ __forceinline__ v8bf ty_bfrag(const uint4* lds, int vb, int l16, int q, bool mirror) {
-  if (!mirror) return as_v8bf(reinterpret_cast<const v4u*>(lds)[vb + atom_vec(l16, q & 1)]);
+// kind (wave-uniform): both atoms of the chunk stored (0) or mirrors (1), or the first a
+// mirror (2: lane groups 0 and 1 take it; both forms are read by every lane, since the
+// transposing load is defined for full waves).
+__device__ __forceinline__ v8bf ty_bfrag(const uint4* lds, int vb, int l16, int q, int kind) {
+  const v4u* stored = reinterpret_cast<const v4u*>(lds) + vb + atom_vec(l16, q & 1);
+  if (kind == 0) return as_v8bf(*stored);
   v4bf t[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
@@ -1144,8 +1148,13 @@ __device__ __forceinline__ v8bf ty_bfrag(const uint4* lds, int vb, int l16, int 
     const char* p = reinterpret_cast<const char*>(lds + vb + atom_vec(r, qt >> 1)) + 8 * (qt & 1);
     t[u] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) v4bf*)p);
   }
-  return __builtin_shufflevector(t[0], t[1], 0, 1, 2, 3, 4, 5, 6, 7);
+  const v8bf m = __builtin_shufflevector(t[0], t[1], 0, 1, 2, 3, 4, 5, 6, 7);
+  if (kind == 1) return m;
+  const v4u d = *stored, mu = __builtin_bit_cast(v4u, m);
+  return as_v8bf(q >> 1 ? d : mu);
 }
+// kind of output atom aj (< NA) and chunk c
+__device__ __forceinline__ int ty_kind(int aj, int c) { return aj <= 2 * c ? 0 : aj > 2 * c + 1 ? 1 : 2; }
 
 __device__ __forceinline__ v8bf neg_bf16(v8bf x) {
   return __builtin_bit_cast(v8bf, __builtin_bit_cast(v4u, x) ^ (v4u){0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u});
@@ -1320,8 +1329,8 @@ __global__ void __launch_bounds__(TY_THREADS) taylor_bf16_kernel(TaylorBf16Args 
       const uint4* Bq = stage + T::SUB_A;
       // this wave's output atom aj against K atom ak of its lane group: stored or mirror
       const int c = t * T::KS + sc, bslot = wave * 2 + (q >> 1);
-      const int aj = 5 * cb + wave, ak = 2 * c + (q >> 1);
-      const bool mirror = aj > ak && aj < NA;
+      const int aj = 5 * cb + wave;
+      const int mirror = __builtin_amdgcn_readfirstlane(aj < NA ? ty_kind(aj, c) : 0);
       // operands swapped in every MFMA: the accumulators hold the transposed tiles
       if (SPLIT) {
         const v8bf brh = ty_bfrag(Bq, (bslot * T::NP + 0) * 32, l16, q, mirror);
@@ -1524,6 +1533,226 @@ __global__ void __launch_bounds__(TY_THREADS) taylor16_kernel(TaylorBf16Args a) 
     }
   }
   ty_epilogue(a, re, im, w, rb, cb, wave, l16, g);
+}
+
+// The whole series in one launch, for N <= 256: a workgroup takes one walker and 32 of
+// its columns, keeps the planes of out_k^T for them in LDS, and reads only VHS atoms
+// between the first term and the last.  Wave v owns the output atoms v, v + waves, ..
+// (at most U); VHS is held in LDS whole (HELD), or each wave stages the two atoms of a K
+// chunk for itself (two 4 KB stages a wave); the waves of a term run without
+// barriers.  The same products in the same order as a launch per term.  Between terms the
+// planes of out_k^T replace those of out_{k-1}^T; the sum of the terms (hi + lo of all
+// but the last, in FP64) stays in registers.
+// What bounds it: HELD, the latency of a chunk (LDS reads, then 24 or 8 MFMAs, three waves a
+// SIMD) and the conversions between terms; staged, the latency of the next chunk's
+// atoms.  Against a launch per term, which moves every term's planes through memory and
+// reads all of them again in the last (us, 6 terms, n columns):
+//   N = 24, W = 10, n = 10      31 -> 14      N = 160, W = 700, n = 48    439 -> 276
+//   N = 101, W = 137, n = 19    80 -> 32      N = 200, W = 512, n = 40    472 -> 376
+//   N = 150, W = 300, n = 30   182 -> 90      N = 250, W = 1000, n = 30  1172 -> 483
+//   N = 150, W = 1000, n = 30  498 -> 205     N = 180, W = 300, n = 70    355 -> 312
+constexpr int TS_R = 32;  // columns of a group (rows of the planes)
+constexpr int TS_WAVES = 10;
+template <int U, bool HELD>
+__global__ void __launch_bounds__(64 * (HELD ? TS_WAVES : 8), HELD ? 3 : 2)
+    taylor_bf16_series_kernel(TaylorBf16Args a) {
+  extern __shared__ uint4 lds_u4[];
+  const int N = a.nbasis, Kp = a.kpad, S = Kp / 8, NA = a.natom_side, nch = Kp / BX_KC;
+  const int groups = (int)ceil_div(a.ncol, TS_R);
+  const int lin = xcd_remap(blockIdx.x, gridDim.x);
+  const int cg = lin % groups, w = lin / groups;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+  const int64_t tplane = (int64_t)a.wcap * a.rpad * Kp;
+  const int row0 = cg * TS_R;
+  const bool both = row0 + 16 < a.ncol;  // the group's second 16 columns exist
+  // 16-byte vector s of row r: the vectors of 8 rows read together lie in 8 slots modulo 8
+  const int sh = S % 8 == 0 ? 0 : 1, mask = S % 8 == 0 ? 7 : 3;
+  const auto slot = [&](int plane, int r, int v) { return (plane * TS_R + r) * S + (v ^ ((r >> sh) & mask)); };
+  for (int v = threadIdx.x; v < 4 * TS_R * S; v += blockDim.x) {
+    const int p = v / (TS_R * S), r = v / S % TS_R, x = v % S;
+    uint4 t = make_uint4(0, 0, 0, 0);
+    if (row0 + r < a.rpad)
+      t = *reinterpret_cast<const uint4*>(a.tin + p * tplane + ((int64_t)w * a.rpad + row0 + r) * Kp + 8 * x);
+    lds_u4[slot(p, r, x)] = t;
+  }
+  uint4* ring = lds_u4 + 4 * TS_R * S + (HELD ? 0 : wave * 512);
+  const uint16_t* wat = a.vatoms + (int64_t)w * a.atom_stride;
+  // atoms (aj, 2 c), (aj, 2 c + 1) or their mirrors into stage `buf`: NP of the planes each
+  const auto issue = [&](auto np, int aj, int c, int buf) __attribute__((always_inline)) {
+    constexpr int NP = decltype(np)::value;
+#pragma unroll
+    for (int j = 0; j < NP; ++j) {
+      const int sp = 2 * j + (lane >> 5), e = lane & 31, ar = e >> 1;  // sub-block (atom, plane), vector
+      const int ak = 2 * c + sp / NP, pi = NP == 4 ? sp % NP : 2 * (sp % NP);
+      const int lo = min(aj, ak), hi = max(aj, ak);
+      const int off = pi * 256 + ar * 16 + 8 * ((e & 1) ^ (((ar >> 2) ^ (ar >> 3)) & 1));
+      const uint16_t* src = hi >= NA ? a.zatom + off : wat + (int64_t)(lo * NA - lo * (lo - 1) / 2 + hi - lo) * 1024 + off;
+      __builtin_amdgcn_global_load_lds((const void*)src,
+                                       (__attribute__((address_space(3))) void*)(ring + buf * 256 + j * 64), 16, 0, 0);
+    }
+  };
+  if constexpr (HELD) {  // every atom, planes as in a stage
+    for (int b = wave; b < NA * (NA + 1); b += waves) {
+      const int e = lane & 31, ar = e >> 1, off = (lane >> 5) * 256 + ar * 16 + 8 * ((e & 1) ^ (((ar >> 2) ^ (ar >> 3)) & 1));
+      __builtin_amdgcn_global_load_lds((const void*)(wat + b * 512 + off),
+                                       (__attribute__((address_space(3))) void*)(ring + b * 64), 16, 0, 0);
+    }
+  }
+  double sre[U][2][4], sim[U][2][4];
+  v4f re[U][2], im[U][2];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sre[u][i][r] = sim[u][i][r] = 0.0;
+  int buf = 0;
+  const auto term = [&](auto np) __attribute__((always_inline)) {
+    constexpr int NP = decltype(np)::value;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) re[u][i] = im[u][i] = zero4f();
+      const int aj = wave + u * waves;
+      if (aj >= NA) continue;
+      const int after = aj + waves;
+      const bool more = u + 1 < U && after < NA;  // another atom follows
+#pragma unroll 1
+      for (int c = 0; c < nch; ++c) {
+        // the other stage's fragments were used a chunk ago
+        const int mirror = ty_kind(aj, c);
+        int vb, pstep = 32;  // this lane group's atom, its planes re_hi, re_lo, im_hi, im_lo (or re_hi, im_hi)
+        if constexpr (HELD) {
+          const auto at = [&](int ak) {  // (past the matrix: any atom, its K entries of the planes are zero)
+            ak = min(ak, NA - 1);
+            const int lo = min(aj, ak), hi = max(aj, ak);
+            return 128 * (lo * NA - lo * (lo - 1) / 2 + hi - lo);
+          };
+          const int a0 = at(2 * c), a1 = at(2 * c + 1);
+          vb = q >> 1 ? a1 : a0;
+          if (NP == 2) pstep = 64;
+        } else {
+          const bool next = c + 1 < nch || more;
+          if (next) {
+            issue(np, c + 1 < nch ? aj : after, c + 1 < nch ? c + 1 : 0, buf ^ 1);
+            wait_vm<NP>();
+          } else {
+            wait_vm<0>();
+          }
+          vb = buf * 256 + (q >> 1) * NP * 32;
+        }
+        const uint4* B = ring;
+        const v8bf brh = ty_bfrag(B, vb, l16, q, mirror);
+        const v8bf bih = ty_bfrag(B, vb + (NP == 4 ? 2 : 1) * pstep, l16, q, mirror);
+        v8bf brl, bil;
+        if constexpr (NP == 4) {
+          brl = ty_bfrag(B, vb + 32, l16, q, mirror);
+          bil = ty_bfrag(B, vb + 3 * 32, l16, q, mirror);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          if (i == 1 && !both) break;
+          const auto frag = [&](int p) {
+            return as_v8bf(reinterpret_cast<const v4u*>(lds_u4)[slot(p, i * 16 + l16, 4 * c + q)]);
+          };
+          const v8bf arh = frag(0), aih = frag(2), naih = neg_bf16(aih);
+          if constexpr (NP == 4) {
+            const v8bf arl = frag(1), ail = frag(3), nail = neg_bf16(ail);
+            re[u][i] = mfma_bf16(brh, arh, re[u][i]);
+            im[u][i] = mfma_bf16(bih, arh, im[u][i]);
+            re[u][i] = mfma_bf16(brl, arh, re[u][i]);
+            im[u][i] = mfma_bf16(bil, arh, im[u][i]);
+            re[u][i] = mfma_bf16(brh, arl, re[u][i]);
+            im[u][i] = mfma_bf16(bih, arl, im[u][i]);
+            re[u][i] = mfma_bf16(bih, naih, re[u][i]);
+            im[u][i] = mfma_bf16(brh, aih, im[u][i]);
+            re[u][i] = mfma_bf16(bil, naih, re[u][i]);
+            im[u][i] = mfma_bf16(brl, aih, im[u][i]);
+            re[u][i] = mfma_bf16(bih, nail, re[u][i]);
+            im[u][i] = mfma_bf16(brh, ail, im[u][i]);
+          } else {
+            re[u][i] = mfma_bf16(brh, arh, re[u][i]);
+            im[u][i] = mfma_bf16(bih, arh, im[u][i]);
+            re[u][i] = mfma_bf16(bih, naih, re[u][i]);
+            im[u][i] = mfma_bf16(brh, aih, im[u][i]);
+          }
+        }
+        if constexpr (!HELD) {
+          // this stage's reads are done before the next chunk's loads go into it
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          buf ^= 1;
+        }
+      }
+    }
+  };
+  using Split = std::integral_constant<int, 4>;
+  using Single = std::integral_constant<int, 2>;
+  if constexpr (HELD) wait_vm<0>();
+  else issue(Split{}, wave, 0, 0);
+  __syncthreads();
+#pragma unroll 1
+  for (int k = 1;; ++k) {
+    const bool split_next = k + 1 <= TAYLOR_SPLIT_TERMS;
+    if (k <= TAYLOR_SPLIT_TERMS) term(Split{});
+    else term(Single{});
+    const double alpha = 1.0 / k;
+    if (k == a.nterms) break;
+    // the next term's first atoms, in flight over the exchange of the planes
+    if constexpr (!HELD) {
+      if (split_next) issue(Split{}, wave, 0, buf);
+      else issue(Single{}, wave, 0, buf);
+    }
+    dl_barrier();  // every wave has read the term's planes
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int aj = wave + u * waves, kc0 = aj * 16 + 4 * q;
+      if (aj >= NA) continue;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        uint16_t h[4][4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const bool in = kc0 + r < N;
+          split_bf16(in ? alpha * re[u][i][r] : 0.0, h[0][r], h[1][r]);
+          split_bf16(in ? alpha * im[u][i][r] : 0.0, h[2][r], h[3][r]);
+          sre[u][i][r] += (double)bf2f(h[0][r]) + bf2f(h[1][r]);
+          sim[u][i][r] += (double)bf2f(h[2][r]) + bf2f(h[3][r]);
+        }
+#pragma unroll
+        for (int p = 0; p < 4; ++p)
+          if (split_next || p % 2 == 0)
+            *(reinterpret_cast<ushort4*>(lds_u4 + slot(p, i * 16 + l16, kc0 >> 3)) + ((kc0 >> 2) & 1)) =
+                make_ushort4(h[p][0], h[p][1], h[p][2], h[p][3]);
+      }
+    }
+    dl_barrier();
+  }
+  const double alpha = 1.0 / a.nterms;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int aj = wave + u * waves, kc0 = aj * 16 + 4 * q;
+    if (aj >= NA) continue;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int crow = row0 + i * 16 + l16;
+      if (crow >= a.ncol || kc0 >= N) continue;
+      uint16_t h[4][4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) h[p][r] = 0;
+        if (kc0 + r >= N) continue;
+        const int64_t qi = ((int64_t)w * N + kc0 + r) * a.ncol + crow;
+        const cplx v = cmake(alpha * re[u][i][r] + sre[u][i][r], alpha * im[u][i][r] + sim[u][i][r]);
+        const cplx qv = cadd(ld(a.init, qi), v);
+        st(a.q, qi, qv);
+        split_bf16(qv.re, h[0][r], h[1][r]);
+        split_bf16(qv.im, h[2][r], h[3][r]);
+      }
+      if (a.qout) store_planes_ty(a.qout, tplane, ((int64_t)w * a.rpad + crow) * Kp + kc0, h, N - kc0);
+    }
+  }
 }
 
 // phi [W][N][ncol] complex -> transposed split planes [4][W][rpad][kpad] at
@@ -1759,6 +1988,41 @@ hipError_t launch_taylor_bf16(const TaylorBf16Args& a, hipStream_t stream) {
     hipLaunchKernelGGL(taylor_bf16_kernel<true>, dim3((unsigned)grid), dim3(TY_THREADS), lds, stream, a);
   else
     hipLaunchKernelGGL(taylor_bf16_kernel<false>, dim3((unsigned)grid), dim3(TY_THREADS), lds, stream, a);
+  return hipGetLastError();
+}
+
+// The one-launch series: VHS held in LDS (one atom a wave) while it fits beside the
+// planes, N <= 160, else staged with two atoms a wave, N <= 256.  Four atoms a wave (N <= 416)
+// spill, one workgroup a CU: N = 300, 200 walkers 591 us where a launch per term takes
+// 412, N = 400, 1024 walkers 4300 against 2870.
+static size_t taylor_series_lds(int nbasis, int kpad, bool held) {
+  const int64_t NA = vhs_atom_side(nbasis);
+  return 16 * (size_t)(4 * TS_R * (kpad / 8) + (held ? 64 * NA * (NA + 1) : 512 * ceil_div(NA, 2)));
+}
+static bool taylor_series_held(int nbasis, int kpad) {
+  return vhs_atom_side(nbasis) <= TS_WAVES && taylor_series_lds(nbasis, kpad, true) <= 163840;
+}
+
+bool taylor_bf16_in_one(int nbasis, int kpad) {
+  return taylor_series_held(nbasis, kpad) ||
+         (vhs_atom_side(nbasis) <= 16 && taylor_series_lds(nbasis, kpad, false) <= 163840);
+}
+
+hipError_t launch_taylor_bf16_series(const TaylorBf16Args& a, hipStream_t stream) {
+  if (a.nwalkers < 1 || a.wcap < a.nwalkers || a.ncol < 1 || a.rpad < a.ncol || a.rpad % 16 != 0 ||
+      a.kpad % BX_KC != 0 || a.kpad < a.nbasis || !a.tin || !a.init || !a.q || !a.vatoms || !a.zatom ||
+      a.natom_side != vhs_atom_side(a.nbasis) || a.atom_stride < vhs_atom_count(a.nbasis) * 1024 || a.nterms < 1 ||
+      !taylor_bf16_in_one(a.nbasis, a.kpad))
+    return hipErrorInvalidValue;
+  const bool held = taylor_series_held(a.nbasis, a.kpad);
+  const size_t lds = taylor_series_lds(a.nbasis, a.kpad, held);
+  const void* kern = held ? (const void*)taylor_bf16_series_kernel<1, true> : (const void*)taylor_bf16_series_kernel<2, false>;
+  hipError_t e = allow_lds(kern, lds);
+  if (e != hipSuccess) return e;
+  const dim3 grid((unsigned)(a.nwalkers * ceil_div(a.ncol, TS_R)));
+  const dim3 block((unsigned)(64 * ceil_div(a.natom_side, held ? 1 : 2)));
+  if (held) hipLaunchKernelGGL((taylor_bf16_series_kernel<1, true>), grid, block, lds, stream, a);
+  else hipLaunchKernelGGL((taylor_bf16_series_kernel<2, false>), grid, block, lds, stream, a);
   return hipGetLastError();
 }
 

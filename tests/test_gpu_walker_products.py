@@ -27,7 +27,7 @@ CASES = [
 ]
 
 
-def _context(N, na, nb, W, terms, seed, rhf=False):
+def _context(N, na, nb, W, terms, seed, rhf=False, precision="fp64"):
     import torch
 
     from ipie_amd import _lib
@@ -40,7 +40,7 @@ def _context(N, na, nb, W, terms, seed, rhf=False):
     packed = torch.from_numpy(chol[numpy.triu_indices(N)].reshape(-1, 1).copy()).to(dev)
     exp = rs.normal(size=(2, N, N))
     z = lambda *s: torch.zeros(*s, dtype=c128, device=dev)
-    ctx = _lib.Context(N, 1, na, nb, W, exp_nmax=terms, rhf=rhf, device=dev)
+    ctx = _lib.Context(N, 1, na, nb, W, exp_nmax=terms, rhf=rhf, device=dev, precision=precision)
     ctx.set_static(chol_packed=packed, rchola=torch.zeros(1, na * N, dtype=f64, device=dev),
                    rcholb=torch.zeros(1, nb * N, dtype=f64, device=dev), rH1a=z(na, N), rH1b=z(nb, N),
                    expH1=torch.from_numpy(exp).to(dev), mf_shift=z(1), psia=z(N, na), psib=z(N, nb), dt=0.04, ecore=0.0)
