@@ -13,7 +13,34 @@ namespace afqmc {
 
 namespace {
 
-constexpr int FLD_THREADS = 256;
+// Sums of v[0 .. S) and maxima of v[S .. S + M) over the workgroup's T threads, in thread 0:
+// every value's steps side by side, one barrier.
+template <int T, int S, int M>
+__device__ __forceinline__ void reduce_all(double (&v)[S + M]) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < S + M; ++i) {
+      const double o = __shfl_xor(v[i], off, 64);
+      v[i] = i < S ? v[i] + o : fmax(v[i], o);
+    }
+  if (T == 64) return;
+  __shared__ double waves[T / 64][S + M];
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int i = 0; i < S + M; ++i) waves[threadIdx.x >> 6][i] = v[i];
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int t = 1; t < T / 64; ++t)
+#pragma unroll
+      for (int i = 0; i < S + M; ++i) v[i] = i < S ? v[i] + waves[t][i] : fmax(v[i], waves[t][i]);
+}
+
+// Threads of a walker's workgroup for `items` items: a wave for at most 64, else 256, or
+// more for at most `few` walkers, which leave CUs idle.
+int walker_threads(int nwalkers, int64_t items, int few, int more) {
+  return items <= 64 ? 64 : items > 256 && nwalkers <= few ? more : 256;
+}
 
 // Two standard normals (Philox key = seed, counter = (pair index, stream)) for pair index p of stream `counter`.
 __device__ __forceinline__ double2 normal_pair(uint64_t seed, uint64_t counter, uint64_t p) {
@@ -30,87 +57,90 @@ __device__ __forceinline__ double2 normal_pair(uint64_t seed, uint64_t counter, 
   return make_double2(rad * co, rad * s);
 }
 
-__device__ __forceinline__ double draw_normal(uint64_t seed, uint64_t counter, uint64_t idx) {
-  const double2 v = normal_pair(seed, counter, idx >> 1);
-  return (idx & 1) ? v.y : v.x;
-}
-
-__global__ void __launch_bounds__(FLD_THREADS) fields_kernel(FieldsArgs a) {
+// A thread takes the pairs of entries that share a Philox draw (entries 2 p, 2 p + 1 of the
+// [W, X] array; a pair may end in the next walker).  Latency-bound: the partial sums of
+// 4 ranges are loaded together, the walker's sums reduced together.  (W, X, ranges)
+// = (10, 72, 5): 7.8 -> 5.0 us; (12, 2400, 16): 46 -> 15; (300, 750, 16 in FP32): 23 -> 13;
+// (1024, 2400, 16 in FP32): 117 -> 96, against one entry a thread, each range's load waited for,
+// and six reductions of two barriers.
+template <int T>
+__global__ void __launch_bounds__(T) fields_kernel(FieldsArgs a) {
   phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
-  __shared__ double red[FLD_THREADS / 64];
   const int w = blockIdx.x;
   const int X = a.nchol;
-  const int64_t plane = (int64_t)a.nwalkers * X;
-  double cmf_r = 0, cmf_i = 0, cfb_r = 0, cfb_i = 0, ec_r = 0, ec_i = 0;
-  double xb_sum = 0.0, xb_max = 0.0;
+  const int64_t plane = (int64_t)a.nwalkers * X, first = (int64_t)w * X, end = first + X;
+  // ecoul re, im, cmf re, im, cfb re, im, sum |xbar|; max |xbar|
+  double sums[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   unsigned long long ncap = 0;
   const uint64_t counter = a.state ? a.state->counter : a.counter;
-  for (int x = threadIdx.x; x < X; x += FLD_THREADS) {
-    const int64_t idx = (int64_t)w * X + x;
-    cplx vb;
-    if (a.part32) {  // split-BF16 partials, FP32 (their accumulation precision), summed in FP64
-      const float2* p32 = reinterpret_cast<const float2*>(a.vbias_part);
-      vb = cmake(0.0, 0.0);
-      for (int z = 0; z < a.ksplit; ++z) {
-        const float2 v = p32[z * plane + idx];
-        vb = cadd(vb, cmake((double)v.x, (double)v.y));
+  for (int64_t p = (first >> 1) + threadIdx.x; 2 * p < end; p += T) {
+    const int64_t i0 = max(2 * p, first), i1 = min(2 * p + 1, end - 1);  // (i0 == i1: one of them is the neighbour's)
+    cplx vb[2] = {cmake(0.0, 0.0), cmake(0.0, 0.0)};
+    for (int z0 = 0; z0 < a.ksplit; z0 += 4) {
+      cplx v[4][2];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t at = min(z0 + u, a.ksplit - 1) * plane;
+        if (a.part32) {  // split-BF16 partials, FP32 (their accumulation precision), summed in FP64
+          const float2* p32 = reinterpret_cast<const float2*>(a.vbias_part) + at;
+          const float2 f0 = p32[i0], f1 = p32[i1];
+          v[u][0] = cmake((double)f0.x, (double)f0.y);
+          v[u][1] = cmake((double)f1.x, (double)f1.y);
+        } else {
+          v[u][0] = ld(a.vbias_part, at + i0);
+          v[u][1] = ld(a.vbias_part, at + i1);
+        }
       }
-    } else {
-      vb = ld(a.vbias_part, idx);
-      for (int z = 1; z < a.ksplit; ++z) vb = cadd(vb, ld(a.vbias_part, z * plane + idx));
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (z0 + u < a.ksplit) {
+          vb[0] = cadd(vb[0], v[u][0]);
+          vb[1] = cadd(vb[1], v[u][1]);
+        }
     }
-    if (a.vbias_out) st(a.vbias_out, idx, vb);
-    ec_r += vb.re * vb.re - vb.im * vb.im;
-    ec_i += 2.0 * vb.re * vb.im;
-    const cplx mf = ld(a.mf_shift, x);
-    // xbar = -sqrt(dt) (i vbias - mf_shift)
-    cplx xb = cmake(a.sqrt_dt * (mf.re + vb.im), a.sqrt_dt * (mf.im - vb.re));
-    const double axb = cabs(xb);
-    if (axb > a.fbbound) {
-      ++ncap;
-      if (axb > 1e-13) xb = cmake(xb.re / axb, xb.im / axb);
-    }
-    const double axc = axb > a.fbbound ? 1.0 : axb;
-    xb_sum += axc;
-    xb_max = fmax(xb_max, axc);
-    if (!a.want_fields) continue;
-    const double xi = a.xi ? a.xi[idx] : draw_normal(a.seed, counter, (uint64_t)idx);
-    if (a.xi_out) a.xi_out[idx] = xi;
-    const cplx xs = cmake(xi - xb.re, -xb.im);
-    st(a.xshifted, idx, xs);
-    cmf_r += xs.re * mf.re - xs.im * mf.im;
-    cmf_i += xs.re * mf.im + xs.im * mf.re;
-    cfb_r += xi * xb.re - 0.5 * (xb.re * xb.re - xb.im * xb.im);
-    cfb_i += xi * xb.im - xb.re * xb.im;
-  }
-  ec_r = block_sum(ec_r, red);
-  ec_i = block_sum(ec_i, red);
-  if (a.xbar_mean) {
-    xb_sum = block_sum(xb_sum, red);
-    // block max: wave shuffles then the per-wave maxima in order
-    for (int off = 32; off > 0; off >>= 1) xb_max = fmax(xb_max, __shfl_xor(xb_max, off, 64));
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = xb_max;
-    __syncthreads();
-    double m = 0.0;
-    for (int i = 0; i < FLD_THREADS / 64; ++i) m = fmax(m, red[i]);
-    if (threadIdx.x == 0) {
-      a.xbar_mean[w] = xb_sum / X;
-      a.xbar_max[w] = m;
+    double2 normal = make_double2(0.0, 0.0);
+    if (a.want_fields && !a.xi) normal = normal_pair(a.seed, counter, (uint64_t)p);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t idx = 2 * p + h;
+      if (idx < first || idx >= end) continue;
+      const cplx v = vb[h];
+      if (a.vbias_out) st(a.vbias_out, idx, v);
+      sums[0] += v.re * v.re - v.im * v.im;
+      sums[1] += 2.0 * v.re * v.im;
+      const cplx mf = ld(a.mf_shift, idx - first);
+      // xbar = -sqrt(dt) (i vbias - mf_shift)
+      cplx xb = cmake(a.sqrt_dt * (mf.re + v.im), a.sqrt_dt * (mf.im - v.re));
+      const double axb = cabs(xb);
+      if (axb > a.fbbound) {
+        ++ncap;
+        if (axb > 1e-13) xb = cmake(xb.re / axb, xb.im / axb);
+      }
+      const double axc = axb > a.fbbound ? 1.0 : axb;
+      sums[6] += axc;
+      sums[7] = fmax(sums[7], axc);
+      if (!a.want_fields) continue;
+      const double xi = a.xi ? a.xi[idx] : h ? normal.y : normal.x;
+      if (a.xi_out) a.xi_out[idx] = xi;
+      const cplx xs = cmake(xi - xb.re, -xb.im);
+      st(a.xshifted, idx, xs);
+      sums[2] += xs.re * mf.re - xs.im * mf.im;
+      sums[3] += xs.re * mf.im + xs.im * mf.re;
+      sums[4] += xi * xb.re - 0.5 * (xb.re * xb.re - xb.im * xb.im);
+      sums[5] += xi * xb.im - xb.re * xb.im;
     }
   }
-  if (a.want_fields) {
-    cmf_r = block_sum(cmf_r, red);
-    cmf_i = block_sum(cmf_i, red);
-    cfb_r = block_sum(cfb_r, red);
-    cfb_i = block_sum(cfb_i, red);
-    if (ncap && a.nfb) atomicAdd(a.nfb, ncap);
-  }
+  if (a.want_fields && ncap && a.nfb) atomicAdd(a.nfb, ncap);
+  reduce_all<T, 7, 1>(sums);
   if (threadIdx.x == 0) {
-    if (a.ecoul) st(a.ecoul, w, cmake(0.5 * ec_r, 0.5 * ec_i));
+    if (a.xbar_mean) {
+      a.xbar_mean[w] = sums[6] / X;
+      a.xbar_max[w] = sums[7];
+    }
+    if (a.ecoul) st(a.ecoul, w, cmake(0.5 * sums[0], 0.5 * sums[1]));
     if (a.want_fields) {
-      st(a.cmf, w, cmake(-a.sqrt_dt * cmf_r, -a.sqrt_dt * cmf_i));
-      st(a.cfb, w, cmake(cfb_r, cfb_i));
+      st(a.cmf, w, cmake(-a.sqrt_dt * sums[2], -a.sqrt_dt * sums[3]));
+      st(a.cfb, w, cmake(sums[4], sums[5]));
     }
   }
 }
@@ -145,25 +175,39 @@ __global__ void update_weight_kernel(WeightArgs a) {
   phase_mark(PhaseMark{a.mark.acc, a.mark.phase, -1}, w == 0);
 }
 
-__global__ void __launch_bounds__(FLD_THREADS) energy_kernel(EnergyArgs a) {
+// (Four entries of both operands in flight a thread, four partial sums.)
+template <int T>
+__global__ void __launch_bounds__(T) energy_kernel(EnergyArgs a) {
   phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
-  __shared__ double red[FLD_THREADS / 64];
   const int w = blockIdx.x;
   const int N = a.nbasis;
-  double er = 0.0, ei = 0.0;
+  double sums[2] = {0.0, 0.0};
   const int nspin = a.e1_in ? 0 : (a.rhf || a.nbeta == 0) ? 1 : 2;
   for (int s = 0; s < nspin; ++s) {
-    const int n = s == 0 ? a.nalpha : a.nbeta;
+    const int n = s == 0 ? a.nalpha : a.nbeta, end = n * N;
     const double* g = (s == 0 ? a.ghalfa : a.ghalfb) + 2 * (int64_t)w * n * N;
     const double* h = s == 0 ? a.rH1a : a.rH1b;
-    for (int e = threadIdx.x; e < n * N; e += FLD_THREADS) {
-      const cplx gv = ld(g, e), hv = ld(h, e);
-      er += gv.re * hv.re - gv.im * hv.im;
-      ei += gv.re * hv.im + gv.im * hv.re;
+    double er[4] = {0.0, 0.0, 0.0, 0.0}, ei[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int e0 = threadIdx.x; e0 < end; e0 += 4 * T) {
+      cplx gv[4], hv[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int e = min(e0 + u * T, end - 1);
+        gv[u] = ld(g, e);
+        hv[u] = ld(h, e);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (e0 + u * T < end) {
+          er[u] += gv[u].re * hv[u].re - gv[u].im * hv[u].im;
+          ei[u] += gv[u].re * hv[u].im + gv[u].im * hv[u].re;
+        }
     }
+    sums[0] += (er[0] + er[1]) + (er[2] + er[3]);
+    sums[1] += (ei[0] + ei[1]) + (ei[2] + ei[3]);
   }
-  er = block_sum(er, red);
-  ei = block_sum(ei, red);
+  reduce_all<T, 2, 0>(sums);
+  const double er = sums[0], ei = sums[1];
   if (threadIdx.x == 0) {
     const double f = a.rhf ? 2.0 : 1.0;
     const cplx e1 = a.e1_in ? ld(a.e1_in, w) : cmake(f * er + a.ecore, f * ei);
@@ -217,7 +261,11 @@ __global__ void normals_kernel(double* out, int64_t n, uint64_t seed, uint64_t c
 }  // namespace
 
 hipError_t launch_fields(const FieldsArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL(fields_kernel, dim3(a.nwalkers), dim3(FLD_THREADS), 0, stream, a);
+  switch (walker_threads(a.nwalkers, a.nchol / 2 + 1, 256, 512)) {  // (129 registers: one workgroup of 512 a CU)
+    case 64: hipLaunchKernelGGL(fields_kernel<64>, dim3(a.nwalkers), dim3(64), 0, stream, a); break;
+    case 256: hipLaunchKernelGGL(fields_kernel<256>, dim3(a.nwalkers), dim3(256), 0, stream, a); break;
+    default: hipLaunchKernelGGL(fields_kernel<512>, dim3(a.nwalkers), dim3(512), 0, stream, a);
+  }
   return hipGetLastError();
 }
 
@@ -227,7 +275,12 @@ hipError_t launch_update_weight(const WeightArgs& a, hipStream_t stream) {
 }
 
 hipError_t launch_energy(const EnergyArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL(energy_kernel, dim3(a.nwalkers), dim3(FLD_THREADS), 0, stream, a);
+  const int nmax = a.nalpha > a.nbeta ? a.nalpha : a.nbeta;
+  switch (walker_threads(a.nwalkers, a.e1_in ? 1 : ceil_div((int64_t)nmax * a.nbasis, 4), 512, 1024)) {
+    case 64: hipLaunchKernelGGL(energy_kernel<64>, dim3(a.nwalkers), dim3(64), 0, stream, a); break;
+    case 256: hipLaunchKernelGGL(energy_kernel<256>, dim3(a.nwalkers), dim3(256), 0, stream, a); break;
+    default: hipLaunchKernelGGL(energy_kernel<1024>, dim3(a.nwalkers), dim3(1024), 0, stream, a);
+  }
   return hipGetLastError();
 }
 
