@@ -60,8 +60,8 @@ __device__ __forceinline__ double2 normal_pair(uint64_t seed, uint64_t counter, 
 // A thread takes the pairs of entries that share a Philox draw (entries 2 p, 2 p + 1 of the
 // [W, X] array; a pair may end in the next walker).  Latency-bound: the partial sums of
 // 4 ranges are loaded together, the walker's sums reduced together.  (W, X, ranges)
-// = (10, 72, 5): 7.8 -> 5.0 us; (12, 2400, 16): 46 -> 15; (300, 750, 16 in FP32): 23 -> 13;
-// (1024, 2400, 16 in FP32): 117 -> 96, against one entry a thread, each range's load waited for,
+// = (10, 72, 5): 7.8 -> 5.0 us; (12, 2400, 16): 46 -> 16; (300, 750, 16 in FP32): 23 -> 18;
+// (1024, 2400, 16 in FP32): 117 -> 89, against one entry a thread, each range's load waited for,
 // and six reductions of two barriers.
 template <int T>
 __global__ void __launch_bounds__(T) fields_kernel(FieldsArgs a) {

@@ -30,6 +30,8 @@
 #include <algorithm>
 #include <cmath>
 
+#include <queue>
+
 #include "afqmc_internal.hpp"
 
 namespace afqmc {
@@ -354,26 +356,48 @@ int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, int most) {
 int nt64_quad_units(int64_t m, int64_t n, std::vector<int4>& units) {
   const int64_t kchunks = ceil_div(n, NT_KC), tiles = ceil_div(n, NT_TN);
   auto extent = [&](int64_t t) { return std::min<int64_t>((t + 1) * (NT_TN / NT_KC), kchunks); };
-  auto count = [&](int T) {
-    int64_t u = 0;
-    for (int64_t t = 0; t < tiles; ++t) u += ceil_div(extent(t), T);
-    return u;
+  auto list = [&](int T, std::vector<int4>& u) {
+    u.clear();
+    for (int64_t z = 0; z * T < kchunks; ++z)
+      for (int64_t t = 0; t < tiles; ++t)
+        if (z * T < extent(t))
+          u.push_back(make_int4((int)t, (int)(z * T), (int)std::min<int64_t>((z + 1) * T, extent(t)), 0));
+  };
+  // When the last workgroup ends, in chunks, with the units handed in their order to the
+  // first free of 512 places (two a CU): a unit shorter than T fills a round's end.
+  // (N = 200, 512 walkers: T = 24 in 3 rounds 685 us, 32 in 2.25 755; N = 300, 512
+  // walkers: 48 2600, 32 2670; N = 101, 137 walkers: 12 41, 16 46.)  Many rounds end
+  // together whatever T.
+  auto cost = [&](int T, const std::vector<int4>& u) {
+    const double each = T + NT_QDOT_CHUNKS;
+    const int rm = nt_rows(m, (int64_t)u.size(), each, 4);
+    const int64_t rows = ceil_div(m, 16 * rm);
+    if (rows * (int64_t)u.size() > 8192) return nt_cost(m, (int64_t)u.size(), rm, each);
+    std::priority_queue<double, std::vector<double>, std::greater<double>> free;
+    for (int i = 0; i < 512; ++i) free.push(0.0);
+    double end = 0.0;
+    for (const int4& e : u)
+      for (int64_t r = 0; r < rows; ++r) {
+        const double t = free.top() + (e.z - e.y) + NT_QDOT_CHUNKS;
+        free.pop();
+        free.push(t);
+        end = std::max(end, t);
+      }
+    return 2.0 * end * (rm + 0.25);
   };
   int best = 0;
   double least = 0.0;
-  for (int T = 64; T >= 4; T /= 2) {
-    const double each = T + NT_QDOT_CHUNKS;
-    const double cost = nt_cost(m, count(T), nt_rows(m, count(T), each, 4), each);
-    if (best == 0 || cost < 0.98 * least) {
+  std::vector<int4> u;
+  // (a tile's own columns are 8 chunks: other lengths leave short units)
+  for (int T : {64, 56, 48, 40, 32, 24, 16, 12, 8, 4}) {
+    list(T, u);
+    const double t = cost(T, u);
+    if (best == 0 || t < 0.98 * least) {
       best = T;
-      least = cost;
+      least = t;
     }
   }
-  units.clear();
-  for (int64_t z = 0; z * best < kchunks; ++z)
-    for (int64_t t = 0; t < tiles; ++t)
-      if (z * best < extent(t))
-        units.push_back(make_int4((int)t, (int)(z * best), (int)std::min<int64_t>((z + 1) * best, extent(t)), 0));
+  list(best, units);
   return best;
 }
 
