@@ -269,21 +269,26 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
   }
 }
 
+// What a chunk costs beside its products, in 16-row tiles: the B columns each row tile
+// reads again, with 16-byte loads, and with 4-byte ones four times the load instructions
+// (N = 255, 71 walkers, VHS of 1275 vectors: 48 rows 263 us, 16 rows 308).
+constexpr double NT_OVER = 0.25, NT_OVER_B4 = 0.75;
+
 // Cost of a launch in units of one 16-row tile's MFMA time per K chunk (1024
 // cycles): the workgroups of the fullest CU (a fraction of one once there are
 // many rounds), each its chunks and about two chunks' worth of start and
-// epilogue, a quarter of a tile per chunk for the B columns each row tile reads again.
-double nt_cost(int64_t m, int64_t colblocks, int rm, double chunks) {
+// epilogue, `over` of a tile per chunk.
+double nt_cost(int64_t m, int64_t colblocks, int rm, double chunks, double over = NT_OVER) {
   const double rounds = (double)(ceil_div(m, 16 * rm) * colblocks) / 256.0;
-  return (rounds < 4.0 ? std::ceil(rounds) : rounds) * (chunks + 2.0) * (rm + 0.25);
+  return (rounds < 4.0 ? std::ceil(rounds) : rounds) * (chunks + 2.0) * (rm + over);
 }
 
 // Rows per workgroup tile, in 16s (1 .. most): the least padding of m on a full
 // GPU; smaller tiles where larger ones would leave CUs idle.
-int nt_rows(int64_t m, int64_t colblocks, double chunks, int most) {
+int nt_rows(int64_t m, int64_t colblocks, double chunks, int most, double over = NT_OVER) {
   int best = 1;
   for (int rm = 2; rm <= most; ++rm)
-    if (nt_cost(m, colblocks, rm, chunks) < 0.999 * nt_cost(m, colblocks, best, chunks)) best = rm;
+    if (nt_cost(m, colblocks, rm, chunks, over) < 0.999 * nt_cost(m, colblocks, best, chunks, over)) best = rm;
   return best;
 }
 
@@ -326,7 +331,7 @@ hipError_t launch_nt(const NtArgs& a, hipStream_t stream) {
   const int64_t colblocks = EPI == NT_EPI_QDOT ? a.nunits : ceil_div(a.n, NT_TN) * a.ksplit;
   const double each = EPI == NT_EPI_QDOT ? a.unit_chunks + NT_QDOT_CHUNKS : (double)chunks / a.ksplit;
   // (the 4-byte loads' addresses and 64 rows do not fit the registers together)
-  switch (nt_rows(a.m, colblocks, each, b_vec ? 4 : 3)) {
+  switch (nt_rows(a.m, colblocks, each, b_vec ? 4 : 3, b_vec ? NT_OVER : NT_OVER_B4)) {
     case 1: return launch_nt_rm<1, EPI>(a, b_vec, stream);
     case 2: return launch_nt_rm<2, EPI>(a, b_vec, stream);
     case 3: return launch_nt_rm<3, EPI>(a, b_vec, stream);
