@@ -640,7 +640,7 @@ int one_body64(afqmc_ctx* c, int nw, const double* const phi[2], double* const p
   const int N = c->d.nbasis, nc = c->ncol, n[2] = {c->d.nalpha, c->d.nbeta};
   if (!c->exp_ready) {
     HIP_TRY(c, launch_pad_rows(c->s.expH1, 2 * N, N, exp_ld(c), c->exp_pad, c->stream));
-    c->exp_ready = true;
+    c->exp_ready = !c->capturing;  // (a recorded launch has not run yet)
   }
   OneBody64Args a{};
   a.mark = mark;

@@ -15,12 +15,13 @@
 //                         16 x 16 atoms of its upper triangle (VHS epilogue of
 //                         bf16_gemm_kernel), mirrors by transposing LDS loads
 //                         (ipie/propagation/operations.py:58-117)
+//   taylor_bf16_series_kernel  all terms in one launch (N <= 256)
 //
 // Operand planes are bf16 [rows, Kp] with Kp = K rounded up to 32 and zero
 // padding, so a 32-wide K chunk of a row is one aligned 64-byte segment:
 //   Ghalf: 4 planes (re_hi, re_lo, im_hi, im_lo), rows = (walker, j)
 //   rchol: 2 planes (hi, lo), rows = (x, i)
-// Exchange / GEMM workgroup: 8 waves in a 4 x 2 grid, each wave owns 2 x 5
+// Exchange / GEMM workgroup (shape 0): 8 waves in a 4 x 2 grid, each wave owns 2 x 5
 // output tiles of 16 x 16, so one workgroup covers 128 rows (wb walkers) by
 // 160 columns (xb Cholesky vectors); two waves share each SIMD, so one wave's
 // LDS and barrier waits are covered by the other's MFMAs.  Double-buffered LDS

@@ -30,8 +30,6 @@
 #include <algorithm>
 #include <cmath>
 
-#include <queue>
-
 #include "afqmc_internal.hpp"
 
 namespace afqmc {
@@ -378,17 +376,25 @@ int nt64_quad_units(int64_t m, int64_t n, std::vector<int4>& units) {
     const int rm = nt_rows(m, (int64_t)u.size(), each, 4);
     const int64_t rows = ceil_div(m, 16 * rm);
     if (rows * (int64_t)u.size() > 8192) return nt_cost(m, (int64_t)u.size(), rm, each);
-    std::priority_queue<double, std::vector<double>, std::greater<double>> free;
-    for (int i = 0; i < 512; ++i) free.push(0.0);
-    double end = 0.0;
-    for (const int4& e : u)
-      for (int64_t r = 0; r < rows; ++r) {
-        const double t = free.top() + (e.z - e.y) + NT_QDOT_CHUNKS;
-        free.pop();
-        free.push(t);
-        end = std::max(end, t);
+    // places that become free at each time, in chunks
+    const int start = (int)NT_QDOT_CHUNKS;
+    int64_t work = 0;
+    for (const int4& e : u) work += rows * (e.z - e.y + start);
+    std::vector<int> free((size_t)(work / 512 + 2 * (T + start) + 2), 0);
+    free[0] = 512;
+    size_t t = 0, end = 0;
+    for (const int4& e : u) {
+      const int d = e.z - e.y + start;
+      for (int64_t left = rows; left > 0;) {
+        while (free[t] == 0) ++t;
+        const int k = (int)std::min<int64_t>(free[t], left);
+        free[t] -= k;
+        free[t + d] += k;
+        left -= k;
+        end = std::max(end, t + d);
       }
-    return 2.0 * end * (rm + 0.25);
+    }
+    return 2.0 * (double)end * (rm + NT_OVER);
   };
   int best = 0;
   double least = 0.0;
