@@ -80,7 +80,7 @@ def exchange_flops_per_launch(N, X, n, W, form="t"):
     context uses: 't' forms every T_x = L_x Ghalf^T (ipie's contraction), 'quad'
     is Y = G Wq (complex G, real Wq of size (nN)^2) plus a dot per walker,
     'quad_sym' the same quadratic form over the (nN)(nN + 1) / 2 distinct
-    entries of the symmetric Wq (the block-triangular split-BF16 form)."""
+    entries of the symmetric Wq (the block-triangular W')."""
     if form == "quad":
         return float(W) * (4.0 * (n * N) ** 2 + 8.0 * n * N)
     if form == "quad_sym":
@@ -372,7 +372,7 @@ def run_graph(st, w, steps, one_step, counter, energy, eshift):
 
 
 def run_gpu(st, w, steps, warmup, graph=True):
-    """Warm-up, then `steps` eager steps timed with per-phase HIP events, then
+    """Warm-up, then `steps` eager steps timed per phase (device clock), then
     (graph=True) the same number of steps replayed from a step graph.  Returns
     (eager seconds, per-phase profile, eager per-step weighted energies, finite
     flag, graph result (seconds, energies, steps) or None)."""
@@ -497,7 +497,7 @@ def traffic_per_launch(mode, w):
 
 def phase_rooflines(mode, phases, w):
     """Algorithmic rate of the step's other large phases (ms per step from the
-    phase events of the eager pass; each phase is its kernels alone, launched
+    phase times of the eager pass; each phase is its kernels alone, launched
     back to back): flops as ipie performs them (step_flops) against the MFMA
     peak of the arithmetic the phase runs in, per algorithmic flop (split-BF16
     x3: a third of the BF16 peak; the Taylor series: three 3-product and three
@@ -507,16 +507,16 @@ def phase_rooflines(mode, phases, w):
     f64 = mode == "fp64"
     bf3 = PEAK["f64_mfma_tflops"] if f64 else PEAK["bf16_mfma_tflops"] / 3.0
     rows = [
-        ("vhs", "VHS, one launch per step (fp64: vhs_kernel; mixed: bf16_gemm_kernel<true, true, true> writing "
+        ("vhs", "VHS, one launch per step (fp64: nt64_kernel; mixed: bf16_gemm_kernel<true, true, true> writing "
                 "the split atoms)", 4.0 * X * N * (N + 1) / 2 * W, bf3),
-        ("taylor", "Taylor series, six terms (fp64: batched_nn_kernel; mixed: taylor_bf16_kernel, three 3-product "
+        ("taylor", "Taylor series, six terms (fp64: taylor64_kernel; mixed: taylor_bf16_kernel, three 3-product "
                    "and three 1-product terms)", 6 * 8.0 * N * N * nsum * W,
          PEAK["f64_mfma_tflops"] if f64 else PEAK["bf16_mfma_tflops"] / 2.0),
         ("one_body", "one body, two applications per step (mixed: bf16_gemm_kernel<true, true, true>, ADD epilogue, "
                      "and the transposed split of phi)", 2 * 8.0 * N * N * nsum * W, bf3),
         ("force_bias", "force bias (mixed: bf16_gemm_kernel<true, false, true>, split-K partials)",
          4.0 * X * N * nsum * W, bf3),
-        ("gf", "Green's function: O, LU with the inverse, Ghalf (FP64 MFMA and one wave per LU)",
+        ("gf", "Green's function: O, its inverse, Ghalf (FP64 MFMA and elimination, gf_kernel)",
          sum(12.0 * N * n * n + 11.0 * n**3 for n in (w.nalpha, w.nbeta)) * W, PEAK["f64_mfma_tflops"]),
     ]
     out = []
@@ -569,8 +569,8 @@ def run_modes(args, w, host, mode_list, K, warmup, tuner):
         log(f"[bench] {w.name} {mode}: done")
         ex_ms, ex_n = prof["exchange"]
         form = st["walkers"]._engine.ctx.exchange_form()
-        if form == "quad" and mode != "fp64":
-            form = "quad_sym"  # the split-BF16 planes hold the block-triangular Wq
+        if form == "quad":
+            form = "quad_sym"  # W' is block-triangular in FP64 and in split-BF16
         fl = 0.5 * (exchange_flops_per_launch(w.nbasis, w.nchol, w.nalpha, w.nwalkers, form)
                     + exchange_flops_per_launch(w.nbasis, w.nchol, w.nbeta, w.nwalkers, form))
         fl_t = 0.5 * (exchange_flops_per_launch(w.nbasis, w.nchol, w.nalpha, w.nwalkers, "t")
@@ -607,8 +607,9 @@ def run_modes(args, w, host, mode_list, K, warmup, tuner):
         if "surrogate" not in mode:
             rec["exchange_tflops"] = fl / ex_avg_s / 1e12
             rec["exchange_flops_per_launch"] = fl
-            if form == "quad":
-                kname = "Y = G Wq on FP64 MFMA (force_bias_kernel NT mainloop) + quad_reduce_kernel"
+            if form == "quad_sym" and mode == "fp64":
+                kname = ("Y = G W' over block-triangular W' on FP64 MFMA (nt64_kernel, g.Y in the epilogue) + "
+                         "quad_sum_kernel")
             elif form == "quad_sym":
                 kname = ("Y = G W' over block-triangular W' split-BF16 x3 (bf16_gemm_kernel<true, false, true>, g.Y "
                          "in the epilogue) + quad_sum_kernel")
@@ -824,10 +825,10 @@ def main():
             "traffic": traffic_per_launch(head, w),
             "avg_launch_ms": rk["avg_launch_ms"],
             "flops_per_launch": rk["flops_per_launch"],
-            "timing": "HIP events on the context's stream around each launch, over the eager pass of the same "
-                      "number of steps that precedes the step-graph replay (events cannot bracket kernels "
+            "timing": "device clock stamps at each phase's start and end, over the eager pass of the same "
+                      "number of steps that precedes the step-graph replay (phases are not stamped "
                       "inside a replayed graph)" if m.get("timed") == "step graph" else
-                      "HIP events on the context's stream around each launch, over the timed steps",
+                      "device clock stamps at each phase's start and end, over the timed steps",
             # the step's other large phases, each against its own MFMA peak (the
             # VHS GEMM is the largest single launch of the step)
             "other_phases": phase_rooflines(head, m["phases_ms_per_step"], w),
