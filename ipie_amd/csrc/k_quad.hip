@@ -22,8 +22,10 @@ namespace afqmc {
 
 namespace {
 
-constexpr int QW_T = 64;   // output tile edge
-constexpr int QW_XC = 16;  // Cholesky vectors staged per chunk
+constexpr int QW_T = 128;          // tile edge of G = R^T R
+constexpr int QW_XC = 16;          // Cholesky vectors per chunk
+constexpr int QW_LD = QW_T + 16;   // LDS row, doubles: the four rows of a K step 128 bytes apart in the banks
+constexpr size_t QW_LDS = 2 * 2 * 8 * (size_t)QW_XC * QW_LD;  // two stages of both operands
 
 __device__ __forceinline__ uint16_t qf2bf(float f) {
   uint32_t u = __float_as_uint(f);
@@ -32,80 +34,119 @@ __device__ __forceinline__ uint16_t qf2bf(float f) {
 }
 __device__ __forceinline__ float qbf2f(uint16_t h) { return __uint_as_float(((uint32_t)h) << 16); }
 
-// One 64 x 64 tile of W' for the orbital pair (i, j): rows a = (i, m'), columns
-// b = (j, m); out[a][b] = f sum_x R[x][j][m'] R[x][i][m].  Np is the column
-// stride per orbital of the output (N for FP64, Kp for the padded planes).  In
-// FP64 the tiles past their rows' column tile, which nothing reads, are skipped:
-// half the products.
-__global__ void __launch_bounds__(256) quad_w_kernel(const double* __restrict__ R, int X, int n, int N, int Np,
-                                                    double* __restrict__ w64, int64_t ld64,
-                                                    uint16_t* __restrict__ wplanes) {
-  __shared__ double fa[QW_XC][QW_T];  // R[x][j][m' range]
-  __shared__ double fb[QW_XC][QW_T];  // R[x][i][m range]
-  const int mblocks = (Np + QW_T - 1) / QW_T;
-  int blk = blockIdx.x;
-  const int mb = blk % mblocks;
-  blk /= mblocks;
-  const int ma = blk % mblocks;
-  blk /= mblocks;
-  const int j = blk % n, i = blk / n;
-  const int m0a = ma * QW_T, m0b = mb * QW_T;
-  if (w64 && ((int64_t)j * Np + m0b) / QUAD64_TILE > ((int64_t)i * Np + min(m0a + QW_T, N) - 1) / QUAD64_TILE) return;
-  const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-  double acc[4][4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int c = 0; c < 4; ++c) acc[r][c] = 0.0;
+// One 128 x 128 tile of G[P][Q] = sum_x R[x][P] R[x][Q], P = (j, p) and Q = (i, q) over the
+// n N columns of R; G is symmetric, and only the tiles P <= Q are computed.  G[P][Q]
+// is Wq[(i, p)][(j, q)] and, transposed, Wq[(j, q)][(i, p)]: each goes to its place in W'
+// where that is kept (b's column tile at most a's).  Np is the column stride per
+// orbital of the output (N for FP64, Kp for the padded planes, zero beforehand).
+// What bounds it: the matrix units (v_mfma_f64_16x16x4f64, four waves of 64 x 64); the
+// next chunk's loads are in flight under a chunk's products.  n N = 16000, 2400 vectors, per
+// spin: 64 x 64 tiles per orbital pair on the vector units, 188 GB through L2, took
+// 22.7 ms in FP64 and 44 ms as planes (every tile); now 12.0 and 11.7 ms (51 TFLOP/s).
+__global__ void __launch_bounds__(256, 2) quad_w_kernel(const double* __restrict__ R, int X, int n, int N, int Np,
+                                                       double* __restrict__ w64, int64_t ld64,
+                                                       uint16_t* __restrict__ wplanes) {
+  extern __shared__ double qw_lds[];
+  const int tp = blockIdx.x, tq = blockIdx.y;
+  if (tp > tq) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  const int wr = wave & 1, wc = wave >> 1;
   const int64_t nN = (int64_t)n * N;
-  for (int x0 = 0; x0 < X; x0 += QW_XC) {
-    __syncthreads();
-    for (int e = tid; e < QW_XC * QW_T; e += 256) {
-      const int xx = e / QW_T, k = e % QW_T, x = x0 + xx;
-      const int mpa = m0a + k, mpb = m0b + k;
-      fa[xx][k] = (x < X && mpa < N) ? R[x * nN + (int64_t)j * N + mpa] : 0.0;
-      fb[xx][k] = (x < X && mpb < N) ? R[x * nN + (int64_t)i * N + mpb] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int xx = 0; xx < QW_XC; ++xx) {
-      double av[4], bv[4];
+  // this thread loads columns col, col + 64 of rows row, row + 4, ..
+  const int row = threadIdx.x >> 6, col = lane;
+  double va[QW_XC / 4][2], vb[QW_XC / 4][2];
+  const auto fetch = [&](int x0) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) av[r] = fa[xx][ty * 4 + r];
+    for (int r = 0; r < QW_XC / 4; ++r) {
+      const int x = x0 + row + 4 * r;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) bv[c] = fb[xx][tx * 4 + c];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[r][c] += av[r] * bv[c];
-    }
-  }
-  const int64_t ldo = (int64_t)n * Np;  // row length of the output
-  const int64_t plane = ldo * ldo;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int mp = m0a + ty * 4 + r;  // m'
-    if (mp >= Np) continue;
-    const int64_t a = (int64_t)i * Np + mp;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int m = m0b + tx * 4 + c;
-      if (m >= Np) continue;
-      const int64_t b = (int64_t)j * Np + m;
-      if (w64) {
-        w64[a * ld64 + b] = (b / QUAD64_TILE < a / QUAD64_TILE ? 2.0 : 1.0) * acc[r][c];
-      } else {
-        // plane row a is the output column, b the K index: W'_{b a}
-        const int ta = (int)(a / QUAD_TILE), tb = (int)(b / QUAD_TILE);
-        const double f = tb < ta ? 2.0 : (tb == ta ? 1.0 : 0.0);
-        const double v = (mp < N && m < N) ? f * acc[r][c] : 0.0;
-        const uint16_t hi = qf2bf((float)v);
-        const uint16_t lo = qf2bf((float)(v - (double)qbf2f(hi)));
-        wplanes[a * ldo + b] = hi;
-        wplanes[plane + a * ldo + b] = lo;
+      for (int h = 0; h < 2; ++h) {
+        const int64_t P = (int64_t)tp * QW_T + col + 64 * h, Q = (int64_t)tq * QW_T + col + 64 * h;
+        va[r][h] = x < X && P < nN ? R[x * nN + P] : 0.0;
+        vb[r][h] = x < X && Q < nN ? R[x * nN + Q] : 0.0;
       }
     }
+  };
+  const auto stash = [&](int buf) {
+    double* a = qw_lds + buf * 2 * QW_XC * QW_LD;
+    double* b = a + QW_XC * QW_LD;
+#pragma unroll
+    for (int r = 0; r < QW_XC / 4; ++r)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        a[(row + 4 * r) * QW_LD + col + 64 * h] = va[r][h];
+        b[(row + 4 * r) * QW_LD + col + 64 * h] = vb[r][h];
+      }
+  };
+  v4d acc[4][4];
+#pragma unroll
+  for (int it = 0; it < 4; ++it)
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) acc[it][jt] = zero4d();
+  fetch(0);
+  stash(0);
+  __syncthreads();
+  int buf = 0;
+  for (int x0 = 0; x0 < X; x0 += QW_XC) {
+    const bool more = x0 + QW_XC < X;
+    if (more) fetch(x0 + QW_XC);
+    const double* a = qw_lds + buf * 2 * QW_XC * QW_LD + 64 * wr;
+    const double* b = qw_lds + buf * 2 * QW_XC * QW_LD + QW_XC * QW_LD + 64 * wc;
+#pragma unroll
+    for (int k = 0; k < QW_XC / 4; ++k) {
+      double fa[4], fb[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        fa[t] = a[(4 * k + kq) * QW_LD + 16 * t + r16];
+        fb[t] = b[(4 * k + kq) * QW_LD + 16 * t + r16];
+      }
+#pragma unroll
+      for (int it = 0; it < 4; ++it)
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) acc[it][jt] = mfma64(fa[it], fb[jt], acc[it][jt]);
+    }
+    if (more) stash(buf ^ 1);
+    __syncthreads();
+    buf ^= 1;
   }
+  const int64_t ldo = (int64_t)n * Np;  // row length of the planes
+  const int64_t plane = ldo * ldo;
+  const auto put = [&](uint32_t a, uint32_t b, double g) {
+    if (w64) {
+      const uint32_t ta = a / QUAD64_TILE, tb = b / QUAD64_TILE;
+      if (tb <= ta) w64[(int64_t)a * ld64 + b] = tb < ta ? 2.0 * g : g;
+    } else {
+      // plane row a is the output column, b the K index: W'_{b a}
+      const uint32_t ta = a / QUAD_TILE, tb = b / QUAD_TILE;
+      if (tb > ta) return;
+      const double v = tb < ta ? 2.0 * g : g;
+      const uint16_t hi = qf2bf((float)v);
+      wplanes[a * ldo + b] = hi;
+      wplanes[plane + a * ldo + b] = qf2bf((float)(v - (double)qbf2f(hi)));
+    }
+  };
+  const uint32_t cols = (uint32_t)nN, uN = (uint32_t)N;
+  uint32_t Q[4], oi[4], q[4];
+#pragma unroll
+  for (int jt = 0; jt < 4; ++jt) {
+    Q[jt] = tq * QW_T + 64 * wc + 16 * jt + r16;
+    oi[jt] = Q[jt] / uN * Np;
+    q[jt] = Q[jt] % uN;
+  }
+#pragma unroll
+  for (int it = 0; it < 4; ++it)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t P = tp * QW_T + 64 * wr + 16 * it + 4 * r + kq;
+      if (P >= cols) continue;
+      const uint32_t oj = P / uN * Np, pp = P % uN;
+#pragma unroll
+      for (int jt = 0; jt < 4; ++jt) {
+        if (Q[jt] >= cols) continue;
+        put(oi[jt] + pp, oj + q[jt], acc[it][jt][r]);
+        if (tp != tq) put(oj + q[jt], oi[jt] + pp, acc[it][jt][r]);
+      }
+    }
 }
 
 // out[w] = sum_s part[s][w]: WL walkers x 256 / WL slot lanes per workgroup, the
@@ -329,11 +370,19 @@ hipError_t launch_quad_sum(const double* part, int nslots, int nwalkers, double*
 
 hipError_t launch_quad_w(const double* rchol, int X, int n, int N, int Np, double* w64, int64_t ld64,
                          uint16_t* wplanes, hipStream_t stream) {
-  if ((w64 == nullptr) == (wplanes == nullptr) || Np < N) return hipErrorInvalidValue;
+  if ((w64 == nullptr) == (wplanes == nullptr) || Np < N || X < 1 || (int64_t)n * Np >= INT32_MAX)
+    return hipErrorInvalidValue;
   if (w64 && (Np != N || ld64 < (int64_t)n * N)) return hipErrorInvalidValue;
-  const int64_t mblocks = ceil_div(Np, QW_T);
-  const int64_t grid = (int64_t)n * n * mblocks * mblocks;
-  hipLaunchKernelGGL(quad_w_kernel, dim3((unsigned)grid), dim3(256), 0, stream, rchol, X, n, N, Np, w64, ld64,
+  if (wplanes) {  // the padding and what is past a row's column tile stay zero: [2][n Kp][n Kp] in doubles
+    const int64_t ldo = (int64_t)n * Np;
+    if (ldo % 2 != 0) return hipErrorInvalidValue;
+    const hipError_t e = launch_setup_fill(reinterpret_cast<double*>(wplanes), ldo * ldo / 2, 0.0, stream);
+    if (e != hipSuccess) return e;
+  }
+  const unsigned tiles = (unsigned)ceil_div((int64_t)n * N, QW_T);
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(quad_w_kernel), QW_LDS);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(quad_w_kernel, dim3(tiles, tiles), dim3(256), QW_LDS, stream, rchol, X, n, N, Np, w64, ld64,
                      wplanes);
   return hipGetLastError();
 }
