@@ -14,6 +14,7 @@ LIB = os.path.join(HERE, "libafqmc_hip.so")
 SOURCES = [
     "afqmc_api.hip",
     "k_greens.hip",
+    "k_greens_lu.hip",
     "k_gemm.hip",
     "k_nt64.hip",
     "k_exchange.hip",

@@ -100,6 +100,8 @@ struct afqmc_ctx {
   std::vector<void*> retired;         // buffers a retune replaced: graphs captured before still use them
   int64_t exx_cap = 0;      // capacity (complex entries) of each exchange partial buffer
   double* gcomp = nullptr;  // [W, nmax, N] complex: Ghalf of sampled walkers (FP64 exchange)
+  double* gf_o = nullptr;     // mixed: [W, 2, nmax, nmax] complex, overlap matrices
+  double* gf_oinv = nullptr;  // mixed: [W, 2, nmax, nmax] complex, their inverses
   // learned exchange control variate
   struct {
     bool enabled = false;
@@ -494,9 +496,17 @@ int do_gf(afqmc_ctx* c, int nw, const double* phia, const double* phib, double* 
     a.kpad = c->kpad;
     c->g_planes_nw = nw;
   }
+  // Ghalf that is rounded to BF16 next keeps its last bits (k_greens_lu.hip)
+  const bool lu = want_ghalf && c->d.precision == AFQMC_PREC_MIXED;
+  if (lu && !c->gf_oinv) {
+    const size_t bytes = gf_lu_work_bytes((int)c->d.nwalkers, c->d.nalpha, c->d.nbeta);
+    if ((!c->gf_o && dmalloc((void**)&c->gf_o, bytes) != hipSuccess) ||
+        dmalloc((void**)&c->gf_oinv, bytes) != hipSuccess)
+      return fail(c, AFQMC_ERR_ALLOC, "Green's function workspace allocation failed");
+  }
   PhaseScope ps(c, want_ghalf ? AFQMC_PHASE_GF : AFQMC_PHASE_OVERLAP, PhaseScope::KERNEL);
   a.mark = ps.mark();
-  HIP_TRY(c, launch_gf(a, want_ghalf, c->stream));
+  HIP_TRY(c, lu ? launch_gf_lu(a, c->gf_o, c->gf_oinv, c->stream) : launch_gf(a, want_ghalf, c->stream));
   return AFQMC_OK;
 }
 
@@ -1439,7 +1449,7 @@ void afqmc_destroy(afqmc_ctx* c) {
   else (void)hipDeviceSynchronize();
   void* ptrs[] = {c->vbias_part, c->xshifted, c->wvec, c->exx_a, c->exx_b, c->vhs, c->buf[0], c->buf[1],
                   c->buf[2], c->buf[3], c->exp_pad, c->qr_slow, c->flags, c->wflags, c->psi_flag, c->nfb, c->gplanes[0], c->gplanes[1], c->lplanes[0],
-                  c->lplanes[1], c->xplanes, c->cplanes, c->vatoms, c->zatom, c->dplanes, c->oplanes, c->gcomp, c->qw64[0], c->qw64[1], c->qwp[0],
+                  c->lplanes[1], c->xplanes, c->cplanes, c->vatoms, c->zatom, c->dplanes, c->oplanes, c->gcomp, c->gf_o, c->gf_oinv, c->qw64[0], c->qw64[1], c->qwp[0],
                   c->qwp[1], c->qy, c->qunits[0], c->qunits[1], c->sur.feat, c->sur.pred, c->sur.est, c->sur.target,
                   c->sur.resid, c->sur.walker_of, c->sur.xbar, c->sur.e1, c->sur.master, c->sur.m,
                   c->sur.v, c->sur.wbf, c->sur.bias, c->sur.grad, c->sur.loss, c->sur.state, c->sur.gT,

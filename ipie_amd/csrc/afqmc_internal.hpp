@@ -93,6 +93,10 @@ struct GfArgs {
 // must be zero before; every writer stores 1)
 hipError_t launch_imag_any(const double* z, int64_t n, int* flag, hipStream_t stream);
 hipError_t launch_gf(const GfArgs& a, bool want_ghalf, hipStream_t stream);
+// The same with Ghalf by LU, every sum in the order that the mixed step keeps
+// (k_greens_lu.hip); bytes of each of its work buffers (O, O^{-1})
+size_t gf_lu_work_bytes(int nwalkers, int nalpha, int nbeta);
+hipError_t launch_gf_lu(const GfArgs& a, double* obuf, double* oinv, hipStream_t stream);
 
 // ---------------------------------------------------------------- GEMMs
 // Rows of a complex operand A (K contiguous) times rows of a real operand B
