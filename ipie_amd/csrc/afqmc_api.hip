@@ -36,7 +36,7 @@ struct afqmc_ctx {
   double* exx_b = nullptr;       // [xs_b, W] complex
   double* vhs = nullptr;         // FP64: packed upper triangles [W, N (N + 1) / 2] complex
   double* buf[4] = {nullptr, nullptr, nullptr, nullptr};  // P, Ta, Tb, Q (mixed): [W, N, ncol] complex
-  int* qr_slow = nullptr;        // [W] scratch of the re-orthogonalisation
+  int* qr_slow = nullptr;        // FP64: [W] scratch of the re-orthogonalisation
   double* exp_pad = nullptr;     // FP64: expH1 [2, N, exp_ld], zero past N
   bool exp_ready = false;        // exp_pad holds the current expH1
   int* flags = nullptr;
@@ -383,7 +383,6 @@ int ensure_ws(afqmc_ctx* c) {
   if (ok) c->fb_cap = c->fb_ksplit;
   ok = ok && dmalloc((void**)&c->xshifted, 16 * (size_t)W * X) == hipSuccess;
   ok = ok && dmalloc((void**)&c->wvec, 16 * (size_t)6 * W) == hipSuccess;
-  ok = ok && dmalloc((void**)&c->qr_slow, sizeof(int) * (size_t)W) == hipSuccess;
   // partial sums: at most one per Cholesky vector per walker, whatever the split
   c->exx_cap = (int64_t)X * W;
   ok = ok && dmalloc((void**)&c->exx_a, 16 * (size_t)c->exx_cap) == hipSuccess;
@@ -420,6 +419,7 @@ int ensure_ws(afqmc_ctx* c) {
   if (d.precision != AFQMC_PREC_MIXED) {
     ok = ok && dmalloc((void**)&c->vhs, 16 * (size_t)W * P) == hipSuccess;
     ok = ok && dmalloc((void**)&c->exp_pad, 8 * (size_t)2 * N * exp_ld(c)) == hipSuccess;
+    ok = ok && dmalloc((void**)&c->qr_slow, sizeof(int) * (size_t)W) == hipSuccess;
   }
   for (int i = 0; i < 4; ++i) {  // (the FP64 path takes three)
     if (i == 3 && d.precision != AFQMC_PREC_MIXED) continue;

@@ -568,7 +568,7 @@ struct ReorthoArgs {
   const double* detR_shift;  // [W] or null
   int* flags;
   int* wflags;               // [W] per-walker flags or null
-  int* slow;                 // [W] scratch: walkers left to the general kernel
+  int* slow;                 // [W] scratch: walkers left to the general kernel; null: all
 };
 hipError_t launch_reortho(const ReorthoArgs& a, hipStream_t stream);
 

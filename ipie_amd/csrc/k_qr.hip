@@ -7,8 +7,11 @@
 //   G = X^H X (+ shift),  G = R^H R,  X <- X R^{-1},
 // as sweeps over the rows of X on FP64 MFMA: the Gram matrix of pass p + 1 is
 // formed from the rows of X R_p^{-1} while they are written.
-// Walkers with at most 48 columns that take the first branch below, that is all but
-// ill-conditioned ones, run in reortho_fast_kernel, the others in reortho_kernel.
+// In double precision the walkers with at most 48 columns that take the first branch
+// below, that is all but ill-conditioned ones, run in reortho_fast_kernel, the others
+// in reortho_kernel.  In mixed precision all run in reortho_kernel: the walkers are
+// rounded to pairs of BF16 values next, so that another order of the sums, which
+// moves their last bits, would move a walker by 1e-6 now and then (k_greens_lu.hip).
 //   - CholeskyQR2 (two passes, three sweeps; Yamamoto, Nakatsukasa, Yanagisawa,
 //     Fukaya, ETNA 44 (2015) 306) when the unshifted Cholesky of X^H X succeeds
 //     and 8 kappa sqrt(N n u + n (n + 1) u) <= 1/2 with kappa bounded by
@@ -705,12 +708,15 @@ hipError_t launch_qr_nt(const ReorthoArgs& a, hipStream_t stream) {
   hipError_t e = allow_lds((const void*)reortho_kernel<NT>, 2 * matrix);
   if (e != hipSuccess) return e;
   ReorthoArgs b = a;
-  if constexpr (NT <= 3) {  // (64 columns do not fit the fast kernel's registers)
+  bool fast = a.slow != nullptr;
+  if constexpr (NT > 3) fast = false;  // (64 columns do not fit the fast kernel's registers)
+  if constexpr (NT <= 3) if (fast) {
     const size_t lds = matrix * (a.nbeta > 0 ? 2 : 1);
     e = allow_lds((const void*)reortho_fast_kernel<NT>, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(reortho_fast_kernel<NT>, dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a);
-  } else {
+  }
+  if (!fast) {
     b.slow = nullptr;
     if (a.mark.acc && (e = launch_phase_mark(a.mark, stream)) != hipSuccess) return e;
   }
@@ -722,7 +728,6 @@ hipError_t launch_qr_nt(const ReorthoArgs& a, hipStream_t stream) {
 
 hipError_t launch_reortho(const ReorthoArgs& a, hipStream_t stream) {
   const int nmax = a.nalpha > a.nbeta ? a.nalpha : a.nbeta;
-  if (!a.slow) return hipErrorInvalidValue;
   switch ((nmax + 15) / 16) {
     case 1: return launch_qr_nt<1>(a, stream);
     case 2: return launch_qr_nt<2>(a, stream);

@@ -60,3 +60,18 @@ def test_greens_function(case, want):
     ga, gb, ov = z(W, na, N), z(W, nb, N), z(W)
     ctx.greens_function(*phi, ga, gb, ov)
     assert _digest(ga, gb, ov) == want
+
+
+QR = ["9d456fa24600893d", "bd9f7ffbf511507a", "347a6b8a9cefe073", "b2ea3f048e36f6f3",
+      "c21372017d2d32e3", "b09e3537a776d7b5", "a279fddf69f78a14"]
+
+
+@pytest.mark.parametrize("case, want", list(zip(CASES, QR)))
+def test_reortho(case, want):
+    import torch
+
+    N, na, nb, W, rhf = case
+    ctx, phi, z = _state(*case)
+    det, logdet = (torch.zeros(W, dtype=torch.float64, device=phi[0].device) for _ in range(2))
+    ctx.reortho(*phi, z(W), det, logdet)
+    assert _digest(*phi, det) == want
