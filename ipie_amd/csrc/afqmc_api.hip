@@ -821,6 +821,7 @@ int taylor_bf16(afqmc_ctx* c, int nw, const double** result, const uint16_t** re
     t.init = P;
     t.q = Q;
     t.nterms = c->d.exp_nmax;
+    for (int j = 1; j < t.nterms; ++j) t.terms[j - 1] = c->tplanes[j];
     t.qout = c->tplanes[c->d.exp_nmax == 1 ? 1 : 0];
     HIP_TRY(c, launch_taylor_bf16_series(t, c->stream));
     *result = Q;

@@ -326,7 +326,8 @@ struct TaylorBf16Args {
   const double* init;       // [W][N][ncol] complex: the series' input (read by the last term)
   double* q;                // [W][N][ncol] complex: init + sum of the terms (written by the last term)
   // last term: the planes of the earlier terms out_1 .. out_nterms (layout of tin), summed into q
-  const uint16_t* terms[TAYLOR_MAX_TERMS];
+  // (the series in one launch writes them too: out_1 .. out_{nterms - 1})
+  uint16_t* terms[TAYLOR_MAX_TERMS];
   int nterms;
   int first, last;          // this term is the first / the last of the series
   int split;                // 1: three BF16 products (hi hi + hi lo + lo hi), 0: hi hi only

@@ -75,3 +75,17 @@ def test_reortho(case, want):
     det, logdet = (torch.zeros(W, dtype=torch.float64, device=phi[0].device) for _ in range(2))
     ctx.reortho(*phi, z(W), det, logdet)
     assert _digest(*phi, det) == want
+
+
+STEP = ["ef0c677a9e68a900", "08e2b209ce9f24d2", "aee5d78bfb0f9857", "60706f5073251cc8",
+        "0a09d63071a462d0", "cb88c5e06419f963", "3428e7279e1d83f6"]
+
+
+@pytest.mark.parametrize("case, want", list(zip(CASES, STEP)))
+def test_step(case, want):
+    N, na, nb, W, rhf = case
+    ctx, phi, z = _state(*case)
+    g = [p.transpose(1, 2).conj().resolve_conj().contiguous() for p in phi]
+    ctx.two_body(*phi, *g, z(W), z(W), seed=3, counter=9)
+    ctx.one_body(*phi)
+    assert _digest(*phi) == want
