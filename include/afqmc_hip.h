@@ -110,7 +110,12 @@ void afqmc_destroy(afqmc_ctx* ctx);
 int afqmc_set_stream(afqmc_ctx* ctx, void* stream);
 /* Borrows the static tensors.  Reads the trial orbitals once on the context's
  * stream (and waits for it): when their imaginary parts are all zero, the
- * overlap matrices take two real products per step instead of four. */
+ * overlap matrices take two real products per step instead of four.  Double
+ * precision reads the other tensors in every call, but for the quadratic form of
+ * the exchange, which is made from rchol in the first call that needs it; mixed
+ * precision makes its split planes of rchol, chol_packed and expH1 in the first
+ * call that needs them.  A caller who rewrites one of these in place calls
+ * afqmc_set_static again. */
 int afqmc_set_static(afqmc_ctx* ctx, const afqmc_static* s);
 const char* afqmc_last_error(const afqmc_ctx* ctx);
 int afqmc_sync(afqmc_ctx* ctx);

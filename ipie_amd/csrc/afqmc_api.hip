@@ -37,8 +37,6 @@ struct afqmc_ctx {
   double* vhs = nullptr;         // FP64: packed upper triangles [W, N (N + 1) / 2] complex
   double* buf[4] = {nullptr, nullptr, nullptr, nullptr};  // P, Ta, Tb, Q (mixed): [W, N, ncol] complex
   int* qr_slow = nullptr;        // FP64: [W] scratch of the re-orthogonalisation
-  double* exp_pad = nullptr;     // FP64: expH1 [2, N, exp_ld], zero past N
-  bool exp_ready = false;        // exp_pad holds the current expH1
   int* flags = nullptr;
   int* wflags = nullptr;    // [W] per-walker flags (OR of AFQMC_FLAG_*) since the last take
   int* psi_flag = nullptr;  // scratch of afqmc_set_static's check of the trial orbitals
@@ -241,9 +239,6 @@ int64_t quad64_ld(const afqmc_ctx* c, int spin) {
   return nN + nN % 2;
 }
 
-// row length of the FP64 path's copy of expH1: whole K chunks, zero past N
-int exp_ld(const afqmc_ctx* c) { return (c->d.nbasis + 15) / 16 * 16; }
-
 bool two_spins(const afqmc_ctx* c) { return c->d.nbeta > 0 && !c->d.rhf; }
 
 double* wv(afqmc_ctx* c, int i) { return c->wvec + 2 * (int64_t)i * c->d.nwalkers; }
@@ -418,7 +413,6 @@ int ensure_ws(afqmc_ctx* c) {
   // FP64 VHS, packed upper triangles (1.3 GB at N=400); the split-BF16 path keeps VHS as atoms only
   if (d.precision != AFQMC_PREC_MIXED) {
     ok = ok && dmalloc((void**)&c->vhs, 16 * (size_t)W * P) == hipSuccess;
-    ok = ok && dmalloc((void**)&c->exp_pad, 8 * (size_t)2 * N * exp_ld(c)) == hipSuccess;
     ok = ok && dmalloc((void**)&c->qr_slow, sizeof(int) * (size_t)W) == hipSuccess;
   }
   for (int i = 0; i < 4; ++i) {  // (the FP64 path takes three)
@@ -648,21 +642,16 @@ int do_vhs(afqmc_ctx* c, int nw) {
 int one_body64(afqmc_ctx* c, int nw, const double* const phi[2], double* const phi_out[2], const double* src,
                double* dst, const PhaseMark& mark) {
   const int N = c->d.nbasis, nc = c->ncol, n[2] = {c->d.nalpha, c->d.nbeta};
-  if (!c->exp_ready) {
-    HIP_TRY(c, launch_pad_rows(c->s.expH1, 2 * N, N, exp_ld(c), c->exp_pad, c->stream));
-    c->exp_ready = !c->capturing;  // (a recorded launch has not run yet)
-  }
   OneBody64Args a{};
   a.mark = mark;
   a.nwalkers = nw;
   a.nbasis = N;
   a.nspin = two_spins(c) ? 2 : 1;
-  a.ld_exp = exp_ld(c);
   for (int s = 0; s < a.nspin; ++s) {
     OneBody64Spin& p = a.spin[s];
     const int off = s == 0 ? 0 : n[0];
     p.n = n[s];
-    p.exp = c->exp_pad + (int64_t)s * N * a.ld_exp;
+    p.exp = c->s.expH1 + (int64_t)s * N * N;
     p.src = src ? src : phi[s];
     p.src_ws = (int64_t)N * (src ? nc : n[s]);
     p.src_ld = src ? nc : n[s];
@@ -1449,7 +1438,7 @@ void afqmc_destroy(afqmc_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   else (void)hipDeviceSynchronize();
   void* ptrs[] = {c->vbias_part, c->xshifted, c->wvec, c->exx_a, c->exx_b, c->vhs, c->buf[0], c->buf[1],
-                  c->buf[2], c->buf[3], c->exp_pad, c->qr_slow, c->flags, c->wflags, c->psi_flag, c->nfb, c->gplanes[0], c->gplanes[1], c->lplanes[0],
+                  c->buf[2], c->buf[3], c->qr_slow, c->flags, c->wflags, c->psi_flag, c->nfb, c->gplanes[0], c->gplanes[1], c->lplanes[0],
                   c->lplanes[1], c->xplanes, c->cplanes, c->vatoms, c->zatom, c->dplanes, c->oplanes, c->gcomp, c->gf_o, c->gf_oinv, c->qw64[0], c->qw64[1], c->qwp[0],
                   c->qwp[1], c->qy, c->qunits[0], c->qunits[1], c->sur.feat, c->sur.pred, c->sur.est, c->sur.target,
                   c->sur.resid, c->sur.walker_of, c->sur.xbar, c->sur.e1, c->sur.master, c->sur.m,
@@ -1497,7 +1486,6 @@ int afqmc_set_static(afqmc_ctx* c, const afqmc_static* s) {
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   c->psi_real = any == 0;
   c->planes_ready = false;
-  c->exp_ready = false;
   c->quad_ready = false;
   c->q8_ready = false;
   c->sur.cv_ready = false;

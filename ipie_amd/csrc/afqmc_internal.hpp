@@ -140,8 +140,8 @@ constexpr int QUAD64_TILE = 128;  // column tile of the FP64 W'
 constexpr int FB_MAX_SPLIT = 16;  // most K ranges of the FP64 force bias (heuristic)
 
 // One body of both spins: out[w][i][out_off + c] = sum_k exp[i][k] src[w][k][src_off + c],
-// c < n (complex; walker strides ws and row lengths ld in complex values; exp real,
-// rows of ld_exp, a multiple of 16, zero past nbasis).
+// c < n (complex; walker strides ws and row lengths ld in complex values; exp real
+// [nbasis, nbasis], the caller's).
 struct OneBody64Spin {
   int n;
   const double* exp;
@@ -154,12 +154,10 @@ struct OneBody64Spin {
 };
 struct OneBody64Args {
   PhaseMark mark;
-  int nwalkers, nbasis, nspin, ld_exp;
+  int nwalkers, nbasis, nspin;
   OneBody64Spin spin[2];
 };
 hipError_t launch_one_body64(const OneBody64Args& a, hipStream_t stream);
-// rows of n values -> rows of ld, zero past n
-hipError_t launch_pad_rows(const double* src, int rows, int n, int ld, double* dst, hipStream_t stream);
 
 // out[w] = base[w] + alpha V[w] prev[w] ([W, N, ncol] complex; V symmetric, as the
 // packed upper triangle [W, N (N + 1) / 2] complex)

@@ -35,6 +35,10 @@ __device__ __forceinline__ void pg_load16(const char* src, void* dst) {
   __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 
+__device__ __forceinline__ void pg_load4(const char* src, void* dst) {
+  __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)dst, 4, 0, 0);
+}
+
 // address of 16 zero bytes, kept in scalar registers
 __device__ __forceinline__ const char* pg_zeros() {
   const char* z = reinterpret_cast<const char*>(&pg_zero);
@@ -61,19 +65,21 @@ __device__ __forceinline__ void pg_reads_first() {
 // Workgroup tile: 16 RM rows of expH1 x 128 real columns (64 walker columns of
 // one spin, over the walkers), 32 of them per wave.  LDS: row r of A keeps its
 // pair p of K values in slot r 8 + (p ^ (r % 8)); B is K rows of 64 complex values.
-template <int RM>
+// expH1 is read where the caller keeps it, in every call.  Its rows are 16-byte aligned
+// for even N; for odd N they are loaded 4 bytes a lane (ALIGNED false).
+template <int RM, bool ALIGNED>
 struct ObPlan {
-  static constexpr int A_LOADS = (2 * RM + 3) / 4, LOADS = A_LOADS + 4;  // per wave
-  static constexpr int A_SLOTS = 256 * A_LOADS, STAGE = A_SLOTS + 1024;
+  static constexpr int A_LOADS = ALIGNED ? (2 * RM + 3) / 4 : 2 * RM, LOADS = A_LOADS + 4;  // per wave
+  static constexpr int A_SLOTS = ALIGNED ? 256 * A_LOADS : 128 * RM, STAGE = A_SLOTS + 1024;
   static constexpr int STAGES = RM == 1 ? 4 : RM <= 4 ? 3 : 2;
   static constexpr int LDS_BYTES = 16 * STAGE * STAGES;
   static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
 };
 
-template <int RM>
+template <int RM, bool ALIGNED>
 __global__ void __launch_bounds__(PG_THREADS, 2) one_body64_kernel(OneBody64Args a) {
   phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
-  using P = ObPlan<RM>;
+  using P = ObPlan<RM, ALIGNED>;
   constexpr int ST = P::STAGES, TM = 16 * RM;
   extern __shared__ uint4 pg_lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -90,24 +96,31 @@ __global__ void __launch_bounds__(PG_THREADS, 2) one_body64_kernel(OneBody64Args
   const int row0 = rb * TM;
   const int64_t ncols = (int64_t)a.nwalkers * sp.n;  // complex columns (w, c)
 
-  // this lane's staged rows and column
+  // this lane's staged rows (byte offset, first K value) and column
   uint32_t ao[P::A_LOADS];
+  int ak[P::A_LOADS];
 #pragma unroll
   for (int j = 0; j < P::A_LOADS; ++j) {
-    const int t = (wave * P::A_LOADS + j) * 64 + lane, r = t >> 3, p = (t & 7) ^ (r & 7);
-    ao[j] = 8u * ((uint32_t)min(r, N - 1 - row0) * (uint32_t)a.ld_exp + 2 * p);
+    const int t = ALIGNED ? (wave * P::A_LOADS + j) * 64 + lane : (wave * P::A_LOADS + j) * 16 + (lane >> 2);
+    const int r = t >> 3, p = (t & 7) ^ (r & 7), part = ALIGNED ? 0 : lane & 3;  // part: 4 bytes of a pair
+    ak[j] = 2 * p + (part >> 1);
+    ao[j] = 8u * ((uint32_t)min(r, N - 1 - row0) * (uint32_t)N + 2 * p) + 4 * part;
   }
-  const char* abase = reinterpret_cast<const char*>(sp.exp + (int64_t)row0 * a.ld_exp);
+  const char* abase = reinterpret_cast<const char*>(sp.exp + (int64_t)row0 * N);
   const int64_t col = min(64 * cb + lane, ncols - 1);
   const char* zero = pg_zeros();
   const char* bcol = reinterpret_cast<const char*>(sp.src + 2 * (col / sp.n * sp.src_ws + sp.src_off + col % sp.n));
   const int nch = (int)ceil_div(N, PG_KC);
-  auto fetch = [&](int c) {  // expH1's rows are zero past N up to a multiple of PG_KC
+  auto fetch = [&](int c) {  // (zeros past N)
     const int cc = min(c, nch - 1);
     uint4* As = pg_lds + c % ST * P::STAGE;
     uint4* Bs = As + P::A_SLOTS;
 #pragma unroll
-    for (int j = 0; j < P::A_LOADS; ++j) pg_load16(abase + ao[j] + 8 * PG_KC * cc, As + (wave * P::A_LOADS + j) * 64);
+    for (int j = 0; j < P::A_LOADS; ++j) {
+      const char* p = PG_KC * cc + ak[j] < N ? abase + ao[j] + 8 * PG_KC * cc : zero;
+      if constexpr (ALIGNED) pg_load16(p, As + (wave * P::A_LOADS + j) * 64);
+      else pg_load4(p, As + (wave * P::A_LOADS + j) * 16);
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int k = PG_KC * cc + 4 * wave + j;
@@ -473,14 +486,24 @@ __global__ void __launch_bounds__(NCH > 0 ? 512 : 1024) taylor64_series_kernel(T
   }
 }
 
-template <int RM>
-hipError_t launch_ob_rm(const OneBody64Args& a, int64_t colblocks, hipStream_t stream) {
+inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+template <int RM, bool ALIGNED>
+hipError_t launch_ob_as(const OneBody64Args& a, int64_t colblocks, hipStream_t stream) {
   const int64_t blocks = colblocks * ceil_div(a.nbasis, 16 * RM);
   if (blocks > INT32_MAX) return hipErrorInvalidValue;
-  const hipError_t e = allow_lds(reinterpret_cast<const void*>(one_body64_kernel<RM>), ObPlan<RM>::LDS_BYTES);
+  constexpr int lds = ObPlan<RM, ALIGNED>::LDS_BYTES;
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(one_body64_kernel<RM, ALIGNED>), lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(one_body64_kernel<RM>, dim3((unsigned)blocks), dim3(PG_THREADS), ObPlan<RM>::LDS_BYTES, stream, a);
+  hipLaunchKernelGGL((one_body64_kernel<RM, ALIGNED>), dim3((unsigned)blocks), dim3(PG_THREADS), lds, stream, a);
   return hipGetLastError();
+}
+
+template <int RM>
+hipError_t launch_ob_rm(const OneBody64Args& a, int64_t colblocks, hipStream_t stream) {
+  bool aligned = a.nbasis % 2 == 0;
+  for (int s = 0; s < a.nspin; ++s) aligned = aligned && aligned16(a.spin[s].exp);
+  return aligned ? launch_ob_as<RM, true>(a, colblocks, stream) : launch_ob_as<RM, false>(a, colblocks, stream);
 }
 
 template <int RN>
@@ -514,25 +537,10 @@ hipError_t launch_ty_series_rn(const Taylor64Args& a, hipStream_t stream) {
   }
 }
 
-__global__ void pad_rows_kernel(const double* __restrict__ src, int rows, int n, int ld, double* __restrict__ dst) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)rows * ld) return;
-  const int r = (int)(i / ld), k = (int)(i % ld);
-  dst[i] = k < n ? src[(int64_t)r * n + k] : 0.0;
-}
-
 }  // namespace
 
-hipError_t launch_pad_rows(const double* src, int rows, int n, int ld, double* dst, hipStream_t stream) {
-  hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)ceil_div((int64_t)rows * ld, 256)), dim3(256), 0, stream, src,
-                     rows, n, ld, dst);
-  return hipGetLastError();
-}
-
 hipError_t launch_one_body64(const OneBody64Args& a, hipStream_t stream) {
-  if (a.nwalkers < 1 || a.nspin < 1 || a.nspin > 2 || a.nbasis < 1 || a.ld_exp % PG_KC != 0 || a.ld_exp < a.nbasis ||
-      a.ld_exp > (1 << 20))
-    return hipErrorInvalidValue;
+  if (a.nwalkers < 1 || a.nspin < 1 || a.nspin > 2 || a.nbasis < 1 || a.nbasis > (1 << 20)) return hipErrorInvalidValue;
   int64_t colblocks = 0;
   for (int s = 0; s < a.nspin; ++s) {
     if (a.spin[s].n < 1) return hipErrorInvalidValue;
