@@ -66,20 +66,23 @@ __device__ __forceinline__ void pg_reads_first() {
 // one spin, over the walkers), 32 of them per wave.  LDS: row r of A keeps its
 // pair p of K values in slot r 8 + (p ^ (r % 8)); B is K rows of 64 complex values.
 // expH1 is read where the caller keeps it, in every call.  Its rows are 16-byte aligned
-// for even N; for odd N they are loaded 4 bytes a lane (ALIGNED false).
-template <int RM, bool ALIGNED>
+// for even N; for odd N they are loaded 4 bytes a lane, and so are walkers off 16 bytes
+// (a caller of the C entry points), with 16-row tiles.
+enum { OB_16 = 0, OB_A4 = 1, OB_AB4 = 2 };
+template <int RM, int MODE>
 struct ObPlan {
-  static constexpr int A_LOADS = ALIGNED ? (2 * RM + 3) / 4 : 2 * RM, LOADS = A_LOADS + 4;  // per wave
-  static constexpr int A_SLOTS = ALIGNED ? 256 * A_LOADS : 128 * RM, STAGE = A_SLOTS + 1024;
+  static constexpr int A_LOADS = MODE == OB_16 ? (2 * RM + 3) / 4 : 2 * RM, B_LOADS = MODE == OB_AB4 ? 16 : 4;  // per wave
+  static constexpr int LOADS = A_LOADS + B_LOADS;
+  static constexpr int A_SLOTS = MODE == OB_16 ? 256 * A_LOADS : 128 * RM, STAGE = A_SLOTS + 1024;
   static constexpr int STAGES = RM == 1 ? 4 : RM <= 4 ? 3 : 2;
   static constexpr int LDS_BYTES = 16 * STAGE * STAGES;
-  static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
+  static_assert(2 * LDS_BYTES <= 160 * 1024 && (STAGES - 1) * LOADS <= 63, "two workgroups per CU, vmcnt");
 };
 
-template <int RM, bool ALIGNED>
+template <int RM, int MODE>
 __global__ void __launch_bounds__(PG_THREADS, 2) one_body64_kernel(OneBody64Args a) {
   phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
-  using P = ObPlan<RM, ALIGNED>;
+  using P = ObPlan<RM, MODE>;
   constexpr int ST = P::STAGES, TM = 16 * RM;
   extern __shared__ uint4 pg_lds[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -101,15 +104,21 @@ __global__ void __launch_bounds__(PG_THREADS, 2) one_body64_kernel(OneBody64Args
   int ak[P::A_LOADS];
 #pragma unroll
   for (int j = 0; j < P::A_LOADS; ++j) {
-    const int t = ALIGNED ? (wave * P::A_LOADS + j) * 64 + lane : (wave * P::A_LOADS + j) * 16 + (lane >> 2);
-    const int r = t >> 3, p = (t & 7) ^ (r & 7), part = ALIGNED ? 0 : lane & 3;  // part: 4 bytes of a pair
+    const int t = MODE == OB_16 ? (wave * P::A_LOADS + j) * 64 + lane : (wave * P::A_LOADS + j) * 16 + (lane >> 2);
+    const int r = t >> 3, p = (t & 7) ^ (r & 7), part = MODE == OB_16 ? 0 : lane & 3;  // part: 4 bytes of a pair
     ak[j] = 2 * p + (part >> 1);
     ao[j] = 8u * ((uint32_t)min(r, N - 1 - row0) * (uint32_t)N + 2 * p) + 4 * part;
   }
   const char* abase = reinterpret_cast<const char*>(sp.exp + (int64_t)row0 * N);
-  const int64_t col = min(64 * cb + lane, ncols - 1);
   const char* zero = pg_zeros();
-  const char* bcol = reinterpret_cast<const char*>(sp.src + 2 * (col / sp.n * sp.src_ws + sp.src_off + col % sp.n));
+  constexpr int BC = MODE == OB_AB4 ? 4 : 1;  // loads of a K row: 64 columns, or 16 of 4 x 4 bytes
+  const char* bcol[BC];
+#pragma unroll
+  for (int h = 0; h < BC; ++h) {
+    const int64_t col = min(64 * cb + (MODE == OB_AB4 ? 16 * h + (lane >> 2) : lane), ncols - 1);
+    bcol[h] = reinterpret_cast<const char*>(sp.src + 2 * (col / sp.n * sp.src_ws + sp.src_off + col % sp.n)) +
+              (MODE == OB_AB4 ? 4 * (lane & 3) : 0);
+  }
   const int nch = (int)ceil_div(N, PG_KC);
   auto fetch = [&](int c) {  // (zeros past N)
     const int cc = min(c, nch - 1);
@@ -118,14 +127,18 @@ __global__ void __launch_bounds__(PG_THREADS, 2) one_body64_kernel(OneBody64Args
 #pragma unroll
     for (int j = 0; j < P::A_LOADS; ++j) {
       const char* p = PG_KC * cc + ak[j] < N ? abase + ao[j] + 8 * PG_KC * cc : zero;
-      if constexpr (ALIGNED) pg_load16(p, As + (wave * P::A_LOADS + j) * 64);
+      if constexpr (MODE == OB_16) pg_load16(p, As + (wave * P::A_LOADS + j) * 64);
       else pg_load4(p, As + (wave * P::A_LOADS + j) * 16);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int k = PG_KC * cc + 4 * wave + j;
-      const char* p = bcol + 16 * (int64_t)k * sp.src_ld;
-      pg_load16(k < N ? p : zero, Bs + (4 * wave + j) * 64);
+#pragma unroll
+      for (int h = 0; h < BC; ++h) {
+        const char* p = bcol[h] + 16 * (int64_t)k * sp.src_ld;
+        if constexpr (MODE == OB_AB4) pg_load4(k < N ? p : zero, Bs + (4 * wave + j) * 64 + 16 * h);
+        else pg_load16(k < N ? p : zero, Bs + (4 * wave + j) * 64);
+      }
     }
   };
   auto read = [&](int c, int h, v2d (&af)[RM], double (&bf)[2][2]) {
@@ -488,14 +501,14 @@ __global__ void __launch_bounds__(NCH > 0 ? 512 : 1024) taylor64_series_kernel(T
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-template <int RM, bool ALIGNED>
+template <int RM, int MODE>
 hipError_t launch_ob_as(const OneBody64Args& a, int64_t colblocks, hipStream_t stream) {
   const int64_t blocks = colblocks * ceil_div(a.nbasis, 16 * RM);
   if (blocks > INT32_MAX) return hipErrorInvalidValue;
-  constexpr int lds = ObPlan<RM, ALIGNED>::LDS_BYTES;
-  const hipError_t e = allow_lds(reinterpret_cast<const void*>(one_body64_kernel<RM, ALIGNED>), lds);
+  constexpr int lds = ObPlan<RM, MODE>::LDS_BYTES;
+  const hipError_t e = allow_lds(reinterpret_cast<const void*>(one_body64_kernel<RM, MODE>), lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((one_body64_kernel<RM, ALIGNED>), dim3((unsigned)blocks), dim3(PG_THREADS), lds, stream, a);
+  hipLaunchKernelGGL((one_body64_kernel<RM, MODE>), dim3((unsigned)blocks), dim3(PG_THREADS), lds, stream, a);
   return hipGetLastError();
 }
 
@@ -503,7 +516,7 @@ template <int RM>
 hipError_t launch_ob_rm(const OneBody64Args& a, int64_t colblocks, hipStream_t stream) {
   bool aligned = a.nbasis % 2 == 0;
   for (int s = 0; s < a.nspin; ++s) aligned = aligned && aligned16(a.spin[s].exp);
-  return aligned ? launch_ob_as<RM, true>(a, colblocks, stream) : launch_ob_as<RM, false>(a, colblocks, stream);
+  return aligned ? launch_ob_as<RM, OB_16>(a, colblocks, stream) : launch_ob_as<RM, OB_A4>(a, colblocks, stream);
 }
 
 template <int RN>
@@ -546,6 +559,8 @@ hipError_t launch_one_body64(const OneBody64Args& a, hipStream_t stream) {
     if (a.spin[s].n < 1) return hipErrorInvalidValue;
     colblocks += ceil_div((int64_t)a.nwalkers * a.spin[s].n, 64);
   }
+  for (int s = 0; s < a.nspin; ++s)
+    if (!aligned16(a.spin[s].src)) return launch_ob_as<1, OB_AB4>(a, colblocks, stream);
   // Row tiles of 16 RM: the least padding of N, against half a 16-row tile per
   // workgroup for the columns it reads again; smaller ones while CUs would idle.
   int best = 1;
