@@ -29,6 +29,7 @@
 // (eight rows, one k) hit eight different 16-byte bank groups.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "afqmc_internal.hpp"
 
@@ -59,7 +60,8 @@ __device__ __forceinline__ void nt_load4(const char* src, void* dst) {
 }
 
 // Loads of 16 bytes a lane where the operand's rows are 16-byte aligned (and B's
-// K even, so that a pair is whole or absent), of 4 bytes otherwise.
+// K even, so that a pair is whole or absent), of 4 bytes otherwise.  Byte offsets within
+// a tile take 32 bits, but for NT_AB4, which also takes rows of more than 2^22 values.
 enum { NT_16 = 0, NT_B4 = 1, NT_AB4 = 2 };
 
 template <int RM, int MODE>
@@ -128,7 +130,8 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
     const char* abase = reinterpret_cast<const char*>(sg.A + 2 * (int64_t)row0 * sg.lda);
     const char* bbase = reinterpret_cast<const char*>(sg.B + col0 * sg.ldb);
     const uint32_t last_r = (uint32_t)min((int64_t)TM, a.m - row0) - 1, last_c = (uint32_t)min((int64_t)NT_TN, a.n - col0) - 1;
-    const uint32_t apitch = 16u * (uint32_t)sg.lda, bpitch = 8u * (uint32_t)sg.ldb;
+    using offset = std::conditional_t<MODE == NT_AB4, uint64_t, uint32_t>;
+    const offset apitch = 16u * (offset)sg.lda, bpitch = 8u * (offset)sg.ldb;
     auto a_row = [&](int j) { return MODE == NT_AB4 ? 4 * RM * wave + j : 4 * (RM * wave + j) + (lane >> 4); };
     auto a_k = [&](int j) { return (MODE == NT_AB4 ? lane >> 2 : lane & 15) ^ (a_row(j) & 15); };
     auto a_off = [&](int j) {
@@ -138,9 +141,9 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
     auto b_pair = [&](int j) { return (MODE == NT_16 ? lane & 7 : (lane & 31) >> 2) ^ (b_col(j) & 7); };
     auto b_k = [&](int j) { return 2 * b_pair(j) + (MODE == NT_16 ? 0 : (lane & 3) >> 1); };
     auto b_off = [&](int j) {
-      return min((uint32_t)b_col(j) * bpitch, last_c * bpitch) + 16u * b_pair(j) + (MODE == NT_16 ? 0u : 4u * (lane & 3));
+      return min((offset)b_col(j) * bpitch, last_c * bpitch) + 16u * b_pair(j) + (MODE == NT_16 ? 0u : 4u * (lane & 3));
     };
-    uint32_t ao[RM], bo[4];  // of the 16-byte loads
+    offset ao[RM], bo[4];  // of the 16-byte loads
 #pragma unroll
     for (int j = 0; j < RM; ++j) ao[j] = a_off(j);
 #pragma unroll
@@ -315,17 +318,17 @@ hipError_t launch_nt_rm(const NtArgs& a, bool direct, hipStream_t stream) {
 template <int EPI>
 hipError_t launch_nt(const NtArgs& a, hipStream_t stream) {
   if (a.m < 1 || a.n < 1 || a.nseg < 1 || a.nseg > 2 || a.ksplit < 1) return hipErrorInvalidValue;
-  bool a_vec = true, b_vec = true;
+  bool a_vec = true, b_vec = true, far = false;
   int64_t chunks = 0;
   for (int s = 0; s < a.nseg; ++s) {
     const NtSegment& g = a.seg[s];
-    // 32-bit byte offsets within a tile (64 complex rows, 128 real columns)
-    if (g.K < 1 || g.lda < g.K || g.ldb < g.K || g.lda > (1 << 22) || g.ldb > (1 << 22)) return hipErrorInvalidValue;
+    if (g.K < 1 || g.lda < g.K || g.ldb < g.K) return hipErrorInvalidValue;
+    far = far || g.lda > (1 << 22) || g.ldb > (1 << 22);  // 64 complex rows, 128 real columns in 32 bits
     a_vec = a_vec && aligned16(g.A);
     b_vec = b_vec && g.K % 2 == 0 && g.ldb % 2 == 0 && aligned16(g.B);
     chunks += ceil_div(g.K, NT_KC);
   }
-  if (!a_vec) return launch_nt_mode<1, NT_AB4, EPI>(a, stream);
+  if (!a_vec || far) return launch_nt_mode<1, NT_AB4, EPI>(a, stream);
   const int64_t colblocks = EPI == NT_EPI_QDOT ? a.nunits : ceil_div(a.n, NT_TN) * a.ksplit;
   const double each = EPI == NT_EPI_QDOT ? a.unit_chunks + NT_QDOT_CHUNKS : (double)chunks / a.ksplit;
   // (the 4-byte loads' addresses and 64 rows do not fit the registers together)
