@@ -34,6 +34,8 @@
 //   N = 255, n = 25 RHF, W = 71 184 us ->  58      N = 400, n = 40, W = 1024  1230 us -> 890
 // One copy of a step's code instead of CW, or the step without branches, measured the same
 // or slower; three waves a spin, two workgroups a CU, 1130 us at W = 1024.
+#include <algorithm>
+
 #include "afqmc_internal.hpp"
 
 namespace afqmc {
@@ -104,10 +106,11 @@ __global__ void __launch_bounds__(128 * GfPlan<NT>::SW) gf_kernel(GfArgs a) {
   extern __shared__ cplx smem[];
   __shared__ int prow[2][R];  // pivot row of each step
   __shared__ int odd[2];      // parity of the pivot rows' permutation
-  phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
+  phase_mark(a.mark, blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
-  const int s = wave / SW, sw = wave % SW, w = blockIdx.x, N = a.nbasis;
+  const int s = wave / SW, sw = wave % SW, w = blockIdx.y * gridDim.x + blockIdx.x, N = a.nbasis;
+  if (w >= a.nwalkers) return;
   const int n = s == 0 ? a.nalpha : a.nbeta;
   const double* phi = (s == 0 ? a.phia : a.phib) + 2 * (int64_t)w * N * n;
   const double* psi = s == 0 ? a.psia : a.psib;
@@ -378,7 +381,9 @@ hipError_t launch_gf_as(const GfArgs& a, hipStream_t stream) {
   const size_t lds = nspin * gf_lds<NT>();
   const hipError_t e = allow_lds((const void*)gf_kernel<NT, REAL, GHALF, PLANES>, lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((gf_kernel<NT, REAL, GHALF, PLANES>), dim3((unsigned)a.nwalkers),
+  // (a grid dimension takes less than 2^32 threads)
+  const int64_t gx = std::min(a.nwalkers, 1 << 20);
+  hipLaunchKernelGGL((gf_kernel<NT, REAL, GHALF, PLANES>), dim3((unsigned)gx, (unsigned)ceil_div(a.nwalkers, gx)),
                      dim3(64 * GfPlan<NT>::SW * nspin), lds, stream, a);
   return hipGetLastError();
 }
