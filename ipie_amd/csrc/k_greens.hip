@@ -5,8 +5,8 @@
 //   det O_s, O_s^{-1}            columns dealt to the spin's waves (registers, lane =
 //                                row), pivot rows chosen without moving them
 //   ovlp                         phase_a phase_b exp(logdet_a + logdet_b - log_shift)
-//   Ghalf_s = O_s^{-1} phi_s^T   [n, N], FP64 MFMA, a wave per 16 columns; optionally
-//                                also as split-BF16 planes
+//   Ghalf_s = O_s^{-1} phi_s^T   [n, N], FP64 MFMA, a wave per 16 columns
+// (Ghalf of the mixed step: k_greens_lu.hip.)
 // Restates ipie/estimators/greens_function_single_det.py:62-154 and
 // ipie/propagation/overlap.py:29-59.  All reductions are in a fixed order, so
 // the result is bitwise reproducible run to run.
@@ -99,7 +99,7 @@ constexpr size_t gf_lds() {  // per spin: O, two pivot columns, the pivots
   return sizeof(cplx) * (16 * NT * (16 * NT + 1) + 3 * 16 * NT);
 }
 
-template <int NT, bool REAL, bool GHALF, bool PLANES>
+template <int NT, bool REAL, bool GHALF>
 __global__ void __launch_bounds__(128 * GfPlan<NT>::SW) gf_kernel(GfArgs a) {
   using P = GfPlan<NT>;
   constexpr int SW = P::SW, CW = P::CW, R = 16 * NT, LD = R + 1, KU = P::KU;
@@ -289,8 +289,6 @@ __global__ void __launch_bounds__(128 * GfPlan<NT>::SW) gf_kernel(GfArgs a) {
 
   // ---- Ghalf[i][m] = sum_j Oinv[i][j] phi[m][j], all row tiles of 16 columns m a wave
   double* gh = (s == 0 ? a.ghalfa : a.ghalfb) + 2 * (int64_t)w * n * N;
-  const int64_t pstride = (int64_t)a.nwalkers * n * a.kpad;
-  uint16_t* gp = PLANES && a.gplanes[s] ? a.gplanes[s] + (int64_t)w * n * a.kpad : nullptr;
   constexpr int G = 4;  // K steps per group; a group's loads are issued before the MFMAs of the one before
   const int nmt = (int)ceil_div(N, 16);
   for (int mt = SW - 1 - sw; mt < nmt; mt += SW) {  // (the first wave, busy with the overlap, comes last)
@@ -336,27 +334,7 @@ __global__ void __launch_bounds__(128 * GfPlan<NT>::SW) gf_kernel(GfArgs a) {
       for (int r = 0; r < 4; ++r) {
         const int i = it * 16 + 4 * r + kq;  // accumulator row = 4 r + lane / 16
         if (i < n && mm < N) st(gh, (int64_t)i * N + mm, cmake(re[it][r], im[it][r]));
-        if (PLANES && gp && i < n) {  // (zero past N; kpad covers the tile)
-          uint16_t rh, rl, ih, il;
-          split_bf16_pair(mm < N ? re[it][r] : 0.0, rh, rl);
-          split_bf16_pair(mm < N ? im[it][r] : 0.0, ih, il);
-          const int64_t o = (int64_t)i * a.kpad + mm;
-          gp[o] = rh;
-          gp[pstride + o] = rl;
-          gp[2 * pstride + o] = ih;
-          gp[3 * pstride + o] = il;
-        }
       }
-  }
-  if (PLANES && gp && nmt * 16 < a.kpad) {  // K padding in whole 16-column tiles
-    const int pad = a.kpad - nmt * 16;
-    for (int e = sw * 64 + lane; e < n * pad; e += 64 * SW) {
-      const int64_t o = (int64_t)(e / pad) * a.kpad + nmt * 16 + e % pad;
-      gp[o] = 0;
-      gp[pstride + o] = 0;
-      gp[2 * pstride + o] = 0;
-      gp[3 * pstride + o] = 0;
-    }
   }
 }
 
@@ -375,15 +353,15 @@ hipError_t launch_imag_any(const double* z, int64_t n, int* flag, hipStream_t st
 
 namespace {
 
-template <int NT, bool REAL, bool GHALF, bool PLANES>
+template <int NT, bool REAL, bool GHALF>
 hipError_t launch_gf_as(const GfArgs& a, hipStream_t stream) {
   const int nspin = (a.nbeta > 0 && !a.rhf) ? 2 : 1;
   const size_t lds = nspin * gf_lds<NT>();
-  const hipError_t e = allow_lds((const void*)gf_kernel<NT, REAL, GHALF, PLANES>, lds);
+  const hipError_t e = allow_lds((const void*)gf_kernel<NT, REAL, GHALF>, lds);
   if (e != hipSuccess) return e;
   // (a grid dimension takes less than 2^32 threads)
   const int64_t gx = std::min(a.nwalkers, 1 << 20);
-  hipLaunchKernelGGL((gf_kernel<NT, REAL, GHALF, PLANES>), dim3((unsigned)gx, (unsigned)ceil_div(a.nwalkers, gx)),
+  hipLaunchKernelGGL((gf_kernel<NT, REAL, GHALF>), dim3((unsigned)gx, (unsigned)ceil_div(a.nwalkers, gx)),
                      dim3(64 * GfPlan<NT>::SW * nspin), lds, stream, a);
   return hipGetLastError();
 }
@@ -391,17 +369,15 @@ hipError_t launch_gf_as(const GfArgs& a, hipStream_t stream) {
 template <int NT>
 hipError_t launch_gf_nt(const GfArgs& a, bool want_ghalf, hipStream_t stream) {
   if (!want_ghalf)
-    return a.psi_real ? launch_gf_as<NT, true, false, false>(a, stream) : launch_gf_as<NT, false, false, false>(a, stream);
-  if (a.gplanes[0])
-    return a.psi_real ? launch_gf_as<NT, true, true, true>(a, stream) : launch_gf_as<NT, false, true, true>(a, stream);
-  return a.psi_real ? launch_gf_as<NT, true, true, false>(a, stream) : launch_gf_as<NT, false, true, false>(a, stream);
+    return a.psi_real ? launch_gf_as<NT, true, false>(a, stream) : launch_gf_as<NT, false, false>(a, stream);
+  return a.psi_real ? launch_gf_as<NT, true, true>(a, stream) : launch_gf_as<NT, false, true>(a, stream);
 }
 
 }  // namespace
 
 hipError_t launch_gf(const GfArgs& a, bool want_ghalf, hipStream_t stream) {
   const int nmax = (a.nbeta > 0 && !a.rhf && a.nbeta > a.nalpha) ? a.nbeta : a.nalpha;
-  if (nmax < 1 || nmax > 64 || a.nwalkers < 1) return hipErrorInvalidValue;
+  if (nmax < 1 || nmax > 64 || a.nwalkers < 1 || a.gplanes[0]) return hipErrorInvalidValue;
   switch ((nmax + 15) / 16) {
     case 1: return launch_gf_nt<1>(a, want_ghalf, stream);
     case 2: return launch_gf_nt<2>(a, want_ghalf, stream);
