@@ -188,6 +188,7 @@ struct PhaseScope {
   enum How { KERNEL, STAMP };
   afqmc_ctx* c;
   int phase;  // -1 once marked
+  PhaseMark given;
   PhaseScope(afqmc_ctx* ctx, int ph, How how) : c(ctx), phase(ctx->prof && !ctx->capturing ? ph : -1) {
     if (how == STAMP) stamp();
   }
@@ -197,11 +198,20 @@ struct PhaseScope {
       (void)launch_phase_clear(c->prof_acc, AFQMC_NPHASES, c->stream);
       c->prof_clear = false;
     }
-    const PhaseMark m{c->prof_acc, c->prof_open, phase};
+    given = PhaseMark{c->prof_acc, c->prof_open, phase};
     c->prof_open = phase;
     c->prof_count[phase] += 1;
     phase = -1;
-    return m;
+    return given;
+  }
+  // the launch that took mark(): one that was refused has opened nothing and closed nothing
+  hipError_t launched(hipError_t e) {
+    if (e != hipSuccess && given.acc && c->prof_open == given.phase) {
+      c->prof_open = given.prev;
+      c->prof_count[given.phase] -= 1;
+      given = PhaseMark{};
+    }
+    return e;
   }
   void stamp() {
     if (phase >= 0) (void)launch_phase_mark(mark(), c->stream);
@@ -211,6 +221,13 @@ struct PhaseScope {
     if (!c->prof_chain) close_phase(c);
   }
 };
+
+// HIP_TRY of the launch that took ps.mark()
+#define PHASE_TRY(c, ps, expr)                                                                     \
+  do {                                                                                            \
+    const hipError_t _e = (ps).launched(expr);                                                    \
+    if (_e != hipSuccess) return fail((c), AFQMC_ERR_HIP, "%s: %s", #expr, hipGetErrorString(_e)); \
+  } while (0)
 
 // A sequence of phases with nothing between them: each phase's start is the end of
 // the one before.  Not for the control variate's energies, whose kernels between the
@@ -500,7 +517,7 @@ int do_gf(afqmc_ctx* c, int nw, const double* phia, const double* phib, double* 
   }
   PhaseScope ps(c, want_ghalf ? AFQMC_PHASE_GF : AFQMC_PHASE_OVERLAP, PhaseScope::KERNEL);
   a.mark = ps.mark();
-  HIP_TRY(c, lu ? launch_gf_lu(a, c->gf_o, c->gf_oinv, c->stream) : launch_gf(a, want_ghalf, c->stream));
+  PHASE_TRY(c, ps, lu ? launch_gf_lu(a, c->gf_o, c->gf_oinv, c->stream) : launch_gf(a, want_ghalf, c->stream));
   return AFQMC_OK;
 }
 
@@ -559,7 +576,7 @@ int do_force_bias(afqmc_ctx* c, int nw, const double* ga, const double* gb) {
   a.out = c->vbias_part;
   PhaseScope ps(c, AFQMC_PHASE_FORCE_BIAS, PhaseScope::KERNEL);
   a.mark = ps.mark();
-  HIP_TRY(c, launch_nt64(a, c->stream));
+  PHASE_TRY(c, ps, launch_nt64(a, c->stream));
   return AFQMC_OK;
 }
 
@@ -590,7 +607,7 @@ int do_fields(afqmc_ctx* c, int nw, bool want_fields, const double* xi, uint64_t
   a.xbar_max = c->sur.enabled ? c->sur.xbar + c->d.nwalkers : nullptr;
   PhaseScope ps(c, AFQMC_PHASE_FIELDS, PhaseScope::KERNEL);
   a.mark = ps.mark();
-  HIP_TRY(c, launch_fields(a, c->stream));
+  PHASE_TRY(c, ps, launch_fields(a, c->stream));
   return AFQMC_OK;
 }
 
@@ -633,17 +650,17 @@ int do_vhs(afqmc_ctx* c, int nw) {
   a.times_i = 1;
   PhaseScope ps(c, AFQMC_PHASE_VHS, PhaseScope::KERNEL);
   a.mark = ps.mark();
-  HIP_TRY(c, launch_nt64(a, c->stream));
+  PHASE_TRY(c, ps, launch_nt64(a, c->stream));
   return AFQMC_OK;
 }
 
 // FP64 one body of both spins: phi_s -> the concatenated buffer dst (gather) or the
 // concatenated buffer src -> phi_s (scatter).
 int one_body64(afqmc_ctx* c, int nw, const double* const phi[2], double* const phi_out[2], const double* src,
-               double* dst, const PhaseMark& mark) {
+               double* dst, PhaseScope& ps) {
   const int N = c->d.nbasis, nc = c->ncol, n[2] = {c->d.nalpha, c->d.nbeta};
   OneBody64Args a{};
-  a.mark = mark;
+  a.mark = ps.mark();
   a.nwalkers = nw;
   a.nbasis = N;
   a.nspin = two_spins(c) ? 2 : 1;
@@ -661,7 +678,7 @@ int one_body64(afqmc_ctx* c, int nw, const double* const phi[2], double* const p
     p.out_ld = dst ? nc : n[s];
     p.out_off = dst ? off : 0;
   }
-  HIP_TRY(c, launch_one_body64(a, c->stream));
+  PHASE_TRY(c, ps, launch_one_body64(a, c->stream));
   return AFQMC_OK;
 }
 
@@ -737,7 +754,7 @@ int gather(afqmc_ctx* c, int nw, const double* phia, const double* phib, bool wi
   }
   if (with_expH1) {
     const double* const phi[2] = {phia, phib};
-    return one_body64(c, nw, phi, nullptr, nullptr, P, ps.mark());
+    return one_body64(c, nw, phi, nullptr, nullptr, P, ps);
   }
   HIP_TRY(c, hipMemcpy2DAsync(P, 16 * nc, phia, 16 * na, 16 * na, (size_t)nw * N, hipMemcpyDeviceToDevice,
                               c->stream));
@@ -771,7 +788,7 @@ int scatter(afqmc_ctx* c, int nw, const double* src, double* phia, double* phib,
   }
   if (with_expH1) {
     double* const phi[2] = {phia, phib};
-    return one_body64(c, nw, nullptr, phi, src, nullptr, ps.mark());
+    return one_body64(c, nw, nullptr, phi, src, nullptr, ps);
   }
   HIP_TRY(c, hipMemcpy2DAsync(phia, 16 * na, src, 16 * nc, 16 * na, (size_t)nw * N, hipMemcpyDeviceToDevice,
                               c->stream));
@@ -867,7 +884,7 @@ int taylor(afqmc_ctx* c, int nw, const double** result, const uint16_t** resultT
     t.out = c->buf[1];
     t.terms = c->d.exp_nmax;
     t.mark = ps.mark();
-    HIP_TRY(c, launch_taylor64_series(t, c->stream));
+    PHASE_TRY(c, ps, launch_taylor64_series(t, c->stream));
     *result = t.out;
     return AFQMC_OK;
   }
@@ -876,7 +893,8 @@ int taylor(afqmc_ctx* c, int nw, const double** result, const uint16_t** resultT
     t.out = prev == c->buf[1] ? c->buf[2] : c->buf[1];
     t.alpha = 1.0 / k;
     t.mark = ps.mark();  // the first term's; later ones get none
-    HIP_TRY(c, launch_taylor64(t, c->stream));
+    if (t.mark.acc) PHASE_TRY(c, ps, launch_taylor64(t, c->stream));
+    else HIP_TRY(c, launch_taylor64(t, c->stream));
     prev = t.out;
   }
   *result = prev;
@@ -1060,7 +1078,7 @@ int exchange_spin_quad(afqmc_ctx* c, int nw, int spin, const double* g, const in
     a.unit_chunks = c->quad64_chunks[spin];
     a.dg = g;
     a.mark = ps.mark();
-    HIP_TRY(c, launch_nt64(a, c->stream));
+    PHASE_TRY(c, ps, launch_nt64(a, c->stream));
     HIP_TRY(c, launch_quad_sum(c->qy, a.nunits, nw, part, c->stream));
   }
   c->xs_used[spin] = 1;
@@ -1152,7 +1170,7 @@ int do_energy(afqmc_ctx* c, int nw, const double* ga, const double* gb, double* 
   a.e1_in = e1_in;
   PhaseScope ps(c, AFQMC_PHASE_ENERGY, PhaseScope::KERNEL);
   a.mark = ps.mark();
-  HIP_TRY(c, launch_energy(a, c->stream));
+  PHASE_TRY(c, ps, launch_energy(a, c->stream));
   return AFQMC_OK;
 }
 
@@ -1921,8 +1939,8 @@ int afqmc_update_weight(afqmc_ctx* c, int32_t nw, const double* ovlp, const doub
   a.wflags = c->wflags;
   PhaseScope ps(c, AFQMC_PHASE_WEIGHT, PhaseScope::KERNEL);
   a.mark = ps.mark();
+  PHASE_TRY(c, ps, launch_update_weight(a, c->stream));
   if (a.mark.acc) c->prof_open = -1;  // the kernel closes its phase itself
-  HIP_TRY(c, launch_update_weight(a, c->stream));
   return AFQMC_OK;
 }
 
@@ -2038,7 +2056,7 @@ int afqmc_reortho(afqmc_ctx* c, int32_t nw, double* phia, double* phib, double* 
   a.slow = c->qr_slow;
   PhaseScope ps(c, AFQMC_PHASE_REORTHO, PhaseScope::KERNEL);
   a.mark = ps.mark();
-  HIP_TRY(c, launch_reortho(a, c->stream));
+  PHASE_TRY(c, ps, launch_reortho(a, c->stream));
   return AFQMC_OK;
 }
 

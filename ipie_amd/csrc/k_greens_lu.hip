@@ -414,13 +414,13 @@ __global__ void __launch_bounds__(64 * GF_WAVES) gf_ghalf_kernel(GfArgs a, const
 template <int NT>
 hipError_t launch_gf_lu_nt(const GfArgs& a, double* obuf, double* oinv, int nmax, hipStream_t stream) {
   const int nspin = (a.nbeta > 0 && !a.rhf) ? 2 : 1;
+  const size_t lds = sizeof(cplx) * ((size_t)nmax * (nmax + 1) + nmax);
+  hipError_t e = allow_lds((const void*)gf_lu_kernel, lds);
+  if (e != hipSuccess) return e;
   const dim3 grid((unsigned)ceil_div((int64_t)a.nwalkers * nspin * NT, GF_WAVES)), block(64 * GF_WAVES);
   if (a.psi_real) hipLaunchKernelGGL((gf_obuild_kernel<NT, true>), grid, block, 0, stream, a, obuf, nmax);
   else hipLaunchKernelGGL((gf_obuild_kernel<NT, false>), grid, block, 0, stream, a, obuf, nmax);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const size_t lds = sizeof(cplx) * ((size_t)nmax * (nmax + 1) + nmax);
-  e = allow_lds((const void*)gf_lu_kernel, lds);
+  e = hipGetLastError();
   if (e != hipSuccess) return e;
   double* res = obuf + 2 * (int64_t)a.nwalkers * 2 * nmax * nmax;
   hipLaunchKernelGGL(gf_lu_kernel, dim3((unsigned)(a.nwalkers * nspin)), dim3(64), lds, stream, a, obuf, oinv, nmax,
