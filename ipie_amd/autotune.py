@@ -12,9 +12,10 @@ Eight launch shapes of the step depend on the system's dimensions:
   tile_fb        workgroup tile of the split-BF16 force-bias GEMM
   tile_vhs       workgroup tile of the split-BF16 VHS GEMM
   tile_one_body  workgroup tile of the split-BF16 one-body GEMM
-                 (tiles: 0 = 128 x 160, 1 = 128 x 128, 2 = 128 x 80,
-                 3 = 64 x 160, 4 = 128 x 320, 5 = 64 x 160 with two LDS
-                 stages; walker rows x output columns)
+                 (tiles: 0 = picked by the launch from its sizes, the
+                 heuristic; 1 = 128 x 128, 2 = 128 x 80, 3 = 64 x 160,
+                 4 = 128 x 320, 5 = 64 x 160 with two LDS stages; walker rows
+                 x output columns)
   taylor         kernel of the split-BF16 Taylor series: 32-wide K stages, two
                  in LDS (0); 16-wide stages, four in LDS (1)
 

@@ -2328,7 +2328,8 @@ int afqmc_tune_get(afqmc_ctx* c, int32_t knob, int32_t* value, int32_t* lo, int3
     case AFQMC_TUNE_TILE_ONE_BODY:
       // split-BF16 GEMM tile shapes (mixed precision; the force bias needs Cholesky vectors)
       if (c->d.precision != AFQMC_PREC_MIXED || c->d.nchol < 1) return AFQMC_OK;
-      *value = std::max(0, knob == AFQMC_TUNE_TILE_FB ? c->tile_fb : knob == AFQMC_TUNE_TILE_VHS ? c->tile_vhs : c->tile_ob);  // 0 until it is set
+      // (0: by the launch's rule, kept as -1)
+      *value = std::max(0, knob == AFQMC_TUNE_TILE_FB ? c->tile_fb : knob == AFQMC_TUNE_TILE_VHS ? c->tile_vhs : c->tile_ob);
       *lo = 0;
       *hi = BF16_TILES - 1;
       return AFQMC_OK;
@@ -2371,11 +2372,11 @@ int afqmc_tune_set(afqmc_ctx* c, int32_t knob, int32_t value) {
   } else if (knob == AFQMC_TUNE_QUAD_RGROUP) {
     c->quad_rgroup = value;
   } else if (knob == AFQMC_TUNE_TILE_FB) {
-    c->tile_fb = value;
+    c->tile_fb = value > 0 ? value : -1;
   } else if (knob == AFQMC_TUNE_TILE_VHS) {
-    c->tile_vhs = value;
+    c->tile_vhs = value > 0 ? value : -1;
   } else if (knob == AFQMC_TUNE_TILE_ONE_BODY) {
-    c->tile_ob = value;
+    c->tile_ob = value > 0 ? value : -1;
   } else {
     c->exx_split = value;
   }

@@ -272,8 +272,8 @@ struct Bf16GemmArgs {
   int cols_fast;
 };
 hipError_t launch_bf16_gemm(const Bf16GemmArgs& a, hipStream_t stream);
-constexpr int BF16_TILES = 6;   // shapes 0 .. 5 are the tuning values
-constexpr int BF16_SHAPES = 7;  // shape 6: picked by the rule only
+constexpr int BF16_TILES = 6;   // tuning values: 0 the rule, 1 .. 5 a shape
+constexpr int BF16_SHAPES = 7;  // shapes 0 and 6: picked by the rule only
 // rows x columns of a workgroup tile shape (false for an unknown shape)
 bool bf16_tile_dims(int tile, int* rows, int* cols);
 
