@@ -1403,8 +1403,8 @@ int afqmc_create(afqmc_ctx** out, int device, const afqmc_dims* dims) {
   const bool two = d.nbeta > 0 && !d.rhf;
   c->ncol = two ? d.nalpha + d.nbeta : d.nalpha;
   const int64_t W = d.nwalkers, N = d.nbasis, X = d.nchol > 0 ? d.nchol : 1;
-  c->fb_ksplit = nt64_ksplit(W, X, ceil_div((int64_t)d.nalpha * N, 16) + (two ? ceil_div((int64_t)d.nbeta * N, 16) : 0),
-                             FB_MAX_SPLIT);
+  const int64_t ka = d.nalpha * N, kb = two ? d.nbeta * N : 0;
+  c->fb_ksplit = nt64_ksplit(W, X, ceil_div(ka, 16) + ceil_div(kb, 16), ka % 2 == 0 && kb % 2 == 0, FB_MAX_SPLIT);
   c->xs_a = exchange_xsplit(d.nwalkers, (int)X, d.nalpha);
   c->xs_b = two ? exchange_xsplit(d.nwalkers, (int)X, d.nbeta) : 1;
   snprintf(c->describe_dims, sizeof(c->describe_dims), "N=%d X=%d na=%d nb=%d W=%d", d.nbasis, d.nchol, d.nalpha,

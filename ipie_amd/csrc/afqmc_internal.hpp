@@ -126,10 +126,11 @@ struct NtArgs {
   const double* dg;
 };
 hipError_t launch_nt64(const NtArgs& a, hipStream_t stream);
-// K ranges (1 .. most) for an [m, n] product over `chunks` 16-wide K chunks: enough
+// K ranges (1 .. most) for an [m, n] product over `chunks` 16-wide K chunks (even: of
+// segments of even K, whose B is loaded 16 bytes a lane): enough
 // workgroups to fill the GPU and rounds that end together, against the
 // partial sums each range adds
-int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, int most);
+int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, bool even, int most);
 // Column units of the block-triangular quadratic form of m rows and n = K columns:
 // tile t of QUAD64_TILE columns sums the chunks up to its own columns' end, cut into
 // units of T chunks (returned; 4 .. 64, the largest that still fills the GPU),

@@ -270,26 +270,34 @@ __global__ void __launch_bounds__(NT_THREADS, 2) nt64_kernel(NtArgs a) {
   }
 }
 
-// What a chunk costs beside its products, in 16-row tiles: the B columns each row tile
-// reads again, with 16-byte loads, and with 4-byte ones four times the load instructions
-// (N = 255, 71 walkers, VHS of 1275 vectors: 48 rows 263 us, 16 rows 308).
-constexpr double NT_OVER = 0.25, NT_OVER_B4 = 0.75;
+// The form that B's loads allow: the tallest row tile in 16s (4-byte loads' addresses
+// and 64 rows do not fit the registers together), and what a chunk costs beside its products,
+// in 16-row tiles: the B columns each row tile reads again, and with 4-byte loads four
+// times the load instructions (N = 255, 71 walkers, VHS of 1275 vectors: 48 rows 263 us,
+// 16 rows 308).  The plans (K ranges, units) and the launch take it from here.
+// Up to `whole` rounds the fullest CU's last one counts whole (N = 301, 600 walkers, force
+// bias of 1000 vectors with 4-byte loads: 10 K ranges in 4.06 rounds 920 us, 5 in 2.97 807).
+struct NtForm {
+  int tallest;
+  double over, whole;
+};
+constexpr NtForm nt_form(bool wide) { return wide ? NtForm{4, 0.25, 4.0} : NtForm{3, 0.75, 6.0}; }
 
 // Cost of a launch in units of one 16-row tile's MFMA time per K chunk (1024
 // cycles): the workgroups of the fullest CU (a fraction of one once there are
 // many rounds), each its chunks and about two chunks' worth of start and
-// epilogue, `over` of a tile per chunk.
-double nt_cost(int64_t m, int64_t colblocks, int rm, double chunks, double over = NT_OVER) {
+// epilogue.
+double nt_cost(int64_t m, int64_t colblocks, int rm, double chunks, const NtForm& form) {
   const double rounds = (double)(ceil_div(m, 16 * rm) * colblocks) / 256.0;
-  return (rounds < 4.0 ? std::ceil(rounds) : rounds) * (chunks + 2.0) * (rm + over);
+  return (rounds < form.whole ? std::ceil(rounds) : rounds) * (chunks + 2.0) * (rm + form.over);
 }
 
-// Rows per workgroup tile, in 16s (1 .. most): the least padding of m on a full
+// Rows per workgroup tile, in 16s: the least padding of m on a full
 // GPU; smaller tiles where larger ones would leave CUs idle.
-int nt_rows(int64_t m, int64_t colblocks, double chunks, int most, double over = NT_OVER) {
+int nt_rows(int64_t m, int64_t colblocks, double chunks, const NtForm& form) {
   int best = 1;
-  for (int rm = 2; rm <= most; ++rm)
-    if (nt_cost(m, colblocks, rm, chunks, over) < 0.999 * nt_cost(m, colblocks, best, chunks, over)) best = rm;
+  for (int rm = 2; rm <= form.tallest; ++rm)
+    if (nt_cost(m, colblocks, rm, chunks, form) < 0.999 * nt_cost(m, colblocks, best, chunks, form)) best = rm;
   return best;
 }
 
@@ -331,8 +339,7 @@ hipError_t launch_nt(const NtArgs& a, hipStream_t stream) {
   if (!a_vec || far) return launch_nt_mode<1, NT_AB4, EPI>(a, stream);
   const int64_t colblocks = EPI == NT_EPI_QDOT ? a.nunits : ceil_div(a.n, NT_TN) * a.ksplit;
   const double each = EPI == NT_EPI_QDOT ? a.unit_chunks + NT_QDOT_CHUNKS : (double)chunks / a.ksplit;
-  // (the 4-byte loads' addresses and 64 rows do not fit the registers together)
-  switch (nt_rows(a.m, colblocks, each, b_vec ? 4 : 3, b_vec ? NT_OVER : NT_OVER_B4)) {
+  switch (nt_rows(a.m, colblocks, each, nt_form(b_vec))) {
     case 1: return launch_nt_rm<1, EPI>(a, b_vec, stream);
     case 2: return launch_nt_rm<2, EPI>(a, b_vec, stream);
     case 3: return launch_nt_rm<3, EPI>(a, b_vec, stream);
@@ -342,7 +349,8 @@ hipError_t launch_nt(const NtArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, int most) {
+int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, bool even, int most) {
+  const NtForm form = nt_form(even);
   const int64_t nbn = ceil_div(n, NT_TN);
   // a further range writes and reads m n partial sums: 32 bytes each at 4.4 TB/s, in units of 0.43 us
   const double part = (double)m * n * 32.0 / 4.4e12 / 0.43e-6;
@@ -350,7 +358,7 @@ int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, int most) {
   double least = 0.0;
   for (int ks = 1; ks <= most && 2 * ks <= std::max<int64_t>(chunks, 2); ++ks) {
     const double each = (double)ceil_div(chunks, ks);
-    const double t = nt_cost(m, nbn * ks, nt_rows(m, nbn * ks, each, 4), each) + part * ks;
+    const double t = nt_cost(m, nbn * ks, nt_rows(m, nbn * ks, each, form), each, form) + part * ks;
     if (ks == 1 || t < 0.98 * least) {
       best = ks;
       least = t;
@@ -360,6 +368,7 @@ int nt64_ksplit(int64_t m, int64_t n, int64_t chunks, int most) {
 }
 
 int nt64_quad_units(int64_t m, int64_t n, std::vector<int4>& units) {
+  const NtForm form = nt_form(n % 2 == 0);
   const int64_t kchunks = ceil_div(n, NT_KC), tiles = ceil_div(n, NT_TN);
   auto extent = [&](int64_t t) { return std::min<int64_t>((t + 1) * (NT_TN / NT_KC), kchunks); };
   auto list = [&](int T, std::vector<int4>& u) {
@@ -376,9 +385,9 @@ int nt64_quad_units(int64_t m, int64_t n, std::vector<int4>& units) {
   // together whatever T.
   auto cost = [&](int T, const std::vector<int4>& u) {
     const double each = T + NT_QDOT_CHUNKS;
-    const int rm = nt_rows(m, (int64_t)u.size(), each, 4);
+    const int rm = nt_rows(m, (int64_t)u.size(), each, form);
     const int64_t rows = ceil_div(m, 16 * rm);
-    if (rows * (int64_t)u.size() > 8192) return nt_cost(m, (int64_t)u.size(), rm, each);
+    if (rows * (int64_t)u.size() > 8192) return nt_cost(m, (int64_t)u.size(), rm, each, form);
     // places that become free at each time, in chunks
     const int start = (int)NT_QDOT_CHUNKS;
     int64_t work = 0;
@@ -397,7 +406,7 @@ int nt64_quad_units(int64_t m, int64_t n, std::vector<int4>& units) {
         end = std::max(end, t + d);
       }
     }
-    return 2.0 * (double)end * (rm + NT_OVER);
+    return 2.0 * (double)end * (rm + form.over);
   };
   int best = 0;
   double least = 0.0;
