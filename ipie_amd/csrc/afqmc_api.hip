@@ -811,7 +811,7 @@ int taylor_bf16(afqmc_ctx* c, int nw, const double** result, const uint16_t** re
   if (!c->ptp_ready)
     HIP_TRY(c, launch_split_transpose(P, nw, (int)c->d.nwalkers, N, nc, rpad, c->kpad, c->tplanes[0], c->stream));
   c->ptp_ready = false;
-  if (c->taylor_variant == 0 && taylor_bf16_in_one(N, c->kpad)) {
+  if (c->taylor_variant == 0 && taylor_bf16_in_one(N, c->kpad, c->d.exp_nmax)) {
     TaylorBf16Args t{};
     t.nwalkers = nw;
     t.wcap = (int)c->d.nwalkers;
@@ -827,7 +827,6 @@ int taylor_bf16(afqmc_ctx* c, int nw, const double** result, const uint16_t** re
     t.init = P;
     t.q = Q;
     t.nterms = c->d.exp_nmax;
-    for (int j = 1; j < t.nterms; ++j) t.terms[j - 1] = c->tplanes[j];
     t.qout = c->tplanes[c->d.exp_nmax == 1 ? 1 : 0];
     HIP_TRY(c, launch_taylor_bf16_series(t, c->stream));
     *result = Q;

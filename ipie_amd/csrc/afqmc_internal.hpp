@@ -325,8 +325,7 @@ struct TaylorBf16Args {
   const double* init;       // [W][N][ncol] complex: the series' input (read by the last term)
   double* q;                // [W][N][ncol] complex: init + sum of the terms (written by the last term)
   // last term: the planes of the earlier terms out_1 .. out_nterms (layout of tin), summed into q
-  // (the series in one launch writes them too: out_1 .. out_{nterms - 1})
-  uint16_t* terms[TAYLOR_MAX_TERMS];
+  const uint16_t* terms[TAYLOR_MAX_TERMS];
   int nterms;
   int first, last;          // this term is the first / the last of the series
   int split;                // 1: three BF16 products (hi hi + hi lo + lo hi), 0: hi hi only
@@ -337,7 +336,7 @@ struct TaylorBf16Args {
 };
 hipError_t launch_taylor_bf16(const TaylorBf16Args& a, hipStream_t stream);
 // all nterms terms in one launch (tin: planes of init^T; q, qout as the last term's)
-bool taylor_bf16_in_one(int nbasis, int kpad);
+bool taylor_bf16_in_one(int nbasis, int kpad, int nterms);
 hipError_t launch_taylor_bf16_series(const TaylorBf16Args& a, hipStream_t stream);
 // Taylor terms k <= TAYLOR_SPLIT_TERMS use three BF16 products, later ones one.
 // Each term but the last writes its four split planes to a buffer of its own

@@ -1193,30 +1193,6 @@ __device__ __forceinline__ void store_planes_ty(uint16_t* dst, int64_t tplane, i
   }
 }
 
-// Sum of the n terms before the last at 4 K entries (offset o of a plane), read back
-// from their planes (hi + lo), smallest first, in FP64.
-__device__ __forceinline__ void ty_sum_terms(const TaylorBf16Args& a, int n, int64_t tplane, int64_t o,
-                                             double (&sre)[4], double (&sim)[4]) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) sre[r] = sim[r] = 0.0;
-  for (int t = n - 1; t >= 0; --t) {
-    const uint16_t* tp = a.terms[t] + o;
-    const ushort4 hr = *reinterpret_cast<const ushort4*>(tp);
-    const ushort4 hi = *reinterpret_cast<const ushort4*>(tp + 2 * tplane);
-    const ushort4 lr = *reinterpret_cast<const ushort4*>(tp + tplane);
-    const ushort4 li = *reinterpret_cast<const ushort4*>(tp + 3 * tplane);
-    const double vr[4] = {(double)bf2f(hr.x) + bf2f(lr.x), (double)bf2f(hr.y) + bf2f(lr.y),
-                          (double)bf2f(hr.z) + bf2f(lr.z), (double)bf2f(hr.w) + bf2f(lr.w)};
-    const double vi[4] = {(double)bf2f(hi.x) + bf2f(li.x), (double)bf2f(hi.y) + bf2f(li.y),
-                          (double)bf2f(hi.z) + bf2f(li.z), (double)bf2f(hi.w) + bf2f(li.w)};
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      sre[r] += vr[r];
-      sim[r] += vi[r];
-    }
-  }
-}
-
 // Epilogue of a Taylor term from the accumulators (transposed tiles: element r
 // of tile i is row crow = i 16 + l16, a column of the walker matrix, and basis
 // index kcol = cb 80 + wave 16 + 4 q + r, so 16 lanes touch 16 consecutive
@@ -1233,8 +1209,27 @@ __device__ __forceinline__ void ty_epilogue(const TaylorBf16Args& a, const v4f (
     // a multiple of 4: Kp % 32 == 0, kc0 % 4 == 0; kc0 + 3 < Kp, and the
     // planes' K padding (kcol >= N) is zero
     const int64_t o = ((int64_t)w * a.rpad + crow) * Kp + kc0;
+    // last term: the earlier terms at these 4 K entries, read back from their
+    // planes (hi + lo), smallest terms first, in FP64
     double sre[4] = {0.0, 0.0, 0.0, 0.0}, sim[4] = {0.0, 0.0, 0.0, 0.0};
-    if (a.last) ty_sum_terms(a, a.nterms, tplane, o, sre, sim);
+    if (a.last) {
+      for (int t = a.nterms - 1; t >= 0; --t) {
+        const uint16_t* tp = a.terms[t] + o;
+        const ushort4 hr = *reinterpret_cast<const ushort4*>(tp);
+        const ushort4 hi = *reinterpret_cast<const ushort4*>(tp + 2 * tplane);
+        const ushort4 lr = *reinterpret_cast<const ushort4*>(tp + tplane);
+        const ushort4 li = *reinterpret_cast<const ushort4*>(tp + 3 * tplane);
+        const double vr[4] = {(double)bf2f(hr.x) + bf2f(lr.x), (double)bf2f(hr.y) + bf2f(lr.y),
+                              (double)bf2f(hr.z) + bf2f(lr.z), (double)bf2f(hr.w) + bf2f(lr.w)};
+        const double vi[4] = {(double)bf2f(hi.x) + bf2f(li.x), (double)bf2f(hi.y) + bf2f(li.y),
+                              (double)bf2f(hi.z) + bf2f(li.z), (double)bf2f(hi.w) + bf2f(li.w)};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sre[r] += vr[r];
+          sim[r] += vi[r];
+        }
+      }
+    }
     uint16_t ht[4][4], hq[4][4];  // [plane][r] of out_k and of q
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -1548,7 +1543,12 @@ __global__ void __launch_bounds__(TY_THREADS) taylor16_kernel(TaylorBf16Args a) 
 // chunk for itself (two 4 KB stages a wave); the waves of a term run without
 // barriers.  The same products in the same order as a launch per term.  Between terms the
 // planes of out_k^T replace those of out_{k-1}^T; the sum of the terms (hi + lo of all
-// but the last, in FP64) stays in registers.
+// but the last, in FP64) stays in registers.  The walkers' bits are those of a launch per
+// term, which sums the terms the other way round: five values of two 8-bit parts each
+// have an exact sum in 53 bits, in any order, unless they span more than that, and the last
+// term's product is rounded by itself.  More than six terms span more: a launch per
+// term.  (Storing every term and summing in that order cost 20 to 33%: N = 150, 1000
+// walkers 186 -> 248 us, N = 200, 512 walkers 350 -> 420.)
 // What bounds it: HELD, the latency of a chunk (LDS reads, then 24 or 8 MFMAs, three waves a
 // SIMD) and the conversions between terms; staged, the latency of the next chunk's
 // atoms.  Against a launch per term, which moves every term's planes through memory and
@@ -1559,6 +1559,7 @@ __global__ void __launch_bounds__(TY_THREADS) taylor16_kernel(TaylorBf16Args a) 
 //   N = 150, W = 1000, n = 30  498 -> 205     N = 180, W = 300, n = 70    355 -> 312
 constexpr int TS_R = 32;  // columns of a group (rows of the planes)
 constexpr int TS_WAVES = 10;
+constexpr int TS_TERMS = 6;  // most terms
 // alpha t + s rounded twice, as by the launch per term
 __device__ __forceinline__ cplx ts_last(double alpha, float re, float im, double sre, double sim) {
 #pragma clang fp contract(off)
@@ -1611,7 +1612,14 @@ __global__ void __launch_bounds__(64 * (HELD ? TS_WAVES : 8), HELD ? 3 : 2)
                                        (__attribute__((address_space(3))) void*)(ring + b * 64), 16, 0, 0);
     }
   }
+  double sre[U][2][4], sim[U][2][4];
   v4f re[U][2], im[U][2];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sre[u][i][r] = sim[u][i][r] = 0.0;
   int buf = 0;
   const auto term = [&](auto np) __attribute__((always_inline)) {
     constexpr int NP = decltype(np)::value;
@@ -1721,10 +1729,9 @@ __global__ void __launch_bounds__(64 * (HELD ? TS_WAVES : 8), HELD ? 3 : 2)
           const bool in = kc0 + r < N;
           split_bf16(in ? alpha * re[u][i][r] : 0.0, h[0][r], h[1][r]);
           split_bf16(in ? alpha * im[u][i][r] : 0.0, h[2][r], h[3][r]);
+          sre[u][i][r] += (double)bf2f(h[0][r]) + bf2f(h[1][r]);
+          sim[u][i][r] += (double)bf2f(h[2][r]) + bf2f(h[3][r]);
         }
-        const int crow = row0 + i * 16 + l16;
-        if (crow < a.ncol && kc0 < N)
-          store_planes_ty(a.terms[k - 1], tplane, ((int64_t)w * a.rpad + crow) * Kp + kc0, h, N - kc0);
 #pragma unroll
         for (int p = 0; p < 4; ++p)
           if (split_next || p % 2 == 0)
@@ -1743,9 +1750,6 @@ __global__ void __launch_bounds__(64 * (HELD ? TS_WAVES : 8), HELD ? 3 : 2)
     for (int i = 0; i < 2; ++i) {
       const int crow = row0 + i * 16 + l16;
       if (crow >= a.ncol || kc0 >= N) continue;
-      const int64_t o = ((int64_t)w * a.rpad + crow) * Kp + kc0;
-      double sre[4], sim[4];
-      ty_sum_terms(a, a.nterms - 1, tplane, o, sre, sim);
       uint16_t h[4][4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -1753,13 +1757,13 @@ __global__ void __launch_bounds__(64 * (HELD ? TS_WAVES : 8), HELD ? 3 : 2)
         for (int p = 0; p < 4; ++p) h[p][r] = 0;
         if (kc0 + r >= N) continue;
         const int64_t qi = ((int64_t)w * N + kc0 + r) * a.ncol + crow;
-        const cplx v = ts_last(alpha, re[u][i][r], im[u][i][r], sre[r], sim[r]);
+        const cplx v = ts_last(alpha, re[u][i][r], im[u][i][r], sre[u][i][r], sim[u][i][r]);
         const cplx qv = cadd(ld(a.init, qi), v);
         st(a.q, qi, qv);
         split_bf16(qv.re, h[0][r], h[1][r]);
         split_bf16(qv.im, h[2][r], h[3][r]);
       }
-      if (a.qout) store_planes_ty(a.qout, tplane, o, h, N - kc0);
+      if (a.qout) store_planes_ty(a.qout, tplane, ((int64_t)w * a.rpad + crow) * Kp + kc0, h, N - kc0);
     }
   }
 }
@@ -2012,16 +2016,16 @@ static bool taylor_series_held(int nbasis, int kpad) {
   return vhs_atom_side(nbasis) <= TS_WAVES && taylor_series_lds(nbasis, kpad, true) <= 163840;
 }
 
-bool taylor_bf16_in_one(int nbasis, int kpad) {
-  return taylor_series_held(nbasis, kpad) ||
-         (vhs_atom_side(nbasis) <= 16 && taylor_series_lds(nbasis, kpad, false) <= 163840);
+bool taylor_bf16_in_one(int nbasis, int kpad, int nterms) {
+  return nterms <= TS_TERMS && (taylor_series_held(nbasis, kpad) ||
+                                (vhs_atom_side(nbasis) <= 16 && taylor_series_lds(nbasis, kpad, false) <= 163840));
 }
 
 hipError_t launch_taylor_bf16_series(const TaylorBf16Args& a, hipStream_t stream) {
   if (a.nwalkers < 1 || a.wcap < a.nwalkers || a.ncol < 1 || a.rpad < a.ncol || a.rpad % 16 != 0 ||
       a.kpad % BX_KC != 0 || a.kpad < a.nbasis || !a.tin || !a.init || !a.q || !a.vatoms || !a.zatom ||
       a.natom_side != vhs_atom_side(a.nbasis) || a.atom_stride < vhs_atom_count(a.nbasis) * 1024 || a.nterms < 1 ||
-      a.nterms > TAYLOR_MAX_TERMS || (a.nterms > 1 && a.terms[a.nterms - 2] == nullptr) || !taylor_bf16_in_one(a.nbasis, a.kpad))
+      !taylor_bf16_in_one(a.nbasis, a.kpad, a.nterms))
     return hipErrorInvalidValue;
   const bool held = taylor_series_held(a.nbasis, a.kpad);
   const size_t lds = taylor_series_lds(a.nbasis, a.kpad, held);
