@@ -48,13 +48,15 @@ struct Tile {
   static constexpr int GR = GR_, GC = GC_, MR = MR_, MC = MC_, ST = ST_, KS1 = KS1_;
   static constexpr int R = 16 * GR * MR, C = 16 * GC * MC, THREADS = 64 * GR * GC;
 };
-// The shapes bf16_gemm_kernel is built for (afqmc_tune_set picks one per
-// contraction; the exchange and the quadratic form use shape 0).  All have 8
-// waves; shapes 0-3 three LDS stages of the 3-product form within 160 KiB,
+// The shapes bf16_gemm_kernel is built for (picked per launch by
+// bf16_tile_by_rule or, for the force bias, VHS and one body, by afqmc_tune_set;
+// the quadratic form takes those of 160 columns in its layout, 0, 5 and 6, the
+// exchange per Cholesky vector shape 0).  All but 6 have 8 waves; shapes 0-3 three LDS stages of the 3-product form within 160 KiB,
 // shape 4 (64 x 80 per wave: 29% fewer LDS bytes per MFMA than 32 x 80) two,
 // shape 5 two stages of 36 KiB, so that two workgroups share a CU (one can
 // run its epilogue while the other computes: short K, heavy epilogues).  Shape 6,
-// 4 waves and two workgroups a CU, is for few rows and is not a tuning value.
+// 4 waves and two workgroups a CU, is for few rows; it and shape 0 are reached
+// through the rule only.
 using Tile0 = Tile<4, 2, 2, 5>;     // 128 x 160
 using Tile1 = Tile<4, 2, 2, 4>;     // 128 x 128
 using Tile2 = Tile<8, 1, 1, 5>;     // 128 x 80
@@ -893,7 +895,7 @@ __global__ void __launch_bounds__(TL::THREADS) bf16_gemm_kernel(Bf16GemmArgs a) 
     }
     }
     if (a.epilogue == BF16_EPI_QDOT) {
-      // (the quadratic form runs with tile shape 0 and plain accumulators only:
+      // (the quadratic form runs with tile shapes 0, 5 and 6 and plain accumulators only:
       // launch_bf16_gemm; each epilogue is compiled only where it can run)
       if constexpr (!TR && QdotTile<TL>::value) {
       // per-row dot with d over this wave's 80 columns, then across the 16 lanes

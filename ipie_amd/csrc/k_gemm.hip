@@ -583,7 +583,10 @@ hipError_t launch_one_body64(const OneBody64Args& a, hipStream_t stream) {
 }
 
 // The series in one launch: at most 16 row tiles, T in LDS.  Column blocks of 8, 16 or
-// 24: the least MFMA time of the fullest CU.
+// 24: the least time of the fullest CU.  One workgroup a CU takes (us for 8, 16, 24
+// columns, 6 terms) 13, 22, 32 at N = 64, 35, 62, 91 at N = 128, 120, 194, 290 at N = 200 and
+// 183, 250, 371 at N = 255: a time for every 8 columns and a fixed part, 0.1 to 0.4 of it up
+// to N = 200 and as much at N = 255.  The rule takes 0.14.
 bool taylor64_in_one(int nbasis) { return nbasis <= 256; }
 
 hipError_t launch_taylor64_series(Taylor64Args a, hipStream_t stream) {
@@ -595,7 +598,7 @@ hipError_t launch_taylor64_series(Taylor64Args a, hipStream_t stream) {
   for (int rn = 1; rn <= 3; ++rn) {
     const int64_t blocks = (int64_t)a.nwalkers * ceil_div(a.ncol, 8 * rn);
     const double rounds = blocks < 1024 ? (double)ceil_div(blocks, 256) : blocks / 256.0;
-    const double t = rounds * (8 * rn * 0.0272 + 0.03);
+    const double t = rounds * (rn + 0.138);
     if (rn == 1 || t < 0.99 * least) {
       best = rn;
       least = t;

@@ -18,8 +18,8 @@
 // the permutation k -> p_k, and only the columns after k are updated.  For the inverse
 // (Gauss-Jordan) the used rows take part and column k becomes (B[i][k] / d, -1 in row p):
 // row p_k then holds -d_k times row k of the inverse, its column j that of row p_j of O.
-// Errors against 80-bit sums (n = 40, N = 400, trial orbitals with noise): Ghalf 6.5e-16,
-// overlap 3.3e-15 (LU and inverse from its factors: 6.7e-16 and 4.0e-15).
+// Errors against 80-bit sums (n = 40, N = 400, trial orbitals with noise, rms): Ghalf
+// 6.3e-16, overlap 1.9e-15 (LU and inverse from its factors: 6.7e-16 and 4.4e-15).
 //
 // What bounds it, by walkers: few (one workgroup a CU) the chain of n pivot steps, 0.6 us
 // each (LDS hand-over of the pivot column, maximum over the rows, reciprocal, the

@@ -14,8 +14,8 @@
 // 16 rows at the row pitch (32 cache lines per load instruction), one K chunk
 // ahead, with one wave per SIMD (296 VGPRs), and ran at 59% of the FP64 MFMA
 // peak.  Here a workgroup of four waves stages K chunks of 16 through LDS with
-// direct global-to-LDS loads (two stages; the next chunk's loads run under the
-// current chunk's MFMAs, one barrier per chunk); a row's piece of a chunk is
+// direct global-to-LDS loads (two to four stages, by the row tile; the next chunks'
+// loads run under the current chunk's MFMAs, one barrier per chunk); a row's piece of a chunk is
 // 256 B (complex) or 128 B (real), so every load instruction covers whole
 // cache lines.  The waves share the rows and each takes 32 of the tile's 128
 // columns, which keeps the kernel within 256 registers (two workgroups per CU:

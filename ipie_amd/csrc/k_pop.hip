@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(POP_THREADS) pop_plan_kernel(PopPlanArgs a) {
               if (gt == up) {
                 bits[i] = kj;
                 bits[j] = ki;
-              const int ti = idx[i];
+                const int ti = idx[i];
                 idx[i] = idx[j];
                 idx[j] = ti;
               }
