@@ -128,8 +128,7 @@ def build_device(host, w, mode, tuner=None):
     prop = PhaselessGeneric(w.dt, seed=w.seed, precision=precision, surrogate=surrogate, autotune=tuner)
     prop.build(host["ham"], host["trial"], walkers)
     torch.cuda.synchronize()
-    log(f"[bench] {mode}: device context + upload in {time.time() - t0:.1f}s"
-        + (f", launch shapes {prop.tuning}" if prop.tuning is not None else ""))
+    log(f"[bench] {mode}: device context + upload in {time.time() - t0:.1f}s")
     return dict(host, walkers=walkers, prop=prop)
 
 
@@ -677,6 +676,30 @@ def run_modes(args, w, host, mode_list, K, warmup, tuner):
     return modes
 
 
+# what the line on stdout keeps of a mode's record (--record holds all of it)
+BRIEF = ("value", "ms_per_step", "eager_ms_per_step", "energy_bias_Ha", "energy_bias_sem_Ha",
+         "added_variance_per_step_Ha2", "within_0p1_mHa", "within_variance_budget")
+
+
+def brief(out, head):
+    """The record as the one line on stdout, of a few KB: per-mode details, the tuner's
+    timings and the batch's systems stay out."""
+    def modes(full):
+        return {m: {k: r[k] for k in BRIEF if k in r} for m, r in full.items()}
+
+    line = dict(out, modes=modes(out["modes"]))
+    line["modes"][head]["phases_ms_per_step"] = out["modes"][head]["phases_ms_per_step"]
+    line["modes"][head]["launch_shapes"] = out["modes"][head]["launch_shapes"]
+    line["roofline"] = dict(out["roofline"], other_phases=[
+        {k: p[k] for k in ("phase", "ms_per_step", "achieved", "peak", "frac")}
+        for p in out["roofline"]["other_phases"]])
+    if "secondary" in out:
+        sur, multi = out["secondary"]["n300_surrogate"], out["secondary"]["multi16"]
+        line["secondary"] = {"n300_surrogate": dict(sur, modes=modes(sur["modes"])),
+                             "multi16": {k: v for k, v in multi.items() if k not in ("config", "launch_shapes")}}
+    return line
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -703,6 +726,9 @@ def main():
                     help="keep the heuristic launch shapes (default: tune them per context at build time)")
     ap.add_argument("--cpu-walkers", type=int, default=4)
     ap.add_argument("--cpu-steps", type=int, default=2)
+    ap.add_argument("--record", default=None, metavar="FILE",
+                    help="also write the whole record (every mode's details and launch shapes, the tuner's "
+                         "timings) to this file")
     ap.add_argument("--calibration-copy-mb", type=int, default=0,
                     help="only copy a device buffer of this many MiB once and exit (the reference for the "
                          "FETCH_SIZE / WRITE_SIZE counters behind roofline.traffic)")
@@ -850,7 +876,10 @@ def main():
         del host
         out["secondary"] = {"n300_surrogate": run_surrogate_workload(args, tuner),
                             "multi16": run_multi(args, emit=False)}
-    print(json.dumps(out), flush=True)
+    if args.record:
+        with open(args.record, "w") as fh:
+            json.dump(out, fh, indent=1)
+    print(json.dumps(brief(out, head)), flush=True)
 
 
 if __name__ == "__main__":
