@@ -36,7 +36,7 @@ struct afqmc_ctx {
   double* exx_b = nullptr;       // [xs_b, W] complex
   double* vhs = nullptr;         // FP64: packed upper triangles [W, N (N + 1) / 2] complex
   double* buf[4] = {nullptr, nullptr, nullptr, nullptr};  // P, Ta, Tb, Q (mixed): [W, N, ncol] complex
-  int* qr_slow = nullptr;        // FP64: [W] scratch of the re-orthogonalisation
+  int* qr_slow = nullptr;        // [W] scratch of the re-orthogonalisation
   int* flags = nullptr;
   int* wflags = nullptr;    // [W] per-walker flags (OR of AFQMC_FLAG_*) since the last take
   int* psi_flag = nullptr;  // scratch of afqmc_set_static's check of the trial orbitals
@@ -395,6 +395,7 @@ int ensure_ws(afqmc_ctx* c) {
   if (ok) c->fb_cap = c->fb_ksplit;
   ok = ok && dmalloc((void**)&c->xshifted, 16 * (size_t)W * X) == hipSuccess;
   ok = ok && dmalloc((void**)&c->wvec, 16 * (size_t)6 * W) == hipSuccess;
+  ok = ok && dmalloc((void**)&c->qr_slow, sizeof(int) * (size_t)W) == hipSuccess;
   // partial sums: at most one per Cholesky vector per walker, whatever the split
   c->exx_cap = (int64_t)X * W;
   ok = ok && dmalloc((void**)&c->exx_a, 16 * (size_t)c->exx_cap) == hipSuccess;
@@ -430,7 +431,6 @@ int ensure_ws(afqmc_ctx* c) {
   // FP64 VHS, packed upper triangles (1.3 GB at N=400); the split-BF16 path keeps VHS as atoms only
   if (d.precision != AFQMC_PREC_MIXED) {
     ok = ok && dmalloc((void**)&c->vhs, 16 * (size_t)W * P) == hipSuccess;
-    ok = ok && dmalloc((void**)&c->qr_slow, sizeof(int) * (size_t)W) == hipSuccess;
   }
   for (int i = 0; i < 4; ++i) {  // (the FP64 path takes three)
     if (i == 3 && d.precision != AFQMC_PREC_MIXED) continue;
@@ -2053,6 +2053,7 @@ int afqmc_reortho(afqmc_ctx* c, int32_t nw, double* phia, double* phib, double* 
   a.flags = c->flags;
   a.wflags = c->wflags;
   a.slow = c->qr_slow;
+  a.ordered = c->d.precision == AFQMC_PREC_MIXED;  // (rounded to BF16 next)
   PhaseScope ps(c, AFQMC_PHASE_REORTHO, PhaseScope::KERNEL);
   a.mark = ps.mark();
   PHASE_TRY(c, ps, launch_reortho(a, c->stream));

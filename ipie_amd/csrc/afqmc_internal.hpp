@@ -567,7 +567,8 @@ struct ReorthoArgs {
   const double* detR_shift;  // [W] or null
   int* flags;
   int* wflags;               // [W] per-walker flags or null
-  int* slow;                 // [W] scratch: walkers left to the general kernel; null: all
+  int* slow;                 // [W] scratch: walkers left to the general kernel
+  int ordered;               // the fast kernel keeps the general one's order of every sum
 };
 hipError_t launch_reortho(const ReorthoArgs& a, hipStream_t stream);
 

@@ -7,11 +7,11 @@
 //   G = X^H X (+ shift),  G = R^H R,  X <- X R^{-1},
 // as sweeps over the rows of X on FP64 MFMA: the Gram matrix of pass p + 1 is
 // formed from the rows of X R_p^{-1} while they are written.
-// In double precision the walkers with at most 48 columns that take the first branch
-// below, that is all but ill-conditioned ones, run in reortho_fast_kernel, the others
-// in reortho_kernel.  In mixed precision all run in reortho_kernel: the walkers are
-// rounded to pairs of BF16 values next, so that another order of the sums, which
-// moves their last bits, would move a walker by 1e-6 now and then (k_greens_lu.hip).
+// Walkers with at most 48 columns that take the first branch below, that is all but
+// ill-conditioned ones, run in reortho_fast_kernel, the others in reortho_kernel.  In
+// mixed precision the walkers are rounded to pairs of BF16 values next, so that another
+// order of the sums, which moves their last bits, would move a walker by 1e-6 now and
+// then (k_greens_lu.hip): there the fast kernel factors in reortho_kernel's order.
 //   - CholeskyQR2 (two passes, three sweeps; Yamamoto, Nakatsukasa, Yanagisawa,
 //     Fukaya, ETNA 44 (2015) 306) when the unshifted Cholesky of X^H X succeeds
 //     and 8 kappa sqrt(N n u + n (n + 1) u) <= 1/2 with kappa bounded by
@@ -279,8 +279,8 @@ __device__ void qr_finish(const ReorthoArgs& a, int w, double logdet) {
 // column), the rest is 16 x 16 MFMA products, and the two spins' matrices run side
 // by side on two waves each.  S holds one matrix per spin: the Gram matrix,
 // then R, then R^-1, all in place, identity in the padding.
-//   N = 400, n = 40, 1024 walkers: 0.98 ms against 2.54 ms in reortho_kernel; 12 walkers 276 us
-//   against 577 us.
+//   N = 400, n = 40, 1024 walkers: 0.91 ms against 2.54 ms in reortho_kernel; 12 walkers 278 us
+//   against 557 us.
 __device__ __forceinline__ double lane_value(double v, int lane) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
                           __builtin_amdgcn_readlane(__double2loint(v), lane));
@@ -463,6 +463,96 @@ __device__ __forceinline__ void qr_factor(cplx* S, int nspin, double* logdet, in
   __syncthreads();
 }
 
+// The same in the order of the general kernel: every entry takes the operations of
+// qr_cholesky and qr_upper_inverse one after the other (fused as the compiled code of
+// those has them), log det R sums in the same order, so that a walker's bits are those of
+// reortho_kernel.  A wave pair per spin side by side, rows through LDS; diag [nspin][16 NT]
+// scratch.  Bound by the chain of n steps: N = 400, n = 40, 1024 walkers 1.11 ms and 12
+// walkers 396 us, where the blocked form takes 0.91 and 278 and reortho_kernel 2.54 and 557.
+// (Cholesky entries kept in registers and 16 columns x four partial sums a wave in the
+// inverse: 1.07 ms and 344 us, in three times the code.)
+template <int NT>
+__device__ __forceinline__ void qr_factor_ordered(cplx* S, int nspin, int n0, int n1, double* diag, double* logdet,
+                                                  int* ok) {
+  constexpr int LD = 16 * NT + 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), spin = wave >> 1, part = wave & 1;
+  const int lane = threadIdx.x & 63, t = threadIdx.x & 127, ti = t >> 4, tj = t & 15;
+  const int n = spin >= nspin ? 0 : spin == 0 ? n0 : n1, steps = nspin > 1 ? max(n0, n1) : n0;
+  cplx* G = S + spin * 16 * NT * LD;
+  diag += spin * 16 * NT;
+  bool good = true;
+  double dprev = 0.0;
+#pragma unroll 1
+  for (int k = 0; k <= steps; ++k) {
+    if (k > 0 && k <= n && good) {  // row k - 1 is not read any more
+      const double inv = 1.0 / dprev;
+      if (k + t < n) G[(k - 1) * LD + k + t] = cscale(G[(k - 1) * LD + k + t], inv);
+      if (t == 0) {
+        G[(k - 1) * LD + k - 1] = cmake(dprev, 0.0);
+        diag[k - 1] = dprev;
+      }
+    }
+    if (k < n && good) {
+      const double dkk = G[k * LD + k].re;  // the same value in every thread
+      good = dkk > 0.0;
+      if (good) {
+        const double idkk = 1.0 / dkk;
+        dprev = sqrt(dkk);
+        for (int i = k + 1 + ti; i < n; i += 8) {
+          const cplx gki = G[k * LD + i];
+          int j = k + 1 + tj;
+          if (j < i) j += (i - j + 15) / 16 * 16;  // first column >= i of this thread's residue class
+          for (; j < n; j += 16) {
+            const cplx gkj = G[k * LD + j], g = G[i * LD + j];
+            const double re = fma(gki.re, gkj.re, gki.im * gkj.im), im = fma(gki.re, gkj.im, -(gki.im * gkj.re));
+            G[i * LD + j] = cmake(fma(-idkk, re, g.re), fma(-idkk, im, g.im));
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (good && part == 1) {
+    const double lg = lane < n ? log(diag[lane]) : 0.0;
+    double sum = 0.0;
+    for (int k = 0; k < n; ++k) sum += lane_value(lg, k);
+    if (lane == 0) logdet[spin] = sum;
+  }
+  // the inverse in place, rows from the last, lane = column: row i takes row i of R (read by
+  // every lane of the wave before any writes) and the rows below of its own column
+  if (good && part == 0) {
+#pragma unroll 1
+    for (int i = n - 1; i >= 0; --i) {
+      const cplx* R = G + i * LD;
+      const double rinv = 1.0 / R[i].re;
+      if (lane >= i && lane < n) {
+        cplx s[4] = {cmake(lane == i ? 1.0 : 0.0, 0.0), cmake(0.0, 0.0), cmake(0.0, 0.0), cmake(0.0, 0.0)};
+        const auto less = [](cplx& v, cplx r, cplx x) {
+          v.re -= fma(r.re, x.re, -(r.im * x.im));
+          v.im -= fma(r.im, x.re, r.re * x.im);
+        };
+        int k = i + 1;
+        for (; k + 3 <= lane; k += 4) {
+          cplx r[4], x[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            r[u] = R[k + u];
+            x[u] = G[(k + u) * LD + lane];
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) less(s[u], r[u], x[u]);
+        }
+        for (; k <= lane; ++k) less(s[0], R[k], G[k * LD + lane]);
+        G[i * LD + lane] = cscale(cadd(cadd(s[0], s[1]), cadd(s[2], s[3])), rinv);
+      } else if (lane < i && lane / 16 == i / 16) {
+        G[i * LD + lane] = cmake(0.0, 0.0);  // below the diagonal in its block
+      }
+    }
+  }
+  if (t == 0 && spin < nspin) ok[spin] = good;
+  __syncthreads();
+}
+
 // The sweep of one matrix (as qr_sweep): APPLY replaces the rows by X S, GRAM leaves
 // the Gram matrix of the (new) rows in S with identity padding and returns its
 // trace.  A tile's 4 NT loads are in flight under the MFMAs before it; values past
@@ -569,12 +659,12 @@ __device__ __forceinline__ double qr_fast_sweep(double* __restrict__ X, int N, i
   return block_sum((int)threadIdx.x < n ? S[threadIdx.x * (LD + 1)].re : 0.0, sums);
 }
 
-template <int NT>
+template <int NT, bool ORDERED>
 __global__ void __launch_bounds__(QR_THREADS, 2) reortho_fast_kernel(ReorthoArgs a) {
   phase_mark(a.mark, blockIdx.x == 0 && threadIdx.x == 0);
   constexpr int LD = 16 * NT + 1;
   extern __shared__ cplx smem[];
-  __shared__ double logdet[2], sums[QR_WAVES];
+  __shared__ double logdet[2], sums[QR_WAVES], diag[ORDERED ? 2 * 16 * NT : 1];
   __shared__ int ok[2];
   cplx* S = smem;  // per spin [16 NT][LD]
   const int w = blockIdx.x, N = a.nbasis, nspin = a.nbeta > 0 ? 2 : 1;
@@ -586,12 +676,14 @@ __global__ void __launch_bounds__(QR_THREADS, 2) reortho_fast_kernel(ReorthoArgs
     double* X = (s == 0 ? a.phia : a.phib) + 2 * (int64_t)w * N * n;
     (s == 0 ? tr0 : tr1) = qr_fast_sweep<NT, false, true>(X, N, n, S + s * 16 * NT * LD, sums);
   }
-  double ld = 0.0;
+  double first[2] = {0.0, 0.0};  // log det R of the first pass
 #pragma unroll 1
   for (int pass = 0; pass < 2; ++pass) {  // (one call site: the factorisation is inlined once)
-    qr_factor<NT>(S, nspin, logdet, ok);
-    ld += logdet[0] + (nspin > 1 ? logdet[1] : 0.0);
+    if constexpr (ORDERED) qr_factor_ordered<NT>(S, nspin, a.nalpha, a.nbeta, diag, logdet, ok);
+    else qr_factor<NT>(S, nspin, logdet, ok);
     if (pass == 1) break;
+    first[0] = logdet[0];
+    if (nspin > 1) first[1] = logdet[1];
     bool slow = false;
     for (int s = 0; s < nspin; ++s) {
       const int n = s == 0 ? a.nalpha : a.nbeta;
@@ -632,7 +724,11 @@ __global__ void __launch_bounds__(QR_THREADS, 2) reortho_fast_kernel(ReorthoArgs
     double* X = (s == 0 ? a.phia : a.phib) + 2 * (int64_t)w * N * n;
     qr_fast_sweep<NT, true, false>(X, N, n, S + s * 16 * NT * LD, sums);
   }
-  if (threadIdx.x == 0) qr_finish(a, w, ld);
+  if (threadIdx.x == 0) {
+    double ld = first[0] + logdet[0];
+    if (nspin > 1) ld = ORDERED ? ld + first[1] + logdet[1] : first[0] + first[1] + (logdet[0] + logdet[1]);
+    qr_finish(a, w, ld);
+  }
 }
 
 template <int NT>
@@ -708,15 +804,15 @@ hipError_t launch_qr_nt(const ReorthoArgs& a, hipStream_t stream) {
   hipError_t e = allow_lds((const void*)reortho_kernel<NT>, 2 * matrix);
   if (e != hipSuccess) return e;
   ReorthoArgs b = a;
-  bool fast = a.slow != nullptr;
-  if constexpr (NT > 3) fast = false;  // (64 columns do not fit the fast kernel's registers)
-  if constexpr (NT <= 3) if (fast) {
+  if constexpr (NT <= 3) {  // (64 columns do not fit the fast kernel's registers)
     const size_t lds = matrix * (a.nbeta > 0 ? 2 : 1);
-    e = allow_lds((const void*)reortho_fast_kernel<NT>, lds);
+    e = allow_lds(a.ordered ? (const void*)reortho_fast_kernel<NT, true> : (const void*)reortho_fast_kernel<NT, false>, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(reortho_fast_kernel<NT>, dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a);
-  }
-  if (!fast) {
+    if (a.ordered)
+      hipLaunchKernelGGL((reortho_fast_kernel<NT, true>), dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a);
+    else
+      hipLaunchKernelGGL((reortho_fast_kernel<NT, false>), dim3(a.nwalkers), dim3(QR_THREADS), lds, stream, a);
+  } else {
     b.slow = nullptr;
     if (a.mark.acc && (e = launch_phase_mark(a.mark, stream)) != hipSuccess) return e;
   }
@@ -728,6 +824,7 @@ hipError_t launch_qr_nt(const ReorthoArgs& a, hipStream_t stream) {
 
 hipError_t launch_reortho(const ReorthoArgs& a, hipStream_t stream) {
   const int nmax = a.nalpha > a.nbeta ? a.nalpha : a.nbeta;
+  if (!a.slow) return hipErrorInvalidValue;
   switch ((nmax + 15) / 16) {
     case 1: return launch_qr_nt<1>(a, stream);
     case 2: return launch_qr_nt<2>(a, stream);
